@@ -1,0 +1,49 @@
+"""GPU tests of the one-launch PCG iteration at the sizes where its tiles and
+chunks begin and end (15 output nodes a tile, 16 cells, chunks of planes), and
+where its residual sums cannot be formed by subtraction."""
+import numpy as np
+import pytest
+
+from conftest import relerr
+
+pytestmark = pytest.mark.gpu
+
+HEAT = [(1, 1), (14, 14), (15, 16), (29, 31), (44, 3), (1, 1, 1), (14, 15, 2), (16, 13, 5),
+        (30, 15, 9), (3, 44, 17)]
+
+
+@pytest.mark.parametrize("nels", HEAT)
+def test_heat_tiles(T, gpu, nels):
+    from oracle import heat_oracle as H
+    sizes = (1.0, 0.7, 1.6)[:len(nels)]
+    kw = dict(Tleft=1.0, Tright=None, heatflux={"top": 1.0}, cload={2: 0.5})
+    prob = T.HeatConductionProblem(nels, sizes, 1.3, **kw)
+    P = H.HeatProblem(nels, sizes, 1.3, **kw)
+    s = T.FEASolver(T.HIPMatrixFreeSolver, prob, xmin=0.01, penalty=T.PowerPenaltyFun(3.0),
+                    abstol=0.0, reltol=1e-13, cg_max_iter=20000)
+    g = np.random.default_rng(sum(nels))
+    x = g.uniform(0.2, 1.0, prob.ncells)
+    s.set_densities(x)
+    K = P.assemble(0.01 + 0.99 * x**3)
+    free = ~P.fixed
+    v = g.standard_normal(prob.ndofs)
+    # every node a sum of at most 27 terms: a few roundings of its largest
+    assert relerr(s.matvec(v)[free], K[free][:, free] @ v[free]) < 1e-14
+    s()
+    Te, _ = P.solve(x, 3.0, 0.01)
+    assert s.converged
+    # ||r|| <= 1e-13 ||r0|| times the condition numbers here (below 1e4)
+    assert relerr(s.u, Te) < 1e-9
+    # a warm start from the solution stops at once or stays there
+    s(initially_zero=False)
+    assert relerr(s.u, Te) < 1e-9
+
+
+def test_heat_maxiter_and_zero_load(T, gpu):
+    prob = T.HeatTree((33, 18))
+    s = T.FEASolver(T.HIPMatrixFreeSolver, prob, abstol=0.0, reltol=1e-12)
+    for n in (0, 1, 2, 7, 8, 9):  # converges after ny = 18
+        s(maxiter=n)
+        assert s.last_iters == n and not s.converged
+    s(rhs=np.zeros(prob.ndofs))
+    assert s.last_iters == 0 and s.converged and not np.any(s.lhs)

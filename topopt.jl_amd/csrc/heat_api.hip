@@ -6,6 +6,7 @@
 // src/Functions/temperature.jl).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <limits>
 #include <string>
@@ -20,6 +21,7 @@ using namespace tohip;
 struct tohip_heat {
     HeatGrid g{};
     HeatKe ke{};
+    HeatModes modes{};
     double xmin = 1e-3;
     Penalty pen{TOHIP_PEN_POWER, TOHIP_PROJ_NONE, 1.0, 0.0};
     int pbi = 1;
@@ -29,17 +31,21 @@ struct tohip_heat {
     hipStream_t stream = nullptr;
     uint8_t* fixmask = nullptr;
     double *fixv = nullptr, *x = nullptr, *E = nullptr, *dinv = nullptr;
-    double *u = nullptr, *r = nullptr, *p[2] = {nullptr, nullptr}, *q = nullptr, *b = nullptr,
-           *t = nullptr, *lam = nullptr, *cell = nullptr, *grad = nullptr;
-    double *partA = nullptr, *partB = nullptr;
-    PcgScalars *sc = nullptr, *h_sc = nullptr;
-    hipGraphExec_t graph = nullptr;
+    // PCG: two sets of r, p, q, partial sums and state (k_pcg1.h)
+    double *u = nullptr, *r[2] = {nullptr, nullptr}, *p[2] = {nullptr, nullptr},
+           *q[2] = {nullptr, nullptr}, *b = nullptr, *t = nullptr, *lam = nullptr,
+           *cell = nullptr, *grad = nullptr;
+    double* part[2] = {nullptr, nullptr};
+    Pcg1State *st = nullptr, *h_st = nullptr;
+    hipGraphExec_t graph = nullptr, graph_short = nullptr;
     std::string err;
 };
 
 namespace {
 
-constexpr int kHeatGraphIters = 32;
+// Iterations (launches) of the two captured graphs; even, so that a graph
+// starts and ends on the first set of vectors.
+constexpr int kHeatGraphIters = 64, kHeatGraphShort = 8;
 thread_local std::string g_heat_error;
 
 #define HCK(call)                                                  \
@@ -73,6 +79,25 @@ void heat_ke(int dim, const double* h, double k, HeatKe& ke) {
             }
             ke.k[a * nc + b] = k * s;
         }
+}
+
+// Ke's diagonal in the Hadamard basis, (H^T Ke H)[m][m] / corners^2.
+void heat_modes(int dim, const HeatKe& ke, HeatModes& B) {
+    const int nc = 1 << dim;
+    auto bits = [](int b) { return ((b & 1) ^ ((b >> 1) & 1)) | (b & 6); };  // Ferrite -> bits
+    auto H = [](int c, int m) {
+        int s = 1;
+        for (int a = 0; a < 3; ++a)
+            if ((m >> a) & 1) s *= ((c >> a) & 1) ? 1 : -1;
+        return s;
+    };
+    for (int m = 0; m < nc; ++m) {
+        double s = 0.0;
+        for (int a = 0; a < nc; ++a)
+            for (int b = 0; b < nc; ++b)
+                s += H(bits(a), m) * H(bits(b), m) * ke.k[a * nc + b];
+        B.b[m] = m == 0 ? 0.0 : s / double(nc * nc);  // constants have no gradient
+    }
 }
 
 template <typename T>
@@ -113,27 +138,24 @@ int refresh(tohip_heat* ctx) {
     return 0;
 }
 
-int capture(tohip_heat* ctx) {
-    if (ctx->graph) return 0;
+int capture(tohip_heat* ctx, hipGraphExec_t* exec, int iters) {
+    if (*exec) return 0;
     hipGraph_t graph;
     HCK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    for (int it = 0; it < kHeatGraphIters; ++it) {
-        int nbA = 0;
-        hipError_t e1 = launch_heat_dirmatvec(ctx->g, ctx->ke, ctx->r, ctx->dinv, ctx->p[0],
-                                              ctx->p[1], ctx->q, ctx->fixmask, ctx->E,
-                                              ctx->meandiag, ctx->sc, ctx->partB, kVecBlocks,
-                                              ctx->partA, &nbA, ctx->stream);
-        hipError_t e2 = launch_pcg_update<double>(ctx->g.nnodes, ctx->u, ctx->r, ctx->p[0],
-                                                  ctx->p[1], ctx->q, ctx->dinv, ctx->sc,
-                                                  ctx->partA, nbA, ctx->partB, ctx->stream);
-        if (e1 != hipSuccess || e2 != hipSuccess) {
+    for (int it = 0; it < iters; ++it) {
+        const int i = it & 1, o = i ^ 1;
+        const Pcg1Args a{ctx->u,    ctx->r[i], ctx->p[i],    ctx->q[i],    ctx->dinv,
+                         ctx->r[o], ctx->p[o], ctx->q[o],    ctx->st + i,  ctx->st + o,
+                         ctx->part[i], ctx->part[o], heat_pcg_blocks(ctx->g)};
+        if (launch_heat_pcg(ctx->g, ctx->modes, ctx->fixmask, ctx->E, ctx->meandiag, a,
+                            ctx->stream) != hipSuccess) {
             hipStreamEndCapture(ctx->stream, &graph);
             ctx->err = "heat PCG graph capture failed";
             return TOHIP_ERR_HIP;
         }
     }
     HCK(hipStreamEndCapture(ctx->stream, &graph));
-    HCK(hipGraphInstantiate(&ctx->graph, graph, nullptr, nullptr, 0));
+    HCK(hipGraphInstantiate(exec, graph, nullptr, nullptr, 0));
     HCK(hipGraphDestroy(graph));
     return 0;
 }
@@ -144,32 +166,56 @@ int capture(tohip_heat* ctx) {
 int solve(tohip_heat* ctx, bool zero, double abstol, double reltol, int64_t maxiter,
           int64_t* iters, double* resid) {
     const int64_t n = ctx->g.nnodes;
-    PcgScalars hs{};
+    Pcg1State hs{};
+    hs.rho_prev = 1.0;  // IterativeSolvers starts from rho_prev = 1 (multiplies p = 0)
+    hs.tol = -1.0;
     hs.abstol = abstol;
     hs.reltol = reltol;
     hs.maxiter = maxiter;
-    *ctx->h_sc = hs;
-    HCK(hipMemcpyAsync(ctx->sc, ctx->h_sc, sizeof(PcgScalars), hipMemcpyHostToDevice,
+    *ctx->h_st = hs;
+    HCK(hipMemcpyAsync(ctx->st, ctx->h_st, sizeof(Pcg1State), hipMemcpyHostToDevice,
                        ctx->stream));
-    if (zero) {
+    if (zero)
         HCK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
-        HCK(launch_pcg_start<double>(n, ctx->b, nullptr, ctx->r, ctx->dinv, ctx->p[0], ctx->sc,
-                                     ctx->partB, 0, ctx->stream));
-    } else {
-        HCK(launch_heat_matvec(ctx->g, ctx->ke, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag,
+    else
+        HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag,
                                ctx->t, 0, ctx->stream));
-        HCK(launch_pcg_start<double>(n, ctx->b, ctx->t, ctx->r, ctx->dinv, ctx->p[0], ctx->sc,
-                                     ctx->partB, 0, ctx->stream));
-    }
-    if (int rc = capture(ctx)) return rc;
+    HCK(launch_pcg1_start(n, ctx->b, zero ? nullptr : ctx->t, ctx->dinv, ctx->r[0], ctx->p[0],
+                          ctx->part[0], heat_pcg_blocks(ctx->g), ctx->stream));
+    if (int rc = capture(ctx, &ctx->graph, kHeatGraphIters)) return rc;
+    if (int rc = capture(ctx, &ctx->graph_short, kHeatGraphShort)) return rc;
+    // long graphs while the residual's history predicts many iterations to go,
+    // several per host check far from the end
+    double prev_res = -1.0;
+    long long prev_it = -1;
+    bool brief = false;
+    int launches = 1;
     for (;;) {
-        HCK(hipGraphLaunch(ctx->graph, ctx->stream));
-        HCK(hipMemcpyAsync(ctx->h_sc, ctx->sc, sizeof(PcgScalars), hipMemcpyDeviceToHost,
+        for (int l = 0; l < launches; ++l)
+            HCK(hipGraphLaunch(brief ? ctx->graph_short : ctx->graph, ctx->stream));
+        HCK(hipMemcpyAsync(ctx->h_st, ctx->st, sizeof(Pcg1State), hipMemcpyDeviceToHost,
                            ctx->stream));
         HCK(hipStreamSynchronize(ctx->stream));
-        if (ctx->h_sc->done) break;
+        const Pcg1State& h = *ctx->h_st;
+        if (h.done) break;
+        const double res = std::sqrt(h.rr);
+        brief = false;
+        launches = 1;
+        if (prev_res > 0 && res > 0 && h.tol > 0 && h.iter > prev_it) {
+            const double rate = std::log(res / prev_res) / double(h.iter - prev_it);
+            if (rate < 0) {
+                const double togo = std::log(h.tol / res) / rate;
+                brief = togo < 0.75 * kHeatGraphIters;
+                if (brief)
+                    launches = std::max(1, (int)(togo / kHeatGraphShort));
+                else
+                    launches = std::max(1, std::min(4, (int)(togo / (1.5 * kHeatGraphIters))));
+            }
+        }
+        prev_res = res;
+        prev_it = h.iter;
     }
-    const PcgScalars& h = *ctx->h_sc;
+    const Pcg1State& h = *ctx->h_st;
     if (iters) *iters = h.iter;
     if (resid) *resid = std::sqrt(h.rr);
     if (h.err) {  // NaN temperatures, as the direct solver's convention
@@ -183,13 +229,15 @@ int solve(tohip_heat* ctx, bool zero, double abstol, double reltol, int64_t maxi
 
 void free_heat(tohip_heat* ctx) {
     if (!ctx) return;
-    if (ctx->graph) hipGraphExecDestroy(ctx->graph);
-    void* bufs[] = {ctx->fixmask, ctx->fixv, ctx->x,     ctx->E,    ctx->dinv, ctx->u,
-                    ctx->r,       ctx->p[0], ctx->p[1],  ctx->q,    ctx->b,    ctx->t,
-                    ctx->lam,     ctx->cell, ctx->grad,  ctx->partA, ctx->partB, ctx->sc};
+    for (hipGraphExec_t ge : {ctx->graph, ctx->graph_short})
+        if (ge) hipGraphExecDestroy(ge);
+    void* bufs[] = {ctx->fixmask, ctx->fixv, ctx->x,    ctx->E,    ctx->dinv,    ctx->u,
+                    ctx->r[0],    ctx->r[1], ctx->p[0], ctx->p[1], ctx->q[0],    ctx->q[1],
+                    ctx->b,       ctx->t,    ctx->lam,  ctx->cell, ctx->grad,    ctx->part[0],
+                    ctx->part[1], ctx->st};
     for (void* b : bufs)
         if (b) hipFree(b);
-    if (ctx->h_sc) hipHostFree(ctx->h_sc);
+    if (ctx->h_st) hipHostFree(ctx->h_st);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -229,6 +277,7 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
         return TOHIP_ERR_ARG;
     }
     heat_ke(dim, h, k, ctx->ke);
+    heat_modes(dim, ctx->ke, ctx->modes);
     double tr = 0.0;
     for (int a = 0; a < (1 << dim); ++a) tr += ctx->ke.k[a * (1 << dim) + a];
     // matrix-free fixed-row rule: the sum of the element traces
@@ -267,14 +316,17 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
     if ((rc = halloc(ctx, &ctx->fixmask, n)) || (rc = halloc(ctx, &ctx->fixv, n)) ||
         (rc = halloc(ctx, &ctx->x, g.ncells)) || (rc = halloc(ctx, &ctx->E, g.ncells)) ||
         (rc = halloc(ctx, &ctx->dinv, n)) || (rc = halloc(ctx, &ctx->u, n)) ||
-        (rc = halloc(ctx, &ctx->r, n)) || (rc = halloc(ctx, &ctx->p[0], n)) ||
-        (rc = halloc(ctx, &ctx->p[1], n)) || (rc = halloc(ctx, &ctx->q, n)) ||
+        (rc = halloc(ctx, &ctx->r[0], n)) || (rc = halloc(ctx, &ctx->r[1], n)) ||
+        (rc = halloc(ctx, &ctx->p[0], n)) || (rc = halloc(ctx, &ctx->p[1], n)) ||
+        (rc = halloc(ctx, &ctx->q[0], n)) || (rc = halloc(ctx, &ctx->q[1], n)) ||
         (rc = halloc(ctx, &ctx->b, n)) || (rc = halloc(ctx, &ctx->t, n)) ||
         (rc = halloc(ctx, &ctx->lam, n)) || (rc = halloc(ctx, &ctx->cell, g.ncells)) ||
-        (rc = halloc(ctx, &ctx->grad, g.ncells)) || (rc = halloc(ctx, &ctx->partA, kMaxPartials)) ||
-        (rc = halloc(ctx, &ctx->partB, 2 * kMaxPartials)) || (rc = halloc(ctx, &ctx->sc, 1)))
+        (rc = halloc(ctx, &ctx->grad, g.ncells)) || 
+        (rc = halloc(ctx, &ctx->part[0], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
+        (rc = halloc(ctx, &ctx->part[1], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
+        (rc = halloc(ctx, &ctx->st, 2)))
         return rc;
-    HCK(hipHostMalloc((void**)&ctx->h_sc, sizeof(PcgScalars), hipHostMallocDefault));
+    HCK(hipHostMalloc((void**)&ctx->h_st, sizeof(Pcg1State), hipHostMallocDefault));
     HCK(hipMemcpyAsync(ctx->fixmask, mask.data(), n, hipMemcpyHostToDevice, ctx->stream));
     HCK(hipMemcpyAsync(ctx->fixv, vals.data(), n * sizeof(double), hipMemcpyHostToDevice,
                        ctx->stream));
@@ -282,8 +334,6 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
     HCK(hipMemcpyAsync(ctx->x, ones.data(), g.ncells * sizeof(double), hipMemcpyHostToDevice,
                        ctx->stream));
     HCK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
-    HCK(hipMemsetAsync(ctx->p[0], 0, n * sizeof(double), ctx->stream));
-    HCK(hipMemsetAsync(ctx->p[1], 0, n * sizeof(double), ctx->stream));
     if ((rc = refresh(ctx))) return rc;
     HCK(hipStreamSynchronize(ctx->stream));
     return 0;
@@ -348,9 +398,9 @@ int tohip_heat_set_densities(tohip_heat* ctx, const double* vars) {
 int tohip_heat_matvec(tohip_heat* ctx, const double* x, double* y) {
     if (!ctx || !x || !y) return TOHIP_ERR_ARG;
     if (int rc = upload_nodes(ctx, x, ctx->t)) return rc;
-    HCK(launch_heat_matvec(ctx->g, ctx->ke, ctx->t, ctx->fixmask, ctx->E, ctx->meandiag, ctx->q,
+    HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->t, ctx->fixmask, ctx->E, ctx->meandiag, ctx->q[0],
                            0, ctx->stream));
-    return download_nodes(ctx, ctx->q, y);
+    return download_nodes(ctx, ctx->q[0], y);
 }
 
 int tohip_heat_solve(tohip_heat* ctx, const double* rhs, double* T, double abstol, double reltol,
@@ -366,12 +416,12 @@ int tohip_heat_solve(tohip_heat* ctx, const double* rhs, double* T, double absto
         ctx->err = "tohip_heat_solve: non-finite right-hand side or initial guess";
         return TOHIP_ERR_ARG;
     }
-    if (int rc = upload_nodes(ctx, rhs, ctx->q)) return rc;
+    if (int rc = upload_nodes(ctx, rhs, ctx->q[0])) return rc;
     const bool lift = apply_dirichlet && ctx->inhom;
     if (lift)
-        HCK(launch_heat_matvec(ctx->g, ctx->ke, ctx->fixv, ctx->fixmask, ctx->E, ctx->meandiag,
+        HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->fixv, ctx->fixmask, ctx->E, ctx->meandiag,
                                ctx->t, 2, ctx->stream));
-    HCK(launch_heat_rhs(n, ctx->q, lift ? ctx->t : nullptr, ctx->fixmask, ctx->fixv,
+    HCK(launch_heat_rhs(n, ctx->q[0], lift ? ctx->t : nullptr, ctx->fixmask, ctx->fixv,
                         ctx->meandiag, lift ? 1 : 0, ctx->b, ctx->stream));
     if (!initially_zero)
         if (int rc = upload_nodes(ctx, T, ctx->u)) return rc;
@@ -400,12 +450,12 @@ int tohip_heat_bench_matvec(tohip_heat* ctx, int reps, double* avg_us) {
     hipEvent_t e0, e1;
     HCK(hipEventCreate(&e0));
     HCK(hipEventCreate(&e1));
-    HCK(launch_heat_matvec(ctx->g, ctx->ke, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag, ctx->q,
+    HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag, ctx->q[0],
                            0, ctx->stream));  // warm-up
     HCK(hipEventRecord(e0, ctx->stream));
     for (int i = 0; i < reps; ++i)
-        HCK(launch_heat_matvec(ctx->g, ctx->ke, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag,
-                               ctx->q, 0, ctx->stream));
+        HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->u, ctx->fixmask, ctx->E, ctx->meandiag,
+                               ctx->q[0], 0, ctx->stream));
     HCK(hipEventRecord(e1, ctx->stream));
     HCK(hipEventSynchronize(e1));
     float ms = 0;

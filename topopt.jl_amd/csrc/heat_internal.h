@@ -5,7 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "tohip_internal.h"
+#include "k_pcg1.h"
 
 namespace tohip {
 
@@ -22,21 +22,24 @@ struct HeatKe {
     double k[64];
 };
 
+// Its eigenvalues in the corners' Hadamard basis over the number of corners:
+// Ke = H diag(b) H^T, mode m's vector prod_{a in m} (2 bit_a(c) - 1).
+struct HeatModes {
+    double b[8];
+};
+
 // y = K x over the nodes.  mode 0: the solver's operator (x masked to 0 at
 // fixed nodes inside the element products, fixed rows y = meandiag * x);
 // mode 2: the full operator (no masking; the Dirichlet lift K v).
-hipError_t launch_heat_matvec(const HeatGrid& g, const HeatKe& ke, const double* x,
+hipError_t launch_heat_matvec(const HeatGrid& g, const HeatModes& B, const double* x,
                               const uint8_t* fixmask, const double* E, double meandiag, double* y,
                               int mode, hipStream_t s);
 
-// PCG direction + matvec (iteration k = iter + 1): launch_pcg_direction
-// (convergence test, p_k = dinv .* r + beta p_{k-1} into p[k & 1]), then
-// q = K p_k (mode 0) with per-block p.q partials into partA (*nbA blocks).
-hipError_t launch_heat_dirmatvec(const HeatGrid& g, const HeatKe& ke, const double* r,
-                                 const double* dinv, double* p0, double* p1, double* q,
-                                 const uint8_t* fixmask, const double* E, double meandiag,
-                                 PcgScalars* sc, const double* partB, int nbB, double* partA,
-                                 int* nbA, hipStream_t s);
+// One PCG iteration in one launch (k_pcg1.h) on the mode 0 operator;
+// a.nb = heat_pcg_blocks(g).
+int heat_pcg_blocks(const HeatGrid& g);
+hipError_t launch_heat_pcg(const HeatGrid& g, const HeatModes& B, const uint8_t* fixmask,
+                           const double* E, double meandiag, const Pcg1Args& a, hipStream_t s);
 
 // E_e = rho(x_e) (get_rho with the penalty), dinv = 1 / diag(K) (free nodes:
 // sum of E_c Ke[a][a]; fixed nodes: 1 / meandiag).

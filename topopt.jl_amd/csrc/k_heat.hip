@@ -4,10 +4,11 @@
 // for the matrix-free product and its fixed-DOF rule).
 //
 // One DOF per node; K = sum_e rho_e Ke with one shared Ke (k * grad phi_a .
-// grad phi_b integrated over the box cell).  A node's row gathers the 4 (2D)
-// or 8 (3D) cells around it, each a 4- or 8-term row of Ke, in a fixed order
-// (one thread per node: deterministic, no atomics).  The kernels are
-// HBM-bound gathers; the 27-point neighbourhood is served from L2.
+// grad phi_b integrated over the box cell).  Ke is a sum of Kronecker products
+// of 1D stiffness and mass matrices, which the +-1 (Hadamard) basis of the
+// corners diagonalises: Ke = H B H^T with B diagonal.
+#include <algorithm>
+
 #include "heat_internal.h"
 #include "k_common.h"
 
@@ -18,73 +19,271 @@ __device__ __forceinline__ int heat_corner(int ox, int oy, int oz) {
     return (oy ? (ox ? 2 : 3) : (ox ? 1 : 0)) + 4 * oz;
 }
 
-// MODE 0: y = K x (masked columns, fixed rows md x); MODE 1: PCG, q = K p_k
-// with p_k = p[k & 1] written by the direction kernel, per-block p.q partials
-// into partA, a no-op once `done`; MODE 2: y = K_full x (no masking).
-template <int DIM, int MODE>
-__global__ __launch_bounds__(kThreads) void k_heat_matvec(
-    HeatGrid g, HeatKe ke, const double* __restrict__ x0, const double* __restrict__ x1,
-    const uint8_t* __restrict__ fixmask, const double* __restrict__ E, double md,
-    double* __restrict__ y, const PcgScalars* sc, double* __restrict__ partA) {
-    __shared__ double red[kWaves];
-    constexpr int NC = DIM == 3 ? 8 : 4;
-    const double* x = x0;
-    if (MODE == 1) {
-        if (sc->done) return;
-        x = (sc->k_cur & 1) ? x1 : x0;
-    }
-    double part = 0.0;
-    for (int64_t n = blockIdx.x * (int64_t)kThreads + threadIdx.x; n < g.nnodes;
-         n += (int64_t)gridDim.x * kThreads) {
-        const int i = (int)(n % g.NX), j = (int)((n / g.NX) % g.NY);
-        const int k = DIM == 3 ? (int)(n / ((int64_t)g.NX * g.NY)) : 0;
-        const double vn = x[n];
-        double yn = 0.0;
-        if (MODE != 2 && fixmask[n]) {
-            yn = md * vn;
+// ---- the operator, alone and inside one-launch PCG ----
+//
+// A 256-thread workgroup owns a column of 15 x 15 output nodes and, in 3D, a
+// chunk of node planes that it walks upwards; 2D is one plane.  Thread (ci, cj)
+// stages node (ci, cj) of the column's 17 x 17 nodes (a one-node halo; threads
+// 0..32 the far row and column too) and handles cell (ci, cj) of the 16 x 16
+// cells.  Per plane: values to LDS with prescribed nodes zeroed; each thread
+// transforms its cell's four nodes to the xy Hadamard basis; the layer's cells
+// are the sum and difference with the transform of the plane below, scaled by
+// E B; the part of the upper plane stays in registers, the lower plane's total
+// is transformed back.  A node's four cell columns are summed as two x-pairs (a
+// DPP row shift brings the left cell's value, a row of 16 lanes is a row of
+// cells) and an LDS exchange between the rows: lower row first.  No atomics,
+// the same bits every run.  About 50 FP64 operations and 7 LDS accesses a cell
+// in place of 64 products and 27 bounds-tested loads a node.
+//
+// One launch is a whole PCG iteration.  Bound by latency on small grids, by the
+// cache traffic of its 4 vectors in (1.3 x (zc + 2) / zc with the halo) and 4
+// out on larger ones.  MI355X, one iteration: 128x96x80 26 us (direction, a
+// 27-point gather of K p and update in three launches: 85 us; the 57 MB it must
+// move take 12 us at the copy rate), 80x60 6.0 us (14 us).
+constexpr int kHC = 16, kHO = kHC - 1, kHS = kHC + 1;
+
+__device__ __forceinline__ double heat_row_shr1(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x111, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x111, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Columns of 15 x 15 nodes and chunks of zc planes, about 768 workgroups (the
+// PCG kernel's 139 VGPRs let three run per CU) when the grid has them; at most
+// kMaxPartials launch and stride over the rest.  Fewer planes a chunk fill the
+// chip better but re-stage more (zc + 2 planes each): at 128x96x80, with 504 /
+// 693 / 756 / 882 / 1008 workgroups, a PCG iteration took 25.2 / 28.2 / 25.9 /
+// 33.5 / 33.6 us.
+struct HeatShape {
+    int ncx, ncy, zc, nch, nwork;
+};
+static HeatShape heat_shape(const HeatGrid& g) {
+    HeatShape s;
+    s.ncx = (g.NX + kHO - 1) / kHO;
+    s.ncy = (g.NY + kHO - 1) / kHO;
+    const int64_t cols = (int64_t)s.ncx * s.ncy;
+    const int64_t want = std::max<int64_t>(1, 768 / cols);
+    s.zc = (int)std::max<int64_t>(std::min(2, g.NZ), (g.NZ + want - 1) / want);
+    s.nch = (g.NZ + s.zc - 1) / s.zc;
+    s.nwork = (int)(cols * s.nch);
+    return s;
+}
+static int heat_op_blocks(const HeatShape& s) { return std::min(s.nwork, kMaxPartials); }
+int heat_pcg_blocks(const HeatGrid& g) { return heat_op_blocks(heat_shape(g)); }
+
+// A staged node: in the mesh or not, its operands.
+struct HeatNode {
+    double v, r, q, d;  // MODE 1: v = p; otherwise v = x
+    uint8_t m;
+    bool in;
+};
+
+// MODE 0: y = K x (prescribed nodes masked, their rows md x); MODE 1: one
+// PCG iteration (k_pcg1.h); MODE 2: y = K_full x (no masking).
+template <int DIM, int MODE, typename Off>
+__global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, HeatShape sh,
+                                                      const double* __restrict__ xin,
+                                                      const uint8_t* __restrict__ fixmask,
+                                                      const double* __restrict__ E, double md,
+                                                      double* __restrict__ y, Pcg1Args a) {
+    __shared__ double pl[2][kHS * kHS];
+    __shared__ double exch[kThreads];
+    __shared__ double red[kWaves][kPcg1Vals];
+    const int tid = threadIdx.x, ci = tid & (kHC - 1), cj = tid / kHC;
+    // the second node of threads 0..32: the far column, then the far row
+    const bool two = tid < 2 * kHC + 1;
+    const int li2 = tid <= kHC ? kHC : tid - kHS, lj2 = tid <= kHC ? tid : kHC;
+    Pcg1Plan plan{0.0, 0.0, kPcg1Step};
+    bool pend = false, update = true;  // an update is pending; and may be applied
+
+    // A node's (cell's) place: a base that is the same for the whole workgroup,
+    // advanced by a plane a step, and an offset in bytes within the column's
+    // plane that stays, so that an access costs no vector address arithmetic.
+    int i0 = 0, j0 = 0;
+    Off oa = 0, ob = 0, oe = 0;  // of the two nodes and the cell
+    auto at64 = [](auto* p, int64_t base, Off o) -> auto& {
+        using T = std::remove_pointer_t<decltype(p)>;
+        using C = std::conditional_t<std::is_const<T>::value, const char, char>;
+        return *reinterpret_cast<T*>(reinterpret_cast<C*>(p + base) + o);
+    };
+    bool ina = false, inb = false, ine = false;
+    int64_t nbase = 0, ebase = 0;
+    auto load = [&](Off o, bool in, int k) {
+        const int nk = DIM == 3 ? min(max(k, 0), g.NZ - 1) : 0;
+        const int64_t base = nbase + (int64_t)nk * g.NX * g.NY;
+        HeatNode h;
+        h.in = in && (DIM == 2 || k == nk);
+        h.m = MODE == 2 ? 0 : at64(fixmask, base, o / 8);
+        if (MODE == 1) {
+            h.v = at64(a.p, base, o);
+            h.r = at64(a.r, base, o);
+            h.q = at64(a.q, base, o);
+            h.d = at64(a.dinv, base, o);
         } else {
-            // the 3^DIM neighbourhood once (masked, 0 outside the grid), then
-            // the 2^DIM cells around the node, each a row of Ke
-            constexpr int NN = DIM == 3 ? 27 : 9;
-            double xv[NN];
-#pragma unroll
-            for (int q = 0; q < NN; ++q) {
-                const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = DIM == 3 ? q / 9 - 1 : 0;
-                const int mi = i + dx, mj = j + dy, mk = k + dz;
-                double v = 0.0;
-                if (mi >= 0 && mi < g.NX && mj >= 0 && mj < g.NY &&
-                    (DIM == 2 || (mk >= 0 && mk < g.NZ))) {
-                    const int64_t m = mi + (int64_t)g.NX * (mj + (int64_t)g.NY * mk);
-                    v = (MODE != 2 && fixmask[m]) ? 0.0 : (m == n ? vn : x[m]);
-                }
-                xv[q] = v;
-            }
-#pragma unroll
-            for (int cq = 0; cq < NC; ++cq) {
-                // cell origin offset (ox - 1, oy - 1, oz - 1) relative to the node
-                const int ox = cq & 1, oy = (cq >> 1) & 1, oz = cq >> 2;
-                const int cx = i - 1 + ox, cy = j - 1 + oy, cz = DIM == 3 ? k - 1 + oz : 0;
-                if (cx < 0 || cx >= g.nx || cy < 0 || cy >= g.ny ||
-                    (DIM == 3 && (cz < 0 || cz >= g.nz)))
-                    continue;
-                const int a = heat_corner(1 - ox, 1 - oy, DIM == 3 ? 1 - oz : 0);
-                double t = 0.0;
-#pragma unroll
-                for (int b = 0; b < NC; ++b) {
-                    const int bx = (b & 1) ^ ((b >> 1) & 1), by = (b >> 1) & 1, bz = b >> 2;
-                    // corner b of the cell is node offset (ox - 1 + bx, ...) from n
-                    const int q = (ox + bx) + 3 * ((oy + by) + 3 * (DIM == 3 ? oz + bz : 0));
-                    t += ke.k[a * NC + b] * xv[q];
-                }
-                yn += E[cx + (int64_t)g.nx * (cy + (int64_t)g.ny * cz)] * t;
-            }
+            h.v = at64(xin, base, o);
         }
-        y[n] = yn;
-        if (MODE == 1) part += vn * yn;
+        return h;
+    };
+    auto load_E = [&](int k) {  // the cell of this thread in layer k (0 outside the mesh)
+        const bool in = ine && (DIM == 2 || (k >= 0 && k < g.nz));
+        const int64_t base = ebase + (int64_t)(DIM == 3 ? min(max(k, 0), g.nz - 1) : 0) * g.nx * g.ny;
+        const double e = at64(E, base, oe);
+        return in ? e : 0.0;
+    };
+    double sum[kPcg1Vals] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int buf = 0;
+    bool first = true;
+    for (int w = blockIdx.x; w < sh.nwork; w += gridDim.x) {
+        const int wr = xcd_remap(w, sh.nwork);
+        const int ncol = sh.ncx * sh.ncy, col = wr % ncol, ch = wr / ncol;
+        i0 = (col % sh.ncx) * kHO;
+        j0 = (col / sh.ncx) * kHO;
+        const int kb = DIM == 3 ? ch * sh.zc : 0, ke = DIM == 3 ? min(kb + sh.zc, g.NZ) : 1;
+        const int gi = i0 - 1 + ci, gj = j0 - 1 + cj;
+        const bool mine = ci >= 1 && cj >= 1 && gi < g.NX && gj < g.NY;
+        {
+            const int bi = max(i0 - 1, 0), bj = max(j0 - 1, 0);
+            auto place = [&](int li, int lj, bool& in) {
+                const int x = i0 - 1 + li, y = j0 - 1 + lj;
+                const int cx = min(max(x, 0), g.NX - 1), cy = min(max(y, 0), g.NY - 1);
+                in = x == cx && y == cy;
+                return 8 * ((Off)(cx - bi) + (Off)g.NX * (Off)(cy - bj));
+            };
+            nbase = bi + (int64_t)g.NX * bj;
+            ebase = bi + (int64_t)g.nx * bj;
+            oa = place(ci, cj, ina);
+            ob = place(two ? li2 : 0, two ? lj2 : 0, inb);
+            ine = gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny;
+            oe = ine ? 8 * ((Off)(gi - bi) + (Off)g.nx * (Off)(gj - bj)) : 0;
+        }
+        auto plane = [&](int k) { return nbase + (int64_t)(DIM == 3 ? k : 0) * g.NX * g.NY; };
+        const int sb = DIM == 3 ? kb - 1 : 0, se = DIM == 3 ? ke : 0;  // staged planes
+        HeatNode na = load(oa, ina, sb), nb{};
+        if (two) nb = load(ob, inb, sb);
+        double xa = 0.0;
+        if (MODE == 1 && mine && sb >= kb) xa = at64(a.x, plane(sb), oa);
+        double en = DIM == 3 ? 0.0 : load_E(0);
+        if (MODE == 1 && first) {
+            // the first plane's loads are in flight while the sums are formed
+            first = false;
+            const Pcg1State s0 = *a.s;
+            if (s0.done) {
+                if (blockIdx.x == 0 && tid == 0) *a.sn = s0;
+                return;
+            }
+            double v[kPcg1Vals];
+            pcg1_reduce<kThreads>(a.part, a.nb, v, red);
+            Pcg1State s1;
+            plan = pcg1_plan(s0, v, s1);
+            if (blockIdx.x == 0 && tid == 0) *a.sn = s1;
+            pend = s0.pend != 0;
+            update = s1.err == 0 || s0.iter != s1.iter;
+        }
+        if (MODE == 1 && plan.mode != kPcg1Step) {
+            // the pending update alone: x, and (exact) r with its two sums
+            if (update) {
+                for (int k = kb; k < ke; ++k) {
+                    if (!mine) break;
+                    const int64_t n = plane(k);
+                    const double p = at64(a.p, n, oa);
+                    if (pend) at64(a.x, n, oa) += plan.alpha * p;
+                    if (plan.mode == kPcg1Exact) {
+                        const double r = fma(-plan.alpha, at64(a.q, n, oa), at64(a.r, n, oa));
+                        at64(a.rn, n, oa) = r;
+                        at64(a.pn, n, oa) = p;
+                        sum[kSumRZ] += at64(a.dinv, n, oa) * r * r;
+                        sum[kSumRR] += r * r;
+                    }
+                }
+            }
+            continue;
+        }
+        double fp[4] = {0, 0, 0, 0}, up[4] = {0, 0, 0, 0};
+        double po = 0.0, ro = 0.0, dd = 0.0;  // own node of the plane below
+        uint8_t mo = 0;
+        for (int k = sb; k <= se; ++k) {
+            // direction (or input) of this plane, then the next plane's loads
+            auto value = [&](HeatNode& h) {
+                if (MODE == 1) {
+                    // explicit FMAs: a halo copy and its owner get the same bits
+                    h.r = fma(-plan.alpha, pend ? h.q : 0.0, h.r);
+                    h.v = fma(plan.beta, h.v, h.d * h.r);
+                }
+                return (h.in && !h.m) ? h.v : 0.0;
+            };
+            const double pold = na.v;
+            const double va = value(na);
+            pl[buf][ci + kHS * cj] = va;
+            if (two) pl[buf][li2 + kHS * lj2] = value(nb);
+            if (MODE == 1 && mine && k >= kb && k < ke) {
+                const int64_t n = plane(k);
+                if (pend) at64(a.x, n, oa) = xa + plan.alpha * pold;
+                at64(a.rn, n, oa) = na.r;
+                at64(a.pn, n, oa) = na.v;
+            }
+            const double ec = en;
+            const HeatNode cur = na;
+            if (k < se) {
+                na = load(oa, ina, k + 1);
+                if (two) nb = load(ob, inb, k + 1);
+                if (MODE == 1 && mine && k + 1 >= kb && k + 1 < ke) xa = at64(a.x, plane(k + 1), oa);
+                en = load_E(k);
+            }
+            __syncthreads();
+            double f[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) f[c] = pl[buf][ci + (c & 1) + kHS * (cj + (c >> 1))];
+            buf ^= 1;
+            hadamard_fwd<double, 2>(f);
+            if (DIM == 2 || k > sb) {
+                double lo[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    if (DIM == 3) {
+                        const double z0 = ec * B.b[m] * (fp[m] + f[m]);
+                        const double z1 = ec * B.b[m + 4] * (f[m] - fp[m]);
+                        lo[m] = up[m] + (z0 - z1);
+                        up[m] = z0 + z1;
+                    } else {
+                        lo[m] = ec * B.b[m] * f[m];
+                    }
+                }
+                hadamard_inv<double, 2>(lo);
+                const double y0 = heat_row_shr1(lo[1]) + lo[0];
+                exch[tid] = heat_row_shr1(lo[3]) + lo[2];
+                __syncthreads();
+                const int ko = DIM == 3 ? k - 1 : 0;
+                if (mine && ko >= kb && ko < ke) {
+                    const double p = DIM == 3 ? po : cur.v, r = DIM == 3 ? ro : cur.r,
+                                 d = DIM == 3 ? dd : cur.d;
+                    double q = exch[tid - kHC] + y0;
+                    if (MODE != 2 && (DIM == 3 ? mo : cur.m)) q = md * p;
+                    if (MODE == 1) {
+                        at64(a.qn, plane(ko), oa) = q;
+                        const double z = d * r, dq = d * q;
+                        sum[kSumRZ] += z * r;
+                        sum[kSumPQ] += p * q;
+                        sum[kSumQZ] += z * q;
+                        sum[kSumQDQ] += dq * q;
+                        sum[kSumRR] += r * r;
+                        sum[kSumRQ] += r * q;
+                        sum[kSumQQ] += q * q;
+                    } else {
+                        at64(y, plane(ko), oa) = q;
+                    }
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 4; ++m) fp[m] = f[m];
+            po = cur.v;
+            ro = cur.r;
+            dd = cur.d;
+            mo = cur.m;
+        }
     }
     if (MODE == 1) {
-        const double s = block_sum_all(part, red);
-        if (threadIdx.x == 0) partA[blockIdx.x] = s;
+        pcg1_store_sums(sum, red, a.partn);
     }
 }
 
@@ -95,38 +294,38 @@ static unsigned heat_blocks(int64_t n) {
     return (unsigned)b;
 }
 
-hipError_t launch_heat_matvec(const HeatGrid& g, const HeatKe& ke, const double* x,
-                              const uint8_t* fixmask, const double* E, double meandiag, double* y,
-                              int mode, hipStream_t s) {
-    const dim3 grid(heat_blocks(g.nnodes)), block(kThreads);
-#define TOHIP_HEAT(D, M)                                                                        \
-    hipLaunchKernelGGL((k_heat_matvec<D, M>), grid, block, 0, s, g, ke, x, x, fixmask, E,       \
-                       meandiag, y, nullptr, nullptr)
-    if (g.dim == 3) {
-        if (mode == 2) TOHIP_HEAT(3, 2); else TOHIP_HEAT(3, 0);
-    } else {
-        if (mode == 2) TOHIP_HEAT(2, 2); else TOHIP_HEAT(2, 0);
-    }
-#undef TOHIP_HEAT
+// The kernel's 32-bit offsets span the 17 rows of a column's plane.
+template <int DIM, int MODE>
+static hipError_t launch_heat_op(const HeatGrid& g, const HeatModes& B, const double* x,
+                                 const uint8_t* fixmask, const double* E, double meandiag,
+                                 double* y, const Pcg1Args& a, hipStream_t s) {
+    const HeatShape sh = heat_shape(g);
+    const dim3 grid(heat_op_blocks(sh)), block(kThreads);
+    if ((int64_t)g.NX * kHS * 8 < ((int64_t)1 << 32))
+        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint32_t>), grid, block, 0, s, g, B, sh, x,
+                           fixmask, E, meandiag, y, a);
+    else
+        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint64_t>), grid, block, 0, s, g, B, sh, x,
+                           fixmask, E, meandiag, y, a);
     return hipGetLastError();
 }
 
-hipError_t launch_heat_dirmatvec(const HeatGrid& g, const HeatKe& ke, const double* r,
-                                 const double* dinv, double* p0, double* p1, double* q,
-                                 const uint8_t* fixmask, const double* E, double meandiag,
-                                 PcgScalars* sc, const double* partB, int nbB, double* partA,
-                                 int* nbA, hipStream_t s) {
-    if (hipError_t e = launch_pcg_direction(g.nnodes, r, dinv, p0, p1, sc, partB, nbB, s))
-        return e;
-    const unsigned nb = heat_blocks(g.nnodes);
+hipError_t launch_heat_matvec(const HeatGrid& g, const HeatModes& B, const double* x,
+                              const uint8_t* fixmask, const double* E, double meandiag, double* y,
+                              int mode, hipStream_t s) {
+    const Pcg1Args a{};
     if (g.dim == 3)
-        hipLaunchKernelGGL((k_heat_matvec<3, 1>), dim3(nb), dim3(kThreads), 0, s, g, ke, p0, p1,
-                           fixmask, E, meandiag, q, sc, partA);
-    else
-        hipLaunchKernelGGL((k_heat_matvec<2, 1>), dim3(nb), dim3(kThreads), 0, s, g, ke, p0, p1,
-                           fixmask, E, meandiag, q, sc, partA);
-    if (nbA) *nbA = (int)nb;
-    return hipGetLastError();
+        return mode == 2 ? launch_heat_op<3, 2>(g, B, x, fixmask, E, meandiag, y, a, s)
+                         : launch_heat_op<3, 0>(g, B, x, fixmask, E, meandiag, y, a, s);
+    return mode == 2 ? launch_heat_op<2, 2>(g, B, x, fixmask, E, meandiag, y, a, s)
+                     : launch_heat_op<2, 0>(g, B, x, fixmask, E, meandiag, y, a, s);
+}
+
+hipError_t launch_heat_pcg(const HeatGrid& g, const HeatModes& B, const uint8_t* fixmask,
+                           const double* E, double meandiag, const Pcg1Args& a, hipStream_t s) {
+    return g.dim == 3
+               ? launch_heat_op<3, 1>(g, B, nullptr, fixmask, E, meandiag, nullptr, a, s)
+               : launch_heat_op<2, 1>(g, B, nullptr, fixmask, E, meandiag, nullptr, a, s);
 }
 
 __global__ void k_heat_density(int64_t ncells, const double* __restrict__ x, double xmin,

@@ -10,7 +10,7 @@
 // a fixed order (see k_common.h), so a solve is bitwise reproducible.  Once
 // `done` is set every later PCG kernel returns at once, which lets the host
 // replay a captured multi-iteration graph without checking in between.
-#include "k_common.h"
+#include "k_pcg1.h"
 
 namespace tohip {
 
@@ -179,6 +179,35 @@ template hipError_t launch_pcg_update_from<float>(int64_t, float*, const float*,
                                                   const float*, const float*, const float*,
                                                   const float*, PcgScalars*, const double*, int,
                                                   double*, hipStream_t);
+
+// ---- one-launch PCG (k_pcg1.h) ----
+
+// r = b - Ax (Ax may be null: x = 0), p = 0 and the rows of (r.z, r.r) that the
+// first launch reduces, from as many workgroups as it has rows.
+__global__ __launch_bounds__(kThreads) void k_pcg1_start(int64_t n, const double* __restrict__ b,
+                                                         const double* __restrict__ Ax,
+                                                         const double* __restrict__ dinv,
+                                                         double* __restrict__ r,
+                                                         double* __restrict__ p,
+                                                         double* __restrict__ part) {
+    __shared__ double red[kWaves][kPcg1Vals];
+    double sum[kPcg1Vals] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * kThreads) {
+        const double ri = Ax ? b[i] - Ax[i] : b[i];
+        r[i] = ri;
+        p[i] = 0.0;
+        sum[kSumRZ] += dinv[i] * ri * ri;
+        sum[kSumRR] += ri * ri;
+    }
+    pcg1_store_sums(sum, red, part);
+}
+
+hipError_t launch_pcg1_start(int64_t n, const double* b, const double* Ax, const double* dinv,
+                             double* r, double* p, double* part, int nb, hipStream_t s) {
+    hipLaunchKernelGGL(k_pcg1_start, dim3(nb), dim3(kThreads), 0, s, n, b, Ax, dinv, r, p, part);
+    return hipGetLastError();
+}
 
 // ---- EnergyCriteria (TopOpt.jl src/FEA/convergence_criteria.jl:26-45) ----
 // IterativeSolvers evaluates the criterion before every iteration on the
