@@ -47,3 +47,38 @@ def test_heat_maxiter_and_zero_load(T, gpu):
         assert s.last_iters == n and not s.converged
     s(rhs=np.zeros(prob.ndofs))
     assert s.last_iters == 0 and s.converged and not np.any(s.lhs)
+
+
+# 2D; 3D by planes (at most 256 of them over all columns) and marching chunks
+# (the last two), cubes and boxes, tiles of 15 nodes cut at every remainder
+ELASTIC = [((1, 2), None), ((14, 14), (1.0, 0.5)), ((15, 16), None), ((61, 30), (1.0, 1.5)),
+           ((1, 2, 2), None), ((14, 14, 2), None), ((15, 16, 4), (1.0, 1.5, 0.75)),
+           ((29, 14, 8), None), ((17, 46, 44), None), ((31, 44, 22), (1.0, 0.5, 1.25))]
+
+
+@pytest.mark.parametrize("case", range(len(ELASTIC)))
+def test_elastic_tiles(T, O, gpu, case):
+    nels, h = ELASTIC[case]
+    prob = T.PointLoadCantilever(nels, sizes=h)
+    s = T.FEASolver(T.HIPMatrixFreeSolver, prob, penalty=T.PowerPenaltyFun(3.0), abstol=0.0,
+                    reltol=1e-12, cg_max_iter=20000)
+    orc = O.Oracle(O.Cantilever(tuple(nels)), p=3.0, h=h)
+    x = np.random.default_rng(case).uniform(0.5, 1.0, prob.ncells)
+    s.vars = x
+    orc.set_vars(x)
+    s()
+    assert s.converged
+    free = ~prob.fixed.astype(bool)
+    # the true residual of the recursive 1e-12: its drift on 1 : 2 boxes is a few 1e-10
+    f = prob.f
+    assert np.linalg.norm((f - orc.matvec(s.u))[free]) <= 1e-9 * np.linalg.norm(f)
+    u, it = s.u.copy(), s.last_iters
+    # the same solve again: the same bits; a warm start from its answer: at once
+    s()
+    assert s.last_iters == it and np.array_equal(s.u, u)
+    s(initially_zero=False, reltol=1.0)
+    assert s.last_iters == 0 and np.array_equal(s.u, u)
+    for n in (0, 1, 2, 3):
+        if n < it:
+            s(maxiter=n)
+            assert s.last_iters == n and not s.converged

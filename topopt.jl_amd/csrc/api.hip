@@ -10,7 +10,6 @@
 #include <limits>
 #include <mutex>
 #include <string>
-#include <type_traits>
 #include <vector>
 
 #include "../../include/topopt_hip.h"
@@ -647,11 +646,9 @@ hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, d
 // One captured PCG graph: `iters` x (direction+matvec, update).  The
 // kernels pick their buffers and parity from the device iteration counter,
 // so a graph can be replayed from any iteration.
-// With `ec` (FP64 only) each iteration ends with the EnergyCriteria check.
 template <typename T>
 int capture_pcg_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters, const ElemOp<T>& op, T* x,
-                      T* r, T* dinv, T** p, T* q, const T* E, PcgScalars* sc,
-                      EnergyCrit* ec = nullptr) {
+                      T* r, T* dinv, T** p, T* q, const T* E, PcgScalars* sc) {
     if (*exec) return 0;
     hipGraph_t graph;
     CK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
@@ -662,10 +659,6 @@ int capture_pcg_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters, const Ele
                                                 ctx->partA, &nbA, ctx->stream);
         hipError_t e2 = launch_pcg_update<T>(ctx->g.ndof, x, r, p[0], p[1], q, dinv, sc,
                                              ctx->partA, nbA, ctx->partB, ctx->stream);
-        if constexpr (std::is_same<T, double>::value)
-            if (ec && e2 == hipSuccess)
-                e2 = launch_energy_check(ctx->g.ndof, x, r, ctx->b64, sc, ec, ctx->partials,
-                                         ctx->stream);
         if (e1 != hipSuccess || e2 != hipSuccess) {
             hipStreamEndCapture(ctx->stream, &graph);
             ctx->err = "PCG graph capture failed";
@@ -793,11 +786,10 @@ int replay_pcg_graphs(tohip_ctx* ctx, hipGraphExec_t big, hipGraphExec_t small, 
 template <typename T>
 int run_pcg_graphs(tohip_ctx* ctx, hipGraphExec_t* big, hipGraphExec_t* small,
                    const ElemOp<T>& op, T* x, T* r, T* dinv, T** p, T* q, const T* E,
-                   PcgScalars* sc, EnergyCrit* ec = nullptr) {
-    if (int rc = capture_pcg_graph<T>(ctx, big, kGraphItersBig, op, x, r, dinv, p, q, E, sc, ec))
+                   PcgScalars* sc) {
+    if (int rc = capture_pcg_graph<T>(ctx, big, kGraphItersBig, op, x, r, dinv, p, q, E, sc))
         return rc;
-    if (int rc =
-            capture_pcg_graph<T>(ctx, small, kGraphItersSmall, op, x, r, dinv, p, q, E, sc, ec))
+    if (int rc = capture_pcg_graph<T>(ctx, small, kGraphItersSmall, op, x, r, dinv, p, q, E, sc))
         return rc;
     return replay_pcg_graphs(ctx, *big, *small, kGraphItersBig, sc);
 }
@@ -833,60 +825,110 @@ int pcg_breakdown(tohip_ctx* ctx, int err) {
     return TOHIP_BREAKDOWN;
 }
 
-// Device-resident Jacobi PCG on K(E) x = b.  x is the initial guess when
-// !initially_zero.  Returns 0, or TOHIP_NOT_CONVERGED.  Under EnergyCriteria
-// (ctx->conv_kind) the residual test is off and the energy test with
-// tolerance `etol` stops the iteration; it is evaluated on the starting
-// iterate too, as IterativeSolvers evaluates its stopping test before every
-// iteration; a NaN or negative energy returns TOHIP_ERR_DOMAIN.
+// One captured graph of `iters` one-launch PCG iterations (even), each followed by
+// the EnergyCriteria check when `energy`.
+int capture_pcg1_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters, bool energy) {
+    if (*exec) return 0;
+    double *r[2] = {ctx->r64, ctx->r64b}, *q[2] = {ctx->q64, ctx->t64};
+    hipGraph_t graph;
+    CK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    for (int it = 0; it < iters; ++it) {
+        const int i = it & 1, o = i ^ 1;
+        const Pcg1Args a{ctx->u,           r[i],
+                         ctx->p64[i],      q[i],
+                         ctx->dinv64,      r[o],
+                         ctx->p64[o],      q[o],
+                         ctx->pcg1_st + i, ctx->pcg1_st + o,
+                         ctx->pcg1_part[i], ctx->pcg1_part[o],
+                         pcg1_blocks(ctx->g)};
+        if (launch_pcg1(ctx->g, ctx->op64, ctx->fixmask, ctx->E64, ctx->meandiag, a,
+                        ctx->stream) != hipSuccess ||
+            (energy && launch_energy_check(ctx->g.ndof, ctx->u, r[o], ctx->b64, ctx->pcg1_st + o,
+                                           ctx->ecrit, ctx->partials,
+                                           ctx->stream) != hipSuccess)) {
+            hipStreamEndCapture(ctx->stream, &graph);
+            ctx->err = "PCG graph capture failed";
+            return TOHIP_ERR_HIP;
+        }
+    }
+    CK(hipStreamEndCapture(ctx->stream, &graph));
+    CK(hipGraphInstantiate(exec, graph, nullptr, nullptr, 0));
+    CK(hipGraphDestroy(graph));
+    return 0;
+}
+
+// Device-resident Jacobi PCG on K(E) x = b, one launch an iteration.  x is the
+// initial guess when !initially_zero.  Returns 0, TOHIP_NOT_CONVERGED or
+// TOHIP_BREAKDOWN.  Under EnergyCriteria (ctx->conv_kind) the residual test is
+// off and the energy test with tolerance `etol` stops the iteration; it is
+// evaluated on the starting iterate too, as IterativeSolvers evaluates its
+// stopping test before every iteration; a NaN or negative energy returns
+// TOHIP_ERR_DOMAIN.
 int solve_fp64(tohip_ctx* ctx, double abstol, double reltol, int64_t maxiter, bool zero,
                int64_t* iters, double* resid, double etol) {
     const int64_t n = ctx->g.ndof;
     const bool energy = ctx->conv_kind == TOHIP_CONV_ENERGY;
-    PcgScalars hs{};
+    if (energy && !(etol > 0)) {
+        ctx->err = "EnergyCriteria needs a positive tolerance";
+        return TOHIP_ERR_ARG;
+    }
+    const int nb = pcg1_blocks(ctx->g);
+    if (!ctx->r64b)
+        if (int rc = dalloc(ctx, &ctx->r64b, n)) return rc;
+    for (double*& p : ctx->pcg1_part)
+        if (!p)
+            if (int rc = dalloc(ctx, &p, (size_t)kPcg1Vals * nb)) return rc;
+    if (!ctx->pcg1_st)
+        if (int rc = dalloc(ctx, &ctx->pcg1_st, 2)) return rc;
+    if (!ctx->h_pcg1)
+        CK(hipHostMalloc((void**)&ctx->h_pcg1, sizeof(Pcg1State), hipHostMallocDefault));
+    Pcg1State hs{};
+    hs.rho_prev = 1.0;  // IterativeSolvers starts from rho_prev = 1 (multiplies p = 0)
+    hs.tol = -1.0;
     hs.abstol = energy ? 0.0 : abstol;
     hs.reltol = energy ? 0.0 : reltol;
     hs.maxiter = maxiter;
-    *ctx->h_sc = hs;
-    CK(hipMemcpyAsync(ctx->sc64, ctx->h_sc, sizeof(PcgScalars), hipMemcpyHostToDevice,
+    *ctx->h_pcg1 = hs;
+    CK(hipMemcpyAsync(ctx->pcg1_st, ctx->h_pcg1, sizeof(Pcg1State), hipMemcpyHostToDevice,
                       ctx->stream));
     if (energy) {
-        if (!(etol > 0)) {
-            ctx->err = "EnergyCriteria needs a positive tolerance";
-            return TOHIP_ERR_ARG;
-        }
         ctx->h_ecrit->tol = etol;
         ctx->h_ecrit->converged = 0;
         ctx->h_ecrit->err = 0;
+        ctx->h_ecrit->last = -1;
         CK(hipMemcpyAsync(ctx->ecrit, ctx->h_ecrit, sizeof(EnergyCrit), hipMemcpyHostToDevice,
                           ctx->stream));
     }
-    if (zero) {
+    if (zero)
         CK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
-        CK(launch_pcg_start<double>(n, ctx->b64, nullptr, ctx->r64, ctx->dinv64, ctx->p64[0],
-                                    ctx->sc64, ctx->partB, 0, ctx->stream));
-    } else {
+    else
         CK(launch_matvec<double>(ctx->g, ctx->op64, ctx->u, ctx->fixmask, ctx->E64, ctx->t64,
                                  ctx->meandiag, ctx->stream));
-        CK(launch_pcg_start<double>(n, ctx->b64, ctx->t64, ctx->r64, ctx->dinv64, ctx->p64[0],
-                                    ctx->sc64, ctx->partB, 0, ctx->stream));
+    CK(launch_pcg1_start(n, ctx->b64, zero ? nullptr : ctx->t64, ctx->dinv64, ctx->r64,
+                         ctx->p64[0], ctx->pcg1_part[0], nb, ctx->stream));
+    if (energy)
+        CK(launch_energy_check(n, ctx->u, ctx->r64, ctx->b64, ctx->pcg1_st, ctx->ecrit,
+                               ctx->partials, ctx->stream));
+    hipGraphExec_t& lg = energy ? ctx->g64e : ctx->g64;
+    hipGraphExec_t& sg = energy ? ctx->g64es : ctx->g64s;
+    if (int rc = capture_pcg1_graph(ctx, &lg, kPcg1GraphLong, energy)) return rc;
+    if (int rc = capture_pcg1_graph(ctx, &sg, kPcg1GraphShort, energy)) return rc;
+    if (ctx->time_graphs) CK(hipEventRecord(ctx->graph_ev[0], ctx->stream));
+    CK(pcg1_replay(lg, sg, ctx->pcg1_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
+                   &ctx->graph_launches));
+    if (ctx->time_graphs) {
+        CK(hipEventRecord(ctx->graph_ev[1], ctx->stream));
+        CK(hipEventSynchronize(ctx->graph_ev[1]));
+        float ms = 0;
+        hipEventElapsedTime(&ms, ctx->graph_ev[0], ctx->graph_ev[1]);
+        ctx->graph_ms += ms;
     }
     if (energy) {
-        CK(launch_energy_check(n, ctx->u, ctx->r64, ctx->b64, ctx->sc64, ctx->ecrit,
-                               ctx->partials, ctx->stream));
-        if (int rc = run_pcg_graphs<double>(ctx, &ctx->g64e, &ctx->g64es, ctx->op64, ctx->u,
-                                            ctx->r64, ctx->dinv64, ctx->p64, ctx->q64, ctx->E64,
-                                            ctx->sc64, ctx->ecrit))
-            return rc;
         CK(hipMemcpyAsync(ctx->h_ecrit, ctx->ecrit, sizeof(EnergyCrit), hipMemcpyDeviceToHost,
                           ctx->stream));
         CK(hipStreamSynchronize(ctx->stream));
-    } else if (int rc = run_pcg_graphs<double>(ctx, &ctx->g64, &ctx->g64s, ctx->op64, ctx->u,
-                                               ctx->r64, ctx->dinv64, ctx->p64, ctx->q64,
-                                               ctx->E64, ctx->sc64)) {
-        return rc;
     }
-    const PcgScalars& h = *ctx->h_sc;
+    const Pcg1State& h = *ctx->h_pcg1;
     if (iters) *iters = h.iter;
     if (resid) *resid = std::sqrt(h.rr);
     if (h.err) return pcg_breakdown(ctx, h.err);
@@ -1203,8 +1245,10 @@ void free_ctx(tohip_ctx* ctx) {
                     (void*)ctx->csr_diag, (void*)ctx->csr_dinv, (void*)ctx->csr_ke,
                     (void*)ctx->csr_md, (void*)ctx->mma_L, (void*)ctx->mma_U,
                     (void*)ctx->mma_x1, (void*)ctx->mma_x2, (void*)ctx->mma_st,
-                    (void*)ctx->mg_M, (void*)ctx->r32b, (void*)ctx->mg_wd})
+                    (void*)ctx->mg_M, (void*)ctx->r32b, (void*)ctx->mg_wd, (void*)ctx->r64b,
+                    (void*)ctx->pcg1_part[0], (void*)ctx->pcg1_part[1], (void*)ctx->pcg1_st})
         if (b) hipFree(b);
+    if (ctx->h_pcg1) hipHostFree(ctx->h_pcg1);
     if (ctx->h_mma) hipHostFree(ctx->h_mma);
     if (ctx->ecrit) hipFree(ctx->ecrit);
     if (ctx->h_ecrit) hipHostFree(ctx->h_ecrit);

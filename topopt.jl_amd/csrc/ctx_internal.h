@@ -5,7 +5,7 @@
 #include <string>
 #include <vector>
 
-#include "tohip_internal.h"
+#include "k_pcg1.h"
 
 struct tohip_nn;
 
@@ -73,6 +73,10 @@ struct tohip_ctx {
     tohip::PcgScalars* h_sc = nullptr;
     double* h_scal = nullptr;
     tohip::OcState* h_oc = nullptr;
+    // one-launch FP64 PCG (k_pcg1.h), on first use: the second residual, the two
+    // sets of partial sums and states (q's second buffer is t64), their host mirror
+    double *r64b = nullptr, *pcg1_part[2] = {nullptr, nullptr};
+    tohip::Pcg1State *pcg1_st = nullptr, *h_pcg1 = nullptr;
     // captured PCG iteration graphs
     hipGraphExec_t g64 = nullptr, g32 = nullptr, g64s = nullptr, g32s = nullptr;
     bool have_u = false;

@@ -6,7 +6,6 @@
 // src/Functions/temperature.jl).
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <limits>
 #include <string>
@@ -43,9 +42,6 @@ struct tohip_heat {
 
 namespace {
 
-// Iterations (launches) of the two captured graphs; even, so that a graph
-// starts and ends on the first set of vectors.
-constexpr int kHeatGraphIters = 64, kHeatGraphShort = 8;
 thread_local std::string g_heat_error;
 
 #define HCK(call)                                                  \
@@ -182,39 +178,11 @@ int solve(tohip_heat* ctx, bool zero, double abstol, double reltol, int64_t maxi
                                ctx->t, 0, ctx->stream));
     HCK(launch_pcg1_start(n, ctx->b, zero ? nullptr : ctx->t, ctx->dinv, ctx->r[0], ctx->p[0],
                           ctx->part[0], heat_pcg_blocks(ctx->g), ctx->stream));
-    if (int rc = capture(ctx, &ctx->graph, kHeatGraphIters)) return rc;
-    if (int rc = capture(ctx, &ctx->graph_short, kHeatGraphShort)) return rc;
-    // long graphs while the residual's history predicts many iterations to go,
-    // several per host check far from the end
-    double prev_res = -1.0;
-    long long prev_it = -1;
-    bool brief = false;
-    int launches = 1;
-    for (;;) {
-        for (int l = 0; l < launches; ++l)
-            HCK(hipGraphLaunch(brief ? ctx->graph_short : ctx->graph, ctx->stream));
-        HCK(hipMemcpyAsync(ctx->h_st, ctx->st, sizeof(Pcg1State), hipMemcpyDeviceToHost,
-                           ctx->stream));
-        HCK(hipStreamSynchronize(ctx->stream));
-        const Pcg1State& h = *ctx->h_st;
-        if (h.done) break;
-        const double res = std::sqrt(h.rr);
-        brief = false;
-        launches = 1;
-        if (prev_res > 0 && res > 0 && h.tol > 0 && h.iter > prev_it) {
-            const double rate = std::log(res / prev_res) / double(h.iter - prev_it);
-            if (rate < 0) {
-                const double togo = std::log(h.tol / res) / rate;
-                brief = togo < 0.75 * kHeatGraphIters;
-                if (brief)
-                    launches = std::max(1, (int)(togo / kHeatGraphShort));
-                else
-                    launches = std::max(1, std::min(4, (int)(togo / (1.5 * kHeatGraphIters))));
-            }
-        }
-        prev_res = res;
-        prev_it = h.iter;
-    }
+    if (int rc = capture(ctx, &ctx->graph, kPcg1GraphLong)) return rc;
+    if (int rc = capture(ctx, &ctx->graph_short, kPcg1GraphShort)) return rc;
+    int64_t syncs = 0, graphs = 0;
+    HCK(pcg1_replay(ctx->graph, ctx->graph_short, ctx->st, ctx->h_st, ctx->stream, &syncs,
+                    &graphs));
     const Pcg1State& h = *ctx->h_st;
     if (iters) *iters = h.iter;
     if (resid) *resid = std::sqrt(h.rr);

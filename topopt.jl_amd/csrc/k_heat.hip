@@ -37,24 +37,15 @@ __device__ __forceinline__ int heat_corner(int ox, int oy, int oz) {
 //
 // One launch is a whole PCG iteration.  Bound by latency on small grids, by the
 // cache traffic of its 4 vectors in (1.3 x (zc + 2) / zc with the halo) and 4
-// out on larger ones.  MI355X, one iteration: 128x96x80 26 us (direction, a
+// out on larger ones.  MI355X, one iteration: 128x96x80 23.8 us (direction, a
 // 27-point gather of K p and update in three launches: 85 us; the 57 MB it must
-// move take 12 us at the copy rate), 80x60 6.0 us (14 us).
+// move take 12 us at the copy rate), 80x60 5.7 us (14 us).
 constexpr int kHC = 16, kHO = kHC - 1, kHS = kHC + 1;
 
-__device__ __forceinline__ double heat_row_shr1(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x111, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x111, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Columns of 15 x 15 nodes and chunks of zc planes, about 768 workgroups (the
-// PCG kernel's 139 VGPRs let three run per CU) when the grid has them; at most
-// kMaxPartials launch and stride over the rest.  Fewer planes a chunk fill the
-// chip better but re-stage more (zc + 2 planes each): at 128x96x80, with 504 /
-// 693 / 756 / 882 / 1008 workgroups, a PCG iteration took 25.2 / 28.2 / 25.9 /
-// 33.5 / 33.6 us.
+// Columns of 15 x 15 nodes and chunks of zc planes, about 768 workgroups when the
+// grid has them; beyond kMaxPartials they stride over the rest.  Fewer planes a
+// chunk fill the chip better but re-stage more (zc + 2 planes each): a PCG
+// iteration at 128x96x80 takes 23.8 us with 756 workgroups, 26.0 with 1008.
 struct HeatShape {
     int ncx, ncy, zc, nch, nwork;
 };
@@ -72,16 +63,16 @@ static HeatShape heat_shape(const HeatGrid& g) {
 static int heat_op_blocks(const HeatShape& s) { return std::min(s.nwork, kMaxPartials); }
 int heat_pcg_blocks(const HeatGrid& g) { return heat_op_blocks(heat_shape(g)); }
 
-// A staged node: in the mesh or not, its operands.
+// A staged node's operands.
 struct HeatNode {
     double v, r, q, d;  // MODE 1: v = p; otherwise v = x
     uint8_t m;
-    bool in;
 };
 
 // MODE 0: y = K x (prescribed nodes masked, their rows md x); MODE 1: one
 // PCG iteration (k_pcg1.h); MODE 2: y = K_full x (no masking).
-template <int DIM, int MODE, typename Off>
+// LOOP: more work than workgroups.
+template <int DIM, int MODE, typename Off, bool LOOP>
 __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, HeatShape sh,
                                                       const double* __restrict__ xin,
                                                       const uint8_t* __restrict__ fixmask,
@@ -109,11 +100,10 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
     };
     bool ina = false, inb = false, ine = false;
     int64_t nbase = 0, ebase = 0;
-    auto load = [&](Off o, bool in, int k) {
+    auto load = [&](Off o, int k) {
         const int nk = DIM == 3 ? min(max(k, 0), g.NZ - 1) : 0;
         const int64_t base = nbase + (int64_t)nk * g.NX * g.NY;
         HeatNode h;
-        h.in = in && (DIM == 2 || k == nk);
         h.m = MODE == 2 ? 0 : at64(fixmask, base, o / 8);
         if (MODE == 1) {
             h.v = at64(a.p, base, o);
@@ -125,11 +115,10 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
         }
         return h;
     };
-    auto load_E = [&](int k) {  // the cell of this thread in layer k (0 outside the mesh)
-        const bool in = ine && (DIM == 2 || (k >= 0 && k < g.nz));
-        const int64_t base = ebase + (int64_t)(DIM == 3 ? min(max(k, 0), g.nz - 1) : 0) * g.nx * g.ny;
-        const double e = at64(E, base, oe);
-        return in ? e : 0.0;
+    auto load_E = [&](int k) {  // the cell of this thread in layer k
+        const int ck = DIM == 3 ? min(max(k, 0), g.nz - 1) : 0;
+        const int64_t base = ebase + (int64_t)ck * g.nx * g.ny;
+        return at64(E, base, oe);
     };
     double sum[kPcg1Vals] = {0, 0, 0, 0, 0, 0, 0, 0};
     int buf = 0;
@@ -159,8 +148,8 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
         }
         auto plane = [&](int k) { return nbase + (int64_t)(DIM == 3 ? k : 0) * g.NX * g.NY; };
         const int sb = DIM == 3 ? kb - 1 : 0, se = DIM == 3 ? ke : 0;  // staged planes
-        HeatNode na = load(oa, ina, sb), nb{};
-        if (two) nb = load(ob, inb, sb);
+        HeatNode na = load(oa, sb), nb{};
+        if (two) nb = load(ob, sb);
         double xa = 0.0;
         if (MODE == 1 && mine && sb >= kb) xa = at64(a.x, plane(sb), oa);
         double en = DIM == 3 ? 0.0 : load_E(0);
@@ -197,37 +186,42 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
                     }
                 }
             }
-            continue;
+            if (LOOP) continue;
+            break;
         }
         double fp[4] = {0, 0, 0, 0}, up[4] = {0, 0, 0, 0};
         double po = 0.0, ro = 0.0, dd = 0.0;  // own node of the plane below
         uint8_t mo = 0;
         for (int k = sb; k <= se; ++k) {
             // direction (or input) of this plane, then the next plane's loads
-            auto value = [&](HeatNode& h) {
+            // (what lies outside the mesh is put to 0 here, not where it is
+            // loaded: a select there would wait for the whole prefetch)
+            const bool kin = DIM == 2 || (k >= 0 && k < g.NZ);
+            auto value = [&](HeatNode& h, bool in) {
                 if (MODE == 1) {
                     // explicit FMAs: a halo copy and its owner get the same bits
                     h.r = fma(-plan.alpha, pend ? h.q : 0.0, h.r);
                     h.v = fma(plan.beta, h.v, h.d * h.r);
                 }
-                return (h.in && !h.m) ? h.v : 0.0;
+                return (in && kin && !h.m) ? h.v : 0.0;
             };
             const double pold = na.v;
-            const double va = value(na);
+            const double va = value(na, ina);
             pl[buf][ci + kHS * cj] = va;
-            if (two) pl[buf][li2 + kHS * lj2] = value(nb);
+            if (two) pl[buf][li2 + kHS * lj2] = value(nb, inb);
             if (MODE == 1 && mine && k >= kb && k < ke) {
                 const int64_t n = plane(k);
                 if (pend) at64(a.x, n, oa) = xa + plan.alpha * pold;
                 at64(a.rn, n, oa) = na.r;
                 at64(a.pn, n, oa) = na.v;
             }
-            const double ec = en;
+            const double ec = ine && (DIM == 2 || (k >= 1 && k <= g.nz)) ? en : 0.0;
             const HeatNode cur = na;
             if (k < se) {
-                na = load(oa, ina, k + 1);
-                if (two) nb = load(ob, inb, k + 1);
-                if (MODE == 1 && mine && k + 1 >= kb && k + 1 < ke) xa = at64(a.x, plane(k + 1), oa);
+                na = load(oa, k + 1);
+                if (two) nb = load(ob, k + 1);
+                if (MODE == 1 && mine && k + 1 >= kb && k + 1 < ke)
+                    xa = at64(a.x, plane(k + 1), oa);
                 en = load_E(k);
             }
             __syncthreads();
@@ -250,8 +244,8 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
                     }
                 }
                 hadamard_inv<double, 2>(lo);
-                const double y0 = heat_row_shr1(lo[1]) + lo[0];
-                exch[tid] = heat_row_shr1(lo[3]) + lo[2];
+                const double y0 = row_shr1(lo[1]) + lo[0];
+                exch[tid] = row_shr1(lo[3]) + lo[2];
                 __syncthreads();
                 const int ko = DIM == 3 ? k - 1 : 0;
                 if (mine && ko >= kb && ko < ke) {
@@ -281,6 +275,7 @@ __global__ __launch_bounds__(kThreads) void k_heat_op(HeatGrid g, HeatModes B, H
             dd = cur.d;
             mo = cur.m;
         }
+        if (!LOOP) break;
     }
     if (MODE == 1) {
         pcg1_store_sums(sum, red, a.partn);
@@ -301,11 +296,15 @@ static hipError_t launch_heat_op(const HeatGrid& g, const HeatModes& B, const do
                                  double* y, const Pcg1Args& a, hipStream_t s) {
     const HeatShape sh = heat_shape(g);
     const dim3 grid(heat_op_blocks(sh)), block(kThreads);
-    if ((int64_t)g.NX * kHS * 8 < ((int64_t)1 << 32))
-        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint32_t>), grid, block, 0, s, g, B, sh, x,
+    const bool loop = sh.nwork > kMaxPartials;
+    if ((int64_t)g.NX * kHS * 8 >= ((int64_t)1 << 32))
+        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint64_t, true>), grid, block, 0, s, g, B, sh, x,
+                           fixmask, E, meandiag, y, a);
+    else if (loop)
+        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint32_t, true>), grid, block, 0, s, g, B, sh, x,
                            fixmask, E, meandiag, y, a);
     else
-        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint64_t>), grid, block, 0, s, g, B, sh, x,
+        hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint32_t, false>), grid, block, 0, s, g, B, sh, x,
                            fixmask, E, meandiag, y, a);
     return hipGetLastError();
 }

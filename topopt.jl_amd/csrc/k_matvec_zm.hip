@@ -39,17 +39,6 @@ constexpr int kZS = kZC + 1;             // staged nodes per row (17)
 constexpr int kZSP = kZS * kZS;          // staged nodes per plane (289)
 constexpr int kZL = (kZSP + kZT - 1) / kZT;  // staged nodes per thread (2)
 
-// v of lane l - 1 within each 16-lane row (0 in the row's first lane).
-__device__ __forceinline__ float row_shr1(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xf, 0xf, true));
-}
-__device__ __forceinline__ double row_shr1(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x111, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x111, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 }  // namespace
 
 // Chunking: columns of 15 x 15 nodes, node planes split so the launch has

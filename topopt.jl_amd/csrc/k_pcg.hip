@@ -214,15 +214,19 @@ hipError_t launch_pcg1_start(int64_t n, const double* b, const double* Ax, const
 // current x and recursive residual r: x'Ax = f.x - x.r; converged when
 // |x'Ax - energy| / x'Ax <= tol and |x.r| / x'Ax <= tol; energy := x'Ax.
 // Its stopping test is `iteration >= maxiter || converged`, so the criterion
-// is not evaluated once maxiter iterations are done.
+// is not evaluated once maxiter iterations are done.  It runs after every
+// launch of the one-launch iteration, on the x and r that launch left; a launch
+// that applied no update (the first, or one after kPcg1Exact) leaves the
+// iterate that was tested before, which `last` tells.
 __global__ __launch_bounds__(kThreads) void k_ecrit_partials(int64_t n,
                                                              const double* __restrict__ x,
                                                              const double* __restrict__ r,
                                                              const double* __restrict__ f,
-                                                             const PcgScalars* sc,
+                                                             const Pcg1State* sc,
+                                                             const EnergyCrit* ec,
                                                              double* __restrict__ partials) {
     __shared__ double red[kWaves];
-    if (sc->done || sc->iter >= sc->maxiter) return;
+    if (sc->done || sc->iter >= sc->maxiter || sc->iter == ec->last) return;
     double xr = 0.0, fx = 0.0;
     for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * kThreads) {
@@ -240,14 +244,15 @@ __global__ __launch_bounds__(kThreads) void k_ecrit_partials(int64_t n,
 
 __global__ __launch_bounds__(kThreads) void k_ecrit_decide(int nb,
                                                            const double* __restrict__ partials,
-                                                           PcgScalars* sc, EnergyCrit* ec) {
+                                                           Pcg1State* sc, EnergyCrit* ec) {
     __shared__ double red[kWaves];
-    if (sc->done || sc->iter >= sc->maxiter) return;
+    if (sc->done || sc->iter >= sc->maxiter || sc->iter == ec->last) return;
     const double xtr = reduce_partials(partials, nb, 2, 0, red);
     const double fx = reduce_partials(partials, nb, 2, 1, red);
     if (threadIdx.x != 0) return;
     const double xAx = fx - xtr;
     const double change = xAx - ec->energy;
+    ec->last = sc->iter;
     ec->xtr = xtr;
     ec->xAx = xAx;
     if (isnan(change) || isnan(xAx)) {
@@ -270,9 +275,9 @@ __global__ __launch_bounds__(kThreads) void k_ecrit_decide(int nb,
 }
 
 hipError_t launch_energy_check(int64_t n, const double* x, const double* r, const double* f,
-                               PcgScalars* sc, EnergyCrit* ec, double* partials, hipStream_t s) {
+                               Pcg1State* sc, EnergyCrit* ec, double* partials, hipStream_t s) {
     hipLaunchKernelGGL(k_ecrit_partials, dim3(kVecBlocks), dim3(kThreads), 0, s, n, x, r, f, sc,
-                       partials);
+                       ec, partials);
     hipLaunchKernelGGL(k_ecrit_decide, dim3(1), dim3(kThreads), 0, s, kVecBlocks, partials, sc,
                        ec);
     return hipGetLastError();

@@ -21,6 +21,8 @@
 // their halos), so launches alternate and a graph holds an even number.  x is
 // read and written by the owner of a node only.
 #pragma once
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "k_common.h"
@@ -83,12 +85,16 @@ __device__ __forceinline__ Pcg1Plan pcg1_plan(const Pcg1State& s, const double (
         o.rr0 = rr;
     }
     o.rr = rr;
+    // ||r|| <= tol; the root is taken only where the squares are near each other
+    // (or tiny), for it is a good part of a small launch's serial chain
+    const double t2 = o.tol * o.tol;
+    const bool met = rr <= 2.0 * t2 || t2 < 1e-280 ? sqrt(rr) <= o.tol : false;
     int err = 0;
     if (!(isfinite(rr) && isfinite(rz)))
         err = kPcgErrNonFinite;
-    else if (!(rz > 0.0) && rr > 0.0 && !(sqrt(rr) <= o.tol))
+    else if (!(rz > 0.0) && rr > 0.0 && !met)
         err = kPcgErrPrecond;
-    if (err != 0 || sqrt(rr) <= o.tol || o.iter >= s.maxiter) {
+    if (err != 0 || met || o.iter >= s.maxiter) {
         o.done = 1;
         o.err = err;
         return {alpha, 0.0, kPcg1Stop};
@@ -131,14 +137,15 @@ __device__ __forceinline__ void block_sum8(double (&v)[kPcg1Vals], double (*red)
 }
 
 // The workgroup's row of partial sums.
+template <int NT = kThreads>
 __device__ __forceinline__ void pcg1_store_sums(double (&sum)[kPcg1Vals],
                                                 double (*red)[kPcg1Vals],
                                                 double* __restrict__ part) {
-    block_sum8<kThreads>(sum, red);
+    block_sum8<NT>(sum, red);
     if (threadIdx.x < kPcg1Vals) {
         double t = 0.0;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) t += red[w][threadIdx.x];
+        for (int w = 0; w < NT / 64; ++w) t += red[w][threadIdx.x];
         part[(size_t)blockIdx.x * kPcg1Vals + threadIdx.x] = t;
     }
 }
@@ -176,5 +183,58 @@ struct Pcg1Args {
 // r = b - Ax (Ax may be null: x = 0), p = 0, nb rows of (r.z, r.r) into part.
 hipError_t launch_pcg1_start(int64_t n, const double* b, const double* Ax, const double* dinv,
                              double* r, double* p, double* part, int nb, hipStream_t s);
+
+// EnergyCriteria check on the current iterate (x, r = f - Ax): partial sums
+// of x.r and f.x over kVecBlocks blocks into `partials`, then one block sets
+// ec and, when converged or on a domain error, sc->done (before the next
+// launch applies the pending update).  No-op once done.
+hipError_t launch_energy_check(int64_t n, const double* x, const double* r, const double* f,
+                               Pcg1State* sc, EnergyCrit* ec, double* partials, hipStream_t s);
+
+// One iteration on the elasticity operator (k_pcg1.hip); a.nb = pcg1_blocks(g).
+int pcg1_blocks(const Grid& g);
+hipError_t launch_pcg1(const Grid& g, const ElemOp<double>& op, const uint8_t* fixmask,
+                       const double* E, double meandiag, const Pcg1Args& a, hipStream_t s);
+
+// Iterations (launches) of the long and the short captured graph; even, so that
+// a graph starts and ends on the first set of vectors.
+constexpr int kPcg1GraphLong = 64, kPcg1GraphShort = 8;
+
+// Replays the graphs until the device has set `done`; st[0] ends up in *h.  Long
+// graphs while the residual's history predicts many iterations to go, several
+// per host check far from the end; then short ones, which leave fewer launches
+// that find nothing to do.
+inline hipError_t pcg1_replay(hipGraphExec_t lg, hipGraphExec_t sg, const Pcg1State* st,
+                              Pcg1State* h, hipStream_t s, int64_t* syncs, int64_t* graphs) {
+    double prev_res = -1.0;
+    long long prev_it = -1;
+    bool brief = false;
+    int launches = 1;
+    for (;;) {
+        hipError_t e;
+        for (int l = 0; l < launches; ++l)
+            if ((e = hipGraphLaunch(brief ? sg : lg, s)) != hipSuccess) return e;
+        if ((e = hipMemcpyAsync(h, st, sizeof(Pcg1State), hipMemcpyDeviceToHost, s)) != hipSuccess)
+            return e;
+        if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+        *syncs += 1;
+        *graphs += launches;
+        if (h->done) return hipSuccess;
+        const double res = std::sqrt(h->rr);
+        brief = false;
+        launches = 1;
+        if (prev_res > 0 && res > 0 && h->tol > 0 && h->iter > prev_it) {
+            const double rate = std::log(res / prev_res) / double(h->iter - prev_it);
+            if (rate < 0) {
+                const double togo = std::min(std::log(h->tol / res) / rate, 1e6);
+                brief = togo < 0.75 * kPcg1GraphLong;
+                launches = brief ? std::max(1, (int)(togo / kPcg1GraphShort))
+                                 : std::max(1, std::min(4, (int)(togo / (1.5 * kPcg1GraphLong))));
+            }
+        }
+        prev_res = res;
+        prev_it = h->iter;
+    }
+}
 
 }  // namespace tohip

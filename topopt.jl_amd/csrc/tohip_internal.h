@@ -90,7 +90,7 @@ struct EnergyCrit {
     double xtr, xAx;
     int converged;
     int err;  // 1: NaN in the energy or its change, 2: negative x'Ax
-    int pad[2];
+    long long last;  // iteration of the last check of this solve (-1: none yet)
 };
 
 constexpr int kMaxPartials = 4096;  // per-block partial slots of one kernel
@@ -255,12 +255,6 @@ hipError_t launch_csr_pcg_iter(int64_t n, const int64_t* rowptr, const int* cols
                                const double* vals, double* x, double* r, const double* dinv,
                                double* p0, double* p1, double* q, PcgScalars* sc, double* partA,
                                double* partB, hipStream_t s);
-
-// EnergyCriteria check on the current iterate (x, r = f - Ax): partial sums
-// of x.r and f.x over kVecBlocks blocks into `partials`, then one block sets
-// ec and, when converged or on a domain error, sc->done.  No-op once done.
-hipError_t launch_energy_check(int64_t n, const double* x, const double* r, const double* f,
-                               PcgScalars* sc, EnergyCrit* ec, double* partials, hipStream_t s);
 
 // Sum-reductions finished by a one-block kernel: out[v] = sum_b part[b*nv+v].
 hipError_t launch_reduce(const double* partials, int nb, int nv, double* out, hipStream_t s);
