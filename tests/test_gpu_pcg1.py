@@ -82,3 +82,37 @@ def test_elastic_tiles(T, O, gpu, case):
         if n < it:
             s(maxiter=n)
             assert s.last_iters == n and not s.converged
+
+
+# rows of one to 27 neighbours; node counts at the remainders of 32 (64 in 2D) a workgroup
+CSR = [(1, 2), (7, 8), (15, 2), (30, 32), (1, 2, 2), (3, 2, 2), (7, 4, 4), (9, 6, 8), (20, 10, 12)]
+
+
+@pytest.mark.parametrize("nels", CSR)
+@pytest.mark.parametrize("jacobi", [False, True])
+def test_assembled_product_and_solve(T, O, gpu, nels, jacobi):
+    from topopt_jl_amd._lib import dptr
+    prob = T.PointLoadCantilever(nels)
+    s = T.FEASolver(T.HIPCGAssemblySolver, prob, xmin=1e-3, penalty=T.PowerPenaltyFun(3.0),
+                    cg_max_iter=20000, preconditioner="jacobi" if jacobi else None)
+    orc = O.Oracle(O.Cantilever(tuple(nels)), xmin=1e-3, p=3.0)
+    g = np.random.default_rng(prob.ncells)
+    x = g.uniform(0.5, 1.0, prob.ncells)
+    s.vars = x
+    orc.set_vars(x)
+    Ke, _ = orc.assembled()
+    v = g.standard_normal(prob.ndofs)
+    s.set_densities(x)
+    y = np.empty_like(v)
+    assert s.lib.tohip_csr_matvec(s.ctx.ptr, dptr(v), dptr(y)) == 0
+    free = ~prob.fixed.astype(bool)
+    assert relerr(y[free], (Ke @ v)[free]) < 1e-14  # sums of at most 81 terms
+    s(abstol=0.0, reltol=1e-11)
+    assert s.converged
+    b = np.where(free, prob.f, 0.0)
+    assert np.linalg.norm(b - Ke @ s.u) <= 1e-9 * np.linalg.norm(b)
+    it = s.last_iters
+    for n in (0, 1, 2):
+        if n < it:
+            s(abstol=0.0, reltol=1e-11, maxiter=n)
+            assert s.last_iters == n and not s.converged

@@ -1238,7 +1238,7 @@ void free_ctx(tohip_ctx* ctx) {
     if (ctx->mg_stream) hipStreamSynchronize(ctx->mg_stream);  // a rebuild may be in flight
     for (void* b : bufs)
         if (b) hipFree(b);
-    for (hipGraphExec_t ge : {ctx->g32mg, ctx->g32mgs, ctx->g64e, ctx->g64es, ctx->gcsr,
+    for (hipGraphExec_t ge : {ctx->g32mg, ctx->g32mgs, ctx->g64e, ctx->g64es, ctx->gcsr, ctx->gcsrs,
                               ctx->g64mg, ctx->g64mgs})
         if (ge) hipGraphExecDestroy(ge);
     for (void* b : {(void*)ctx->csr_rowptr, (void*)ctx->csr_cols, (void*)ctx->csr_vals,
@@ -1246,7 +1246,8 @@ void free_ctx(tohip_ctx* ctx) {
                     (void*)ctx->csr_md, (void*)ctx->mma_L, (void*)ctx->mma_U,
                     (void*)ctx->mma_x1, (void*)ctx->mma_x2, (void*)ctx->mma_st,
                     (void*)ctx->mg_M, (void*)ctx->r32b, (void*)ctx->mg_wd, (void*)ctx->r64b,
-                    (void*)ctx->pcg1_part[0], (void*)ctx->pcg1_part[1], (void*)ctx->pcg1_st})
+                    (void*)ctx->pcg1_part[0], (void*)ctx->pcg1_part[1], (void*)ctx->pcg1_st,
+                    (void*)ctx->csr_part, (void*)ctx->csr_st})
         if (b) hipFree(b);
     if (ctx->h_pcg1) hipHostFree(ctx->h_pcg1);
     if (ctx->h_mma) hipHostFree(ctx->h_mma);
@@ -1412,8 +1413,6 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
 }
 
 // ---- assembled K in CSR (CGAssemblySolver comparator) ----
-constexpr int kCsrGraphIters = 32;
-
 // Pattern (host row pointers, device columns) on first use, then the values
 // of K(current densities) with apply!'s boundary rule and the preconditioner
 // diagonal (jacobi: 1 / diag, else identity).
@@ -1467,10 +1466,9 @@ int capture_csr_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters) {
     hipGraph_t graph;
     CK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     for (int it = 0; it < iters; ++it) {
-        hipError_t e = launch_csr_pcg_iter(ctx->g.ndof, ctx->csr_rowptr, ctx->csr_cols,
-                                           ctx->csr_vals, ctx->u, ctx->r64, ctx->csr_dinv,
-                                           ctx->p64[0], ctx->p64[1], ctx->q64, ctx->sc64,
-                                           ctx->partA, ctx->partB, ctx->stream);
+        hipError_t e = launch_csr_pcg1(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->u, ctx->r64,
+                                       ctx->p64[0], ctx->q64, ctx->csr_dinv, ctx->csr_st + (it & 1),
+                                       ctx->csr_st + ((it & 1) ^ 1), ctx->csr_part, ctx->stream);
         if (e != hipSuccess) {
             hipStreamEndCapture(ctx->stream, &graph);
             ctx->err = "CSR PCG graph capture failed";
@@ -1740,8 +1738,7 @@ int tohip_csr_matvec(tohip_ctx* ctx, const double* x, double* y) {
     if (!ctx || !x || !y) return TOHIP_ERR_ARG;
     if (int rc = csr_assemble(ctx, ctx->csr_safe > 0 ? 1 : 0, 1)) return rc;
     if (int rc = upload_dofs(ctx, x, ctx->r64)) return rc;
-    CK(launch_csr_spmv(ctx->g.ndof, ctx->csr_rowptr, ctx->csr_cols, ctx->csr_vals, ctx->r64,
-                       ctx->t64, ctx->stream));
+    CK(launch_csr_spmv(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->r64, ctx->t64, ctx->stream));
     return download_dofs(ctx, ctx->t64, y);
 }
 
@@ -1767,33 +1764,35 @@ int tohip_csr_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, d
                 fz[ctx->perm.empty() ? dim * node + d : ctx->perm[dim * node + d]] = 0.0;
     if (int rc = upload_dofs(ctx, fz.data(), ctx->b64)) return rc;
     if (int rc = csr_assemble(ctx, safe ? 1 : 0, jacobi ? 1 : 0)) return rc;
-    PcgScalars hs{};
+    const int nb = csr_pcg1_blocks(ctx->g);
+    if (!ctx->csr_part)
+        if (int rc = dalloc(ctx, &ctx->csr_part, (size_t)kPcg1Vals * nb)) return rc;
+    if (!ctx->csr_st)
+        if (int rc = dalloc(ctx, &ctx->csr_st, 2)) return rc;
+    if (!ctx->h_pcg1)
+        CK(hipHostMalloc((void**)&ctx->h_pcg1, sizeof(Pcg1State), hipHostMallocDefault));
+    Pcg1State hs{};
+    hs.rho_prev = 1.0;  // IterativeSolvers starts from rho_prev = 1 (multiplies p = 0)
+    hs.tol = -1.0;
     hs.abstol = abstol;
     hs.reltol = reltol;
     hs.maxiter = maxiter;
-    *ctx->h_sc = hs;
-    CK(hipMemcpyAsync(ctx->sc64, ctx->h_sc, sizeof(PcgScalars), hipMemcpyHostToDevice,
+    *ctx->h_pcg1 = hs;
+    CK(hipMemcpyAsync(ctx->csr_st, ctx->h_pcg1, sizeof(Pcg1State), hipMemcpyHostToDevice,
                       ctx->stream));
     if (initially_zero) {
         CK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
-        CK(launch_pcg_start<double>(n, ctx->b64, nullptr, ctx->r64, ctx->csr_dinv, ctx->p64[0],
-                                    ctx->sc64, ctx->partB, 0, ctx->stream));
     } else {
         if (int rc = upload_dofs(ctx, u, ctx->u)) return rc;
-        CK(launch_csr_spmv(n, ctx->csr_rowptr, ctx->csr_cols, ctx->csr_vals, ctx->u, ctx->t64,
-                           ctx->stream));
-        CK(launch_pcg_start<double>(n, ctx->b64, ctx->t64, ctx->r64, ctx->csr_dinv, ctx->p64[0],
-                                    ctx->sc64, ctx->partB, 0, ctx->stream));
+        CK(launch_csr_spmv(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->u, ctx->t64, ctx->stream));
     }
-    if (int rc = capture_csr_graph(ctx, &ctx->gcsr, kCsrGraphIters)) return rc;
-    for (;;) {
-        CK(hipGraphLaunch(ctx->gcsr, ctx->stream));
-        CK(hipMemcpyAsync(ctx->h_sc, ctx->sc64, sizeof(PcgScalars), hipMemcpyDeviceToHost,
-                          ctx->stream));
-        CK(hipStreamSynchronize(ctx->stream));
-        if (ctx->h_sc->done) break;
-    }
-    const PcgScalars& h = *ctx->h_sc;
+    CK(launch_pcg1_start(n, ctx->b64, initially_zero ? nullptr : ctx->t64, ctx->csr_dinv, ctx->r64,
+                         ctx->p64[0], ctx->csr_part, nb, ctx->stream));
+    if (int rc = capture_csr_graph(ctx, &ctx->gcsr, kPcg1GraphLong)) return rc;
+    if (int rc = capture_csr_graph(ctx, &ctx->gcsrs, kPcg1GraphShort)) return rc;
+    CK(pcg1_replay(ctx->gcsr, ctx->gcsrs, ctx->csr_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
+                   &ctx->graph_launches));
+    const Pcg1State& h = *ctx->h_pcg1;
     if (iters_out) *iters_out = h.iter;
     if (resid_out) *resid_out = std::sqrt(h.rr);
     ctx->have_u = true;
@@ -2544,8 +2543,8 @@ int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
             case TOHIP_K_VCYCLE:
                 return launch_vcycle(ctx, ctx->r32, nullptr, nullptr, nullptr);
             case TOHIP_K_CSR_SPMV:
-                return launch_csr_spmv(ctx->g.ndof, ctx->csr_rowptr, ctx->csr_cols,
-                                       ctx->csr_vals, ctx->r64, ctx->q64, s);
+                return launch_csr_spmv(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->r64,
+                                       ctx->q64, s);
             default:
                 return launch_oc(ctx->g.ncells, ctx->xd, ctx->dc, ctx->f_colsum, 0.3, 0.2, 1e-12,
                                  16, ctx->xnew, ctx->oc, ctx->partials, s);

@@ -104,7 +104,9 @@ struct tohip_ctx {
     // dense coarsest-level operator of the multigrid V-cycle (ndof^2 floats,
     // symmetric); null when the iteration kernel is used instead
     float* mg_M = nullptr;
-    hipGraphExec_t gcsr = nullptr;
+    hipGraphExec_t gcsr = nullptr, gcsrs = nullptr;
+    double* csr_part = nullptr;  // partial sums and states of its PCG (k_pcg1.h)
+    tohip::Pcg1State* csr_st = nullptr;
     int last_replacements = 0;
     size_t dev_bytes = 0;  // device memory held by this context
     // multigrid preconditioner (built on first use by a TOHIP_MIXED_MG solve)

@@ -12,12 +12,18 @@
 // (apply!).  Each (node, neighbour) pair is assembled by one thread as a
 // dim x dim block: no atomics, deterministic.
 //
-// SpMV: 16 lanes per row (a row has at most 81 entries), lane-strided over
-// the row's entries, a width-16 shuffle tree; HBM-bound on the 12 bytes per
-// stored entry (value + column).
-#include "k_common.h"
+#include <algorithm>
+
+#include "k_pcg1.h"
 
 namespace tohip {
+
+// The PCG operands of k_csr_spmv.
+struct CsrPcgArgs {
+    const double *r, *dinv;
+    const Pcg1State* st;
+    double* part;
+};
 
 // Valid neighbour offsets of node (i, j, k) in ascending node order; returns
 // the count and, when o >= 0, the slot of offset o in *slot (-1 if invalid).
@@ -198,87 +204,162 @@ __global__ void k_csr_dinv(int64_t ndof, const double* __restrict__ diag,
     }
 }
 
-// y = K x, 16 lanes per row.  PCG: x is p_k (chosen by the iteration counter),
-// per-block partials of p.q into part; a no-op once `done`.
-template <bool PCG>
-__global__ __launch_bounds__(kThreads) void k_csr_spmv(int64_t nrows,
-                                                       const int64_t* __restrict__ rowptr,
-                                                       const int* __restrict__ cols,
+// y = K x by nodes.  A group of 32 lanes (16 in 2D) takes four consecutive nodes:
+// lane o holds neighbour offset o of each, so it loads x at that neighbour once
+// for the node's D rows and its D x D block from them (D consecutive values a row,
+// the rows of a node contiguous: coalesced).  The neighbour and the slot of its
+// block follow from the grid, so the columns are not read: 8 bytes an entry
+// instead of 12.  The 4 D row sums of a group come out of one reduce-scatter
+// (lanes keep the half of the values that a lane bit selects) in place of a tree
+// a row.
+//
+// PCG: x = p, with the sums of the one-launch iteration (k_pcg1.h) at the rows a
+// lane owns; on a state without a pending update only (r.z, r.r).
+// Bound by the matrix, 1.9 KB a node in 3D: at 60x20x20 (52 MB, in the last-level
+// cache) an iteration with the vector kernel takes 19.8 us, against 32 for a
+// direction, a product of 16 lanes a row over values and columns, and an update.
+// Two nodes a group (5 waves per SIMD instead of 4): 21.1 us; row starts in closed
+// form instead of the row pointers: 20.3.
+constexpr int kCsrNodes = 4;  // nodes of one group
+template <int DIM>
+constexpr int csr_group = DIM == 3 ? 32 : 16;
+template <int DIM, bool PCG>
+__global__ __launch_bounds__(kThreads) void k_csr_spmv(Grid g, const int64_t* __restrict__ rowptr,
                                                        const double* __restrict__ vals,
-                                                       const double* x0, const double* x1,
-                                                       double* __restrict__ y, PcgScalars* sc,
-                                                       double* __restrict__ part) {
-    __shared__ double red[kWaves];
-    const double* x = x0;
+                                                       const double* __restrict__ x,
+                                                       double* __restrict__ y, CsrPcgArgs a) {
+    constexpr int G = csr_group<DIM>, NV = DIM == 3 ? 16 : 8, DV = NV / kCsrNodes;
+    __shared__ double red[kWaves][kPcg1Vals];
+    double sum[kPcg1Vals] = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int lane = threadIdx.x & (G - 1);
+    const int ox = lane % 3 - 1, oy = (lane / 3) % 3 - 1, oz = DIM == 3 ? lane / 9 - 1 : 0;
+    const bool used = lane < (DIM == 3 ? 27 : 9);
+    bool step = true;
     if (PCG) {
-        if (sc->done) return;
-        x = (sc->k_cur & 1) ? x1 : x0;
+        if (a.st->done) return;
+        step = a.st->pend != 0;
     }
-    const int lane = threadIdx.x & 15;
-    const int64_t groups = (int64_t)gridDim.x * (kThreads / 16);
-    double acc = 0.0;
-    for (int64_t row = blockIdx.x * (int64_t)(kThreads / 16) + (threadIdx.x >> 4); row < nrows;
-         row += groups) {
-        const int64_t b = rowptr[row], e = rowptr[row + 1];
-        double s = 0.0;
-        for (int64_t kk = b + lane; kk < e; kk += 16) s += vals[kk] * x[cols[kk]];
-        for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
-        if (lane == 0) {
-            y[row] = s;
-            if (PCG) acc += x[row] * s;
+    const int64_t per = kThreads / G * kCsrNodes;  // nodes a workgroup takes at a time
+    for (int64_t n0 = blockIdx.x * per + threadIdx.x / G * kCsrNodes; n0 < g.nnodes;
+         n0 += gridDim.x * per) {
+        double t[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) t[v] = 0.0;
+        if (!PCG || step) {
+            double xv[kCsrNodes][DIM], kv[kCsrNodes][DIM][DIM];
+            bool on[kCsrNodes];
+#pragma unroll
+            for (int q = 0; q < kCsrNodes; ++q) {
+                const uint32_t n = (uint32_t)(n0 + q < g.nnodes ? n0 + q : n0);
+                const int i = (int)(n % (uint32_t)g.NX), jk = (int)(n / (uint32_t)g.NX);
+                const int j = DIM == 3 ? jk % g.NY : jk, k = DIM == 3 ? jk / g.NY : 0;
+                const int x0 = i > 0 ? -1 : 0, y0 = j > 0 ? -1 : 0, z0 = DIM == 3 && k > 0 ? -1 : 0;
+                const int cx = 1 - x0 + (i < g.NX - 1), cy = 1 - y0 + (j < g.NY - 1),
+                          cz = DIM == 3 ? 1 - z0 + (k < g.NZ - 1) : 1;
+                on[q] = used && n0 + q < g.nnodes && ox >= x0 && ox < x0 + cx && oy >= y0 &&
+                        oy < y0 + cy && oz >= z0 && oz < z0 + cz;
+                const int slot = on[q] ? (ox - x0) + cx * ((oy - y0) + cy * (oz - z0)) : 0;
+                const uint32_t m = on[q] ? n + ox + g.NX * (oy + g.NY * oz) : n;
+                const double* row = vals + rowptr[DIM * (int64_t)n] + DIM * slot;
+                const int len = DIM * cx * cy * cz;
+                ld_node<DIM>(x, m, xv[q]);
+#pragma unroll
+                for (int d = 0; d < DIM; ++d)
+#pragma unroll
+                    for (int e = 0; e < DIM; ++e) kv[q][d][e] = row[d * len + e];
+            }
+#pragma unroll
+            for (int q = 0; q < kCsrNodes; ++q)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int e = 0; e < DIM; ++e) s += kv[q][d][e] * xv[q][e];
+                    t[q * DV + d] = on[q] ? s : 0.0;
+                }
+            // value v of the group ends up in lanes v G / NV ...
+            auto halve = [&](auto half, int bit) {
+                constexpr int h = decltype(half)::value;
+                const bool up = (lane & bit) != 0;
+#pragma unroll
+                for (int v = 0; v < h; ++v) {
+                    const double keep = up ? t[v + h] : t[v], send = up ? t[v] : t[v + h];
+                    t[v] = keep + __shfl_xor(send, bit, 64);
+                }
+            };
+            if constexpr (DIM == 3) halve(std::integral_constant<int, 8>{}, 16);
+            halve(std::integral_constant<int, 4>{}, 8);
+            halve(std::integral_constant<int, 2>{}, 4);
+            halve(std::integral_constant<int, 1>{}, 2);
+            t[0] += __shfl_xor(t[0], 1, 64);
+        }
+        const int v = lane >> 1, q = v / DV, d = v % DV;
+        if ((lane & 1) == 0 && d < DIM && n0 + q < g.nnodes) {
+            const int64_t i = DIM * (n0 + q) + d;
+            if (PCG) {
+                const double r = a.r[i], z = a.dinv[i] * r;
+                sum[kSumRZ] += z * r;
+                sum[kSumRR] += r * r;
+                if (step) {
+                    const double s = t[0];
+                    y[i] = s;
+                    sum[kSumPQ] += x[i] * s;
+                    sum[kSumQZ] += z * s;
+                    sum[kSumQDQ] += a.dinv[i] * s * s;
+                    sum[kSumRQ] += r * s;
+                    sum[kSumQQ] += s * s;
+                }
+            } else {
+                y[i] = t[0];
+            }
         }
     }
-    if (PCG) {
-        const double t = block_sum_all(acc, red);
-        if (threadIdx.x == 0) part[blockIdx.x] = t;
-    }
+    if (PCG) pcg1_store_sums(sum, red, a.part);
 }
 
-// PCG direction for operators that are applied in a separate kernel (the
-// assembled matrix, the heat-conduction operator): reduces the update's
-// (r.z, r.r) partials, tests convergence (the scalar bookkeeping of the fused
-// matrix-free kernel) and writes p_k = dinv .* r + beta p_{k-1} into p[k & 1].
-__global__ __launch_bounds__(kThreads) void k_pcg_direction(int64_t n, const double* __restrict__ r,
-                                                      const double* __restrict__ dinv,
-                                                      const double* p0c, const double* p1c,
-                                                      double* p0, double* p1, PcgScalars* sc,
-                                                      const double* __restrict__ partB, int nbB) {
-    __shared__ double red[kWaves];
-    if (sc->done) return;
-    const long long it = sc->iter;
-    const long long k = it + 1;
-    const double* pold = ((k - 1) & 1) ? p1c : p0c;
-    double* pnew = (k & 1) ? p1 : p0;
-    const double rz = reduce_partials(partB, nbB, 2, 0, red);
-    const double rr = reduce_partials(partB, nbB, 2, 1, red);
-    const double tol_in = sc->tol;
-    const double tol = tol_in < 0.0 ? fmax(sc->reltol * sqrt(rr), sc->abstol) : tol_in;
-    int err;
-    const bool stop = pcg_stop_test(sc, rz, rr, it, tol, err);
-    const double rho_prev = sc->rho[(k - 1) & 1];
-    // Block 0's writes below cannot change what another block computes: rho
-    // goes to the other slot, a block that sees the new tol derives the same
-    // value, and one that sees done = 1 would stop anyway.
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc->rr = rr;
-        if (tol_in < 0.0) {
-            sc->tol = tol;
-            sc->rr0 = rr;
-        }
-        if (stop) {
-            sc->done = 1;
-            if (err) sc->err = err;
-        } else {
-            sc->rho[k & 1] = rz;
-            sc->rho_cur = rz;
-            sc->k_cur = k;
-        }
+// The vector part of an iteration, in place: x += alpha p, r -= alpha q,
+// p = z + beta p (or the update alone, kPcg1Exact), from the product's sums.
+__global__ __launch_bounds__(kThreads) void k_csr_vectors(int64_t n, double* __restrict__ x,
+                                                          double* __restrict__ r,
+                                                          double* __restrict__ p,
+                                                          const double* __restrict__ q,
+                                                          const double* __restrict__ dinv,
+                                                          const Pcg1State* s, Pcg1State* sn,
+                                                          const double* __restrict__ part,
+                                                          int nb) {
+    __shared__ double red[kWaves][kPcg1Vals];
+    const int64_t i0 = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+    const int64_t stride = gridDim.x * (int64_t)kThreads;
+    // the first element's loads are in flight while the sums are formed
+    const int64_t ic = i0 < n ? i0 : 0;
+    double cx = x[ic], cr = r[ic], cp = p[ic], cq = q[ic], cd = dinv[ic];
+    const Pcg1State s0 = *s;
+    if (s0.done) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *sn = s0;
+        return;
     }
-    if (stop) return;
-    const double beta = rz / rho_prev;
-    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * kThreads)
-        pnew[i] = dinv[i] * r[i] + beta * pold[i];
+    double v[kPcg1Vals];
+    pcg1_reduce<kThreads>(part, nb, v, red);
+    Pcg1State s1;
+    const Pcg1Plan plan = pcg1_plan(s0, v, s1);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *sn = s1;
+    if (s1.err != 0 && s0.iter == s1.iter) return;
+    const bool pend = s0.pend != 0;
+    for (int64_t i = i0; i < n; i += stride) {
+        if (i != i0) {
+            cx = x[i];
+            cr = r[i];
+            cp = p[i];
+            cq = q[i];
+            cd = dinv[i];
+        }
+        if (pend) {
+            x[i] = cx + plan.alpha * cp;
+            cr = fma(-plan.alpha, cq, cr);
+            if (plan.mode != kPcg1Stop) r[i] = cr;
+        }
+        if (plan.mode == kPcg1Step) p[i] = fma(plan.beta, cp, cd * cr);
+    }
 }
 
 static unsigned csr_blocks(int64_t work, int per_block) {
@@ -331,32 +412,36 @@ hipError_t launch_csr_dinv(const Grid& g, const double* diag, const uint8_t* fix
     return hipGetLastError();
 }
 
-hipError_t launch_csr_spmv(int64_t nrows, const int64_t* rowptr, const int* cols,
-                           const double* vals, const double* x, double* y, hipStream_t s) {
-    hipLaunchKernelGGL((k_csr_spmv<false>), dim3(csr_blocks(nrows, kThreads / 16)),
-                       dim3(kThreads), 0, s, nrows, rowptr, cols, vals, x, x, y, nullptr,
-                       nullptr);
+static unsigned csr_spmv_blocks(const Grid& g) {
+    const int group = g.dim == 3 ? csr_group<3> : csr_group<2>;
+    return std::min(csr_blocks(g.nnodes, kThreads / group * kCsrNodes), 2048u);
+}
+int csr_pcg1_blocks(const Grid& g) { return (int)csr_spmv_blocks(g); }
+
+hipError_t launch_csr_spmv(const Grid& g, const int64_t* rowptr, const double* vals,
+                           const double* x, double* y, hipStream_t s) {
+    const dim3 grid(csr_spmv_blocks(g)), block(kThreads);
+    const CsrPcgArgs a{};
+    if (g.dim == 3)
+        hipLaunchKernelGGL((k_csr_spmv<3, false>), grid, block, 0, s, g, rowptr, vals, x, y, a);
+    else
+        hipLaunchKernelGGL((k_csr_spmv<2, false>), grid, block, 0, s, g, rowptr, vals, x, y, a);
     return hipGetLastError();
 }
 
-hipError_t launch_pcg_direction(int64_t n, const double* r, const double* dinv, double* p0,
-                                double* p1, PcgScalars* sc, const double* partB, int nbB,
-                                hipStream_t s) {
-    hipLaunchKernelGGL(k_pcg_direction, dim3(kVecBlocks), dim3(kThreads), 0, s, n, r, dinv, p0,
-                       p1, p0, p1, sc, partB, nbB);
+hipError_t launch_csr_pcg1(const Grid& g, const int64_t* rowptr, const double* vals, double* x,
+                           double* r, double* p, double* q, const double* dinv,
+                           const Pcg1State* st, Pcg1State* stn, double* part, hipStream_t s) {
+    const dim3 grid(csr_spmv_blocks(g)), block(kThreads);
+    const unsigned nv = std::min(csr_blocks(g.ndof, kThreads), 1024u);
+    hipLaunchKernelGGL(k_csr_vectors, dim3(nv), block, 0, s, g.ndof, x, r, p, q, dinv, st, stn,
+                       part, (int)grid.x);
+    const CsrPcgArgs a{r, dinv, stn, part};
+    if (g.dim == 3)
+        hipLaunchKernelGGL((k_csr_spmv<3, true>), grid, block, 0, s, g, rowptr, vals, p, q, a);
+    else
+        hipLaunchKernelGGL((k_csr_spmv<2, true>), grid, block, 0, s, g, rowptr, vals, p, q, a);
     return hipGetLastError();
-}
-
-hipError_t launch_csr_pcg_iter(int64_t n, const int64_t* rowptr, const int* cols,
-                               const double* vals, double* x, double* r, const double* dinv,
-                               double* p0, double* p1, double* q, PcgScalars* sc, double* partA,
-                               double* partB, hipStream_t s) {
-    if (hipError_t e = launch_pcg_direction(n, r, dinv, p0, p1, sc, partB, kVecBlocks, s))
-        return e;
-    const unsigned nbA = csr_blocks(n, kThreads / 16);
-    hipLaunchKernelGGL((k_csr_spmv<true>), dim3(nbA), dim3(kThreads), 0, s, n, rowptr, cols,
-                       vals, p0, p1, q, sc, partA);
-    return launch_pcg_update<double>(n, x, r, p0, p1, q, dinv, sc, partA, (int)nbA, partB, s);
 }
 
 }  // namespace tohip

@@ -196,6 +196,17 @@ int pcg1_blocks(const Grid& g);
 hipError_t launch_pcg1(const Grid& g, const ElemOp<double>& op, const uint8_t* fixmask,
                        const double* E, double meandiag, const Pcg1Args& a, hipStream_t s);
 
+// y = K x on the assembled matrix, whose row pattern is the grid's (k_csr.hip).
+hipError_t launch_csr_spmv(const Grid& g, const int64_t* rowptr, const double* vals,
+                           const double* x, double* y, hipStream_t s);
+// One PCG iteration on it: the vectors in place from the state st and the product's
+// sums in part (csr_pcg1_blocks rows), then q = K p with the next sums; stn is the
+// state left.
+int csr_pcg1_blocks(const Grid& g);
+hipError_t launch_csr_pcg1(const Grid& g, const int64_t* rowptr, const double* vals, double* x,
+                           double* r, double* p, double* q, const double* dinv,
+                           const Pcg1State* st, Pcg1State* stn, double* part, hipStream_t s);
+
 // Iterations (launches) of the long and the short captured graph; even, so that
 // a graph starts and ends on the first set of vectors.
 constexpr int kPcg1GraphLong = 64, kPcg1GraphShort = 8;
