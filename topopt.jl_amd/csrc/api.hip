@@ -321,6 +321,7 @@ int mg_refresh(tohip_ctx* ctx) {
         CK(launch_jacobi_inv<float>(C.g, C.op64, C.E64, C.fixmask, ctx->meandiag, C.dinv,
                                     ctx->stream));
     }
+    ctx->mg_sweepM_now = false;
     if (ctx->mg_M) {
         // the coarsest operator changed: rebuild its dense form on the second
         // stream, after the moduli and diagonals above (TOHIP_MG_OVERLAP=0, read
@@ -351,6 +352,18 @@ int mg_join(tohip_ctx* ctx) {
     if (!ctx->mg_pending) return 0;
     CK(hipStreamWaitEvent(ctx->stream, ctx->mg_ev[1], 0));
     ctx->mg_pending = false;
+    return 0;
+}
+
+// Called before a solve's graphs: mg_join, and the matrix of a coarsest level of
+// sweeps, built here and not at the refresh because one V-cycle alone (the
+// inspection entry point) is cheaper by sweeps.
+int mg_solve_ready(tohip_ctx* ctx) {
+    if (int rc = mg_join(ctx)) return rc;
+    if (!ctx->mg_sweepM || ctx->mg_sweepM_now) return 0;
+    const tohip_mg_level& C = ctx->mg.back();
+    CK(launch_mg_sweep_basis(C.view(), C.omega, ctx->mg_sweeps, ctx->mg_sweepM, ctx->stream));
+    ctx->mg_sweepM_now = true;
     return 0;
 }
 
@@ -492,6 +505,14 @@ int mg_setup(tohip_ctx* ctx) {
             return rc;
         }
     }
+    if (mg_sweeps_dense_fits(lv.back().g) && !(ed && atoi(ed) == 0)) {
+        const Grid& gc = lv.back().g;
+        if (int rc = dalloc(ctx, &ctx->mg_sweepM, (size_t)gc.ndof * mg_sweeps_dense_ld(gc))) {
+            hipStreamSynchronize(ctx->stream);
+            free_mg_levels(lv);
+            return rc;
+        }
+    }
     // smoother weights in device memory: the bound's weight until the first
     // estimate; TOHIP_MG_WADAPT=0 (or a forced TOHIP_MG_OMEGA) keeps it
     {
@@ -590,8 +611,10 @@ int mg_build_levels(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<toh
 // kernel reduces (*nb_part of them).  With `upd`, the finest pre-smoothing
 // first applies the pending PCG update to r and x (the cycle then runs on the
 // new residual, which it writes to upd->rnew).
+// `dense`: apply a coarsest level of sweeps as its matrix (the solves' graphs, which
+// run after mg_solve_ready; elsewhere while it is of the current operator).
 hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, double* part,
-                         int* nb_part, const MgFusedUpdate* upd = nullptr) {
+                         int* nb_part, const MgFusedUpdate* upd = nullptr, bool dense = true) {
     std::vector<tohip_mg_level>& M = ctx->mg;
     const int L = (int)M.size() - 1;
     const double md = ctx->meandiag;
@@ -613,6 +636,10 @@ hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, d
     if (ctx->mg_M) {
         if ((e = launch_mg_dense((int)CL.g.ndof, ctx->mg_M, M[L].b, M[L].x, sc,
                                  s)) != hipSuccess)
+            return e;
+    } else if (ctx->mg_sweepM && dense) {
+        if ((e = launch_mg_dense_wide((int)CL.g.ndof, mg_sweeps_dense_ld(CL.g), ctx->mg_sweepM,
+                                      M[L].b, M[L].x, sc, s)) != hipSuccess)
             return e;
     } else if (mg_coarse_fits(CL.g)) {
         if ((e = launch_mg_coarse(CL, ctx->mg_cheb, M[L].b, M[L].x, sc, s)) != hipSuccess)
@@ -809,7 +836,7 @@ std::pair<int, int> mg_graph_iters() {
 }
 
 int run_mg_graphs(tohip_ctx* ctx) {
-    if (int rc = mg_join(ctx)) return rc;
+    if (int rc = mg_solve_ready(ctx)) return rc;
     const auto [nl, ns] = mg_graph_iters();
     if (int rc = capture_mg_graph(ctx, &ctx->g32mg, nl)) return rc;
     if (int rc = capture_mg_graph(ctx, &ctx->g32mgs, ns)) return rc;
@@ -1106,7 +1133,7 @@ int solve_fp64_mg(tohip_ctx* ctx, double abstol, double reltol, int64_t maxiter,
         CK(launch_pcg_start<double>(n, ctx->b64, ctx->t64, ctx->r64, ctx->ones64, ctx->p64[0],
                                     ctx->sc64, ctx->partB, 0, ctx->stream));
     }
-    if (int rc = mg_join(ctx)) return rc;
+    if (int rc = mg_solve_ready(ctx)) return rc;
     const auto [nl, ns] = mg_graph_iters();
     if (int rc = capture_fp64_mg_graph(ctx, &ctx->g64mg, nl)) return rc;
     if (int rc = capture_fp64_mg_graph(ctx, &ctx->g64mgs, ns)) return rc;
@@ -1247,7 +1274,7 @@ void free_ctx(tohip_ctx* ctx) {
                     (void*)ctx->mma_x1, (void*)ctx->mma_x2, (void*)ctx->mma_st,
                     (void*)ctx->mg_M, (void*)ctx->r32b, (void*)ctx->mg_wd, (void*)ctx->r64b,
                     (void*)ctx->pcg1_part[0], (void*)ctx->pcg1_part[1], (void*)ctx->pcg1_st,
-                    (void*)ctx->csr_part, (void*)ctx->csr_st})
+                    (void*)ctx->csr_part, (void*)ctx->csr_st, (void*)ctx->mg_sweepM})
         if (b) hipFree(b);
     if (ctx->h_pcg1) hipHostFree(ctx->h_pcg1);
     if (ctx->h_mma) hipHostFree(ctx->h_mma);
@@ -1812,7 +1839,7 @@ int tohip_mg_apply(tohip_ctx* ctx, const double* r, double* z) {
     if (int rc = upload_dofs(ctx, r, ctx->r64)) return rc;
     CK(launch_f64_to_f32(ctx->g.ndof, ctx->r64, ctx->b32, ctx->stream));
     if (int rc = mg_join(ctx)) return rc;
-    CK(launch_vcycle(ctx, ctx->b32, nullptr, nullptr, nullptr));
+    CK(launch_vcycle(ctx, ctx->b32, nullptr, nullptr, nullptr, nullptr, ctx->mg_sweepM_now));
     std::vector<float> zf(ctx->g.ndof);
     CK(hipMemcpyAsync(zf.data(), ctx->mg[0].rz, zf.size() * sizeof(float),
                       hipMemcpyDeviceToHost, ctx->stream));
@@ -2466,10 +2493,10 @@ int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
         ctx->err = "tohip_bench_kernel: set up the filter first";
         return TOHIP_ERR_STATE;
     }
-    if (kernel >= TOHIP_K_MG_PRE) {
+    if (kernel >= TOHIP_K_MG_PRE && kernel <= TOHIP_K_VCYCLE) {
         // operands of the single-kernel timings: one full V-cycle on r32
         // leaves every level's x, rz and b filled
-        if (int rc = mg_join(ctx)) return rc;
+        if (int rc = mg_solve_ready(ctx)) return rc;
         CK(launch_vcycle(ctx, ctx->r32, nullptr, nullptr, nullptr));
     }
     if (kernel == TOHIP_K_OC) {

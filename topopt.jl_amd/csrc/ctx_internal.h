@@ -104,6 +104,10 @@ struct tohip_ctx {
     // dense coarsest-level operator of the multigrid V-cycle (ndof^2 floats,
     // symmetric); null when the iteration kernel is used instead
     float* mg_M = nullptr;
+    // the same for a coarsest level of sweeps; rebuilt at the start of the first
+    // solve after an operator refresh (mg_sweepM_now: it is of this operator)
+    float* mg_sweepM = nullptr;
+    bool mg_sweepM_now = false;
     hipGraphExec_t gcsr = nullptr, gcsrs = nullptr;
     double* csr_part = nullptr;  // partial sums and states of its PCG (k_pcg1.h)
     tohip::Pcg1State* csr_st = nullptr;

@@ -861,14 +861,33 @@ hipError_t launch_mg_coarse(const MgLevelView& L, const MgCheb& ch, const float*
 // workgroup, in one launch.
 constexpr int kMgDenseMaxSteps = (3 * kMgCoarseMaxNodes + 63) / 64;
 
-__global__ __launch_bounds__(256) void k_mg_dense_sym(int n, float* __restrict__ M) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (int64_t)n * n) return;
-    const int i = (int)(t / n), j = (int)(t % n);
-    if (i >= j) return;  // each unordered pair {i, j} once
-    const float s = 0.5f * (M[(size_t)j * n + i] + M[(size_t)i * n + j]);
-    M[(size_t)j * n + i] = s;
-    M[(size_t)i * n + j] = s;
+// M <- (M + M^T) / 2 by pairs of 32 x 32 tiles through LDS, both sides read and
+// written by rows (the tile pair (I, J), I <= J, is block I + J (J + 1) / 2).
+__global__ __launch_bounds__(256) void k_mg_dense_sym(int n, int ld, float* __restrict__ M) {
+    __shared__ float ta[32][33], tb[32][33];
+    int J = (int)((sqrtf(8.f * (float)blockIdx.x + 1.f) - 1.f) * 0.5f);
+    while ((J + 1) * (J + 2) / 2 <= (int)blockIdx.x) ++J;  // exact against the root's rounding
+    while (J * (J + 1) / 2 > (int)blockIdx.x) --J;
+    const int I = (int)blockIdx.x - J * (J + 1) / 2;
+    const int x = threadIdx.x & 31, y0 = threadIdx.x >> 5;
+    for (int y = y0; y < 32; y += 8) {
+        const int i = 32 * I + y, j = 32 * J + x;
+        ta[y][x] = i < n && j < n ? M[(size_t)i * ld + j] : 0.f;
+        const int i2 = 32 * J + y, j2 = 32 * I + x;
+        tb[y][x] = i2 < n && j2 < n ? M[(size_t)i2 * ld + j2] : 0.f;
+    }
+    __syncthreads();
+    for (int y = y0; y < 32; y += 8) {
+        const int i = 32 * I + y, j = 32 * J + x;
+        if (i < n && j < n) M[(size_t)i * ld + j] = 0.5f * (ta[y][x] + tb[x][y]);
+        const int i2 = 32 * J + y, j2 = 32 * I + x;
+        if (I != J && i2 < n && j2 < n) M[(size_t)i2 * ld + j2] = 0.5f * (tb[y][x] + ta[x][y]);
+    }
+}
+static void launch_mg_dense_sym(int n, int ld, float* M, hipStream_t s) {
+    const int nt = (n + 31) / 32;
+    hipLaunchKernelGGL(k_mg_dense_sym, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(256), 0, s, n, ld,
+                       M);
 }
 
 __global__ __launch_bounds__(256) void k_mg_dense_rows(int n, const float* __restrict__ M,
@@ -912,9 +931,7 @@ hipError_t launch_mg_coarse_basis(const MgLevelView& L, const MgCheb& ch, float*
         hipLaunchKernelGGL((k_mg_coarse<2, false, true>), grid, dim3(kMgCoarseThreads), 0, s,
                            L.g, L.op, L.E32, L.fixmask, L.dinv, ch, nullptr, Mout, nullptr);
     }
-    const int n = (int)L.g.ndof;
-    const unsigned nb = (unsigned)(((int64_t)n * n + 255) / 256);
-    hipLaunchKernelGGL(k_mg_dense_sym, dim3(nb), dim3(256), 0, s, n, Mout);
+    launch_mg_dense_sym((int)L.g.ndof, (int)L.g.ndof, Mout, s);
     return hipGetLastError();
 }
 
@@ -923,6 +940,197 @@ hipError_t launch_mg_dense(int n, const float* M, const float* b, float* x, cons
     if (n < 1 || n > 3 * kMgCoarseMaxNodes) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_mg_dense_rows, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, n, M, b, x,
                        sc);
+    return hipGetLastError();
+}
+
+// ---- dense form of a coarsest level of sweeps ----
+// A coarsest level that cannot be halved again and is too large for k_mg_coarse
+// is solved by damped Jacobi sweeps, a launch each: 30 x 3.9 us of a 176 us
+// V-cycle at 76x36x28 cells (coarsest 19x9x7).  The sweeps are a fixed linear
+// operator too, so its matrix (ld x n floats, 92 MB there) is built by one
+// workgroup per column with the level in LDS, and a V-cycle reads it once: a PCG
+// iteration there takes 84 us instead of 190 (a solve of 104 iterations with its
+// set-up 11.2 ms instead of 25.8).  The limits: a level in LDS, two nodes and two
+// cells a thread, and n^2 floats (117 MB) that a V-cycle reads faster than it
+// launches sweeps.
+constexpr int kMgSweepThreads = 1024, kMgSweepMaxDofs = 5400;
+static size_t mg_sweep_lds(const Grid& g) {
+    return sizeof(float) * (size_t)g.dim * (size_t)(g.nnodes + ((int64_t)g.ncells << g.dim));
+}
+bool mg_sweeps_dense_fits(const Grid& g) {
+    return !mg_coarse_fits(g) && g.ndof <= kMgSweepMaxDofs && g.nnodes <= 2 * kMgSweepThreads &&
+           g.ncells <= 2 * kMgSweepThreads && mg_sweep_lds(g) <= 156 * 1024;
+}
+int mg_sweeps_dense_ld(const Grid& g) { return ((int)g.ndof + 63) / 64 * 64; }
+
+template <int DIM, bool CUBE>
+__global__ __launch_bounds__(kMgSweepThreads) void k_mg_sweep_basis(
+    Grid g, ElemOp<float> op, const float* __restrict__ E, const uint8_t* __restrict__ fixmask,
+    const float* __restrict__ dinv, float w, int sweeps, int ld, float* __restrict__ M) {
+    constexpr int NC = 1 << DIM, PT = 2;
+    extern __shared__ float lds[];
+    const int nn = (int)g.nnodes, ne = (int)g.ncells, n = (int)g.ndof, col = blockIdx.x;
+    float* xs = lds;                 // [DIM][nn]
+    float* res = lds + DIM * nn;     // [DIM * NC][ne]
+    float* row = M + (size_t)col * ld;
+    const int t = threadIdx.x;
+    for (int i = n + t; i < ld; i += kMgSweepThreads) row[i] = 0.f;  // the padding
+    if ((fixmask[col / DIM] >> (col % DIM)) & 1) {  // a prescribed DOF's column is 0
+        for (int i = t; i < n; i += kMgSweepThreads) row[i] = 0.f;
+        return;
+    }
+    float bn[PT][DIM], wd[PT][DIM], Ee[PT];
+    int ecell0[PT], ncorner0[PT];
+    unsigned cmask[PT];
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+        const int v = t + q * kMgSweepThreads;
+        cmask[q] = 0;
+        ecell0[q] = ncorner0[q] = 0;
+        Ee[q] = 0.f;
+        if (v < nn) {
+            const int gi = v % g.NX, gj = (v / g.NX) % g.NY, gk = DIM == 3 ? v / (g.NX * g.NY) : 0;
+            const uint8_t m = fixmask[v];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                const bool fx = (m >> d) & 1;
+                bn[q][d] = !fx && DIM * v + d == col ? 1.f : 0.f;
+                wd[q][d] = fx ? 0.f : w * dinv[DIM * v + d];
+                xs[d * nn + v] = wd[q][d] * bn[q][d];
+            }
+            ecell0[q] = gi + g.nx * (gj + g.ny * gk);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int ci = gi - (c & 1), cj = gj - ((c >> 1) & 1),
+                          ck = DIM == 3 ? gk - ((c >> 2) & 1) : 0;
+                if (ci >= 0 && ci < g.nx && cj >= 0 && cj < g.ny && ck >= 0 && ck < g.nz)
+                    cmask[q] |= 1u << c;
+            }
+        }
+        if (v < ne) {
+            const int ei = v % g.nx, ej = (v / g.nx) % g.ny, ek = DIM == 3 ? v / (g.nx * g.ny) : 0;
+            Ee[q] = E[v];
+            ncorner0[q] = ei + g.NX * (ej + g.NY * ek);
+        }
+    }
+    const int sy = g.NX, sz = g.NX * g.NY, cy = g.nx, cz = g.nx * g.ny;
+    __syncthreads();
+    for (int k = 1; k < sweeps; ++k) {
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+            const int v = t + q * kMgSweepThreads;
+            if (v < ne) {
+                float xe[DIM][NC], ye[DIM][NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const int m = ncorner0[q] + (c & 1) + ((c >> 1) & 1) * sy + ((c >> 2) & 1) * sz;
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) xe[d][c] = xs[d * nn + m];
+                }
+                elem_apply<float, DIM, CUBE>(op, xe, ye);
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) res[(c * DIM + d) * ne + v] = Ee[q] * ye[d][c];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+            const int v = t + q * kMgSweepThreads;
+            if (v < nn) {
+                float s[DIM];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) s[d] = 0.f;
+#pragma unroll
+                for (int c = NC - 1; c >= 0; --c) {
+                    if (!((cmask[q] >> c) & 1)) continue;
+                    const int e = ecell0[q] - (c & 1) - ((c >> 1) & 1) * cy - ((c >> 2) & 1) * cz;
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) s[d] += res[(c * DIM + d) * ne + e];
+                }
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) xs[d * nn + v] += wd[q][d] * (bn[q][d] - s[d]);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+        const int v = t + q * kMgSweepThreads;
+        if (v < nn)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) row[DIM * v + d] = xs[d * nn + v];
+    }
+}
+
+hipError_t launch_mg_sweep_basis(const MgLevelView& L, float w, int sweeps, float* M,
+                                 hipStream_t s) {
+    if (!mg_sweeps_dense_fits(L.g) || sweeps < 1) return hipErrorInvalidValue;
+    const int ld = mg_sweeps_dense_ld(L.g);
+    const size_t lds = mg_sweep_lds(L.g);
+    const dim3 grid((unsigned)L.g.ndof), block(kMgSweepThreads);
+#define TOHIP_BASIS(D, C)                                                                       \
+    do {                                                                                        \
+        const hipError_t e = hipFuncSetAttribute(                                               \
+            reinterpret_cast<const void*>(&k_mg_sweep_basis<D, C>),                             \
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                              \
+        if (e != hipSuccess) return e;                                                          \
+        hipLaunchKernelGGL((k_mg_sweep_basis<D, C>), grid, block, lds, s, L.g, L.op, L.E32,     \
+                           L.fixmask, L.dinv, w, sweeps, ld, M);                                \
+    } while (0)
+    if (L.g.dim == 2)
+        TOHIP_BASIS(2, false);
+    else if (L.op.is_cube)
+        TOHIP_BASIS(3, true);
+    else
+        TOHIP_BASIS(3, false);
+#undef TOHIP_BASIS
+    launch_mg_dense_sym((int)L.g.ndof, ld, M, s);
+    return hipGetLastError();
+}
+
+// x = M b, one wave per row of ld floats (a multiple of 64, zeros past n), 16
+// bytes a lane.
+__global__ __launch_bounds__(256) void k_mg_dense_wide(int n, int ld, const float* __restrict__ M,
+                                                       const float* __restrict__ b,
+                                                       float* __restrict__ x,
+                                                       const PcgScalars* sc) {
+    __shared__ __align__(16) float bs[(kMgSweepMaxDofs + 63) / 64 * 64];
+    const int lane = threadIdx.x & 63;
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const float4* row = reinterpret_cast<const float4*>(M + (size_t)min(i, n - 1) * ld);
+    const int nq = ld / 4;
+    constexpr int U = 8;
+    float4 v[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) v[q] = row[min(lane + 64 * q, nq - 1)];
+    if (mg_done(sc)) return;
+    for (int j = threadIdx.x; j < ld; j += 256) bs[j] = j < n ? b[j] : 0.f;
+    __syncthreads();
+    const float4* bv = reinterpret_cast<const float4*>(bs);
+    float acc = 0.f;
+    for (int q0 = 0; q0 < nq; q0 += 64 * U) {
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int j = q0 + lane + 64 * q;
+            if (j < nq) {
+                const float4 w = bv[j];
+                acc += v[q].x * w.x + v[q].y * w.y + v[q].z * w.z + v[q].w * w.w;
+            }
+            v[q] = row[min(j + 64 * U, nq - 1)];
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0 && i < n) x[i] = acc;
+}
+
+hipError_t launch_mg_dense_wide(int n, int ld, const float* M, const float* b, float* x,
+                                const PcgScalars* sc, hipStream_t s) {
+    if (n < 1 || n > kMgSweepMaxDofs || ld % 64 || ld < n) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mg_dense_wide, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, n, ld, M, b,
+                       x, sc);
     return hipGetLastError();
 }
 

@@ -350,6 +350,14 @@ hipError_t launch_mg_coarse_basis(const MgLevelView& L, const MgCheb& ch, float*
                                   hipStream_t s);
 hipError_t launch_mg_dense(int n, const float* M, const float* b, float* x, const PcgScalars* sc,
                            hipStream_t s);
+// The same for a coarsest level of damped Jacobi sweeps: whether its matrix is
+// worth keeping, its leading dimension, its build and its product.
+bool mg_sweeps_dense_fits(const Grid& g);
+int mg_sweeps_dense_ld(const Grid& g);
+hipError_t launch_mg_sweep_basis(const MgLevelView& L, float w, int sweeps, float* M,
+                                 hipStream_t s);
+hipError_t launch_mg_dense_wide(int n, int ld, const float* M, const float* b, float* x,
+                                const PcgScalars* sc, hipStream_t s);
 // Coarse cell moduli: mean of the 2^dim children.
 hipError_t launch_mg_coarsen(const Grid& gf, const Grid& gc, const double* Ef, double* E64,
                              float* E32, hipStream_t s);
