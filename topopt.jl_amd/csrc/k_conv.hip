@@ -18,6 +18,7 @@
 //   that a second kernel sums in a fixed order (deterministic).
 #include <stdint.h>
 
+#include <algorithm>
 #include <cstdlib>
 
 #include "k_common.h"
@@ -213,261 +214,306 @@ hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t*
 }
 
 // ---------------------------------------------------------- weight grad --
-// Block = one wave: (tap, 16 input channels, 16 output channels, position
-// split).  A[m = co][k = p] = dY[p][co], B[k = p][n = ci] = X[p + tap - pad][ci].
-__global__ __launch_bounds__(64) void k_conv_bwd_w(ConvDesc c, const uint16_t* __restrict__ X,
-                                                   const uint16_t* __restrict__ dY,
-                                                   float* __restrict__ part, int nsplit) {
-    const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
-    const int T = c.kd * c.kh * c.kw;
-    const int nci = c.Cin32 / 16;
-    const int tap = blockIdx.x / nci, ci0 = (blockIdx.x % nci) * 16;
-    const int co0 = blockIdx.y * 16;
-    const int split = blockIdx.z;
-    const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
-    const int64_t chunk = ((P + nsplit - 1) / nsplit + 31) / 32 * 32;
-    const int64_t pb = split * chunk, pe = pb + chunk < P ? pb + chunk : P;
-    const int dz = tap / (c.kh * c.kw), dy = (tap / c.kw) % c.kh, dx = tap % c.kw;
-    const int co = co0 + row, ci = ci0 + row;
-    const bool co_ok = co < c.Cout, ci_ok = ci < c.Cin;
-    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    // Output position of this lane's first element, advanced incrementally
-    // (no div/mod chain per element): p = ((b*OD + oz)*OH + oy)*OW + ox.
-    int ox, oy, oz, bb;
-    {
-        int64_t t = pb + 8 * kq;
-        ox = (int)(t % c.OW);
-        t /= c.OW;
-        oy = (int)(t % c.OH);
-        t /= c.OH;
-        oz = (int)(t % c.OD);
-        bb = (int)(t / c.OD);
-    }
-    for (int64_t base = pb; base < pe; base += 32) {
-        bf16x8 a, bv;
-        int x0 = ox, y0 = oy, z0 = oz, b0 = bb;
+// dW[co][tap][ci] = sum_p dY[p][co] X[p + tap - pad][ci] with the positions as the
+// K dimension of the MFMA.  A lane's 8 consecutive k are the same place of 8
+// separate spatial tiles ("subs"), so that in LDS, [place][16 channels][8 subs], an
+// operand is one aligned 16-byte read for every tap's shift.  A K-step is 4
+// consecutive y (the lane quarters) of the 8 subs.
+//
+// A workgroup takes 16 input channels, MC tiles of 16 output channels and every
+// taps of units of 8 subs (8 x TY x TZ outputs each): it stages the inputs with
+// their halo and the output gradients once (8 channels of 8 subs a thread,
+// transposed in registers) and forms all K^3 taps from them.  A wave keeps one
+// output tile's K^3 accumulators and walks x with a window of K inputs per (dz,
+// dy) in registers: K^2 + 1 LDS reads for K^3 MFMAs.  Waves beyond the MC tiles
+// take other (y, z) places; their sums are added through LDS in wave order.  The
+// bias gradient is one more MFMA a step against ones.  Splits over the units are
+// summed by k_conv_wgrad_sum in a fixed order.
+//
+// Bound by the staging (the halo is read 3 to 4 times from L2) and, per MFMA, by
+// little else: MI355X, 64x32x32, batch 8, the weight and bias gradients of a step's
+// 15 layers take 0.55 ms, against 2.34 ms for a wave per tap and 16 x 16 tile that
+// gathered both operands again for every tap, with kernels of their own for the
+// bias (130 TFLOP/s against 30).
+constexpr int kWgTX = 8, kWgSubs = 8;
+
+struct WgradShape {
+    int ntx, nty, ntz, ntiles, nunits, ns, ct, it;
+};
+
+// 8 subs x 8 channels (one uint4 of 8 channels per sub) -> 8 channels x 8 subs.
+__device__ __forceinline__ void transpose8(const uint4 (&r)[kWgSubs], uint4 (&o)[8]) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int64_t p = base + 8 * kq + i;
-            uint16_t av = 0, xv = 0;
-            if (p < pe) {
-                if (co_ok) av = dY[p * c.Cout + co];
-                const int iz = z0 + dz - c.pd, iy = y0 + dy - c.ph, ix = x0 + dx - c.pw;
-                if (ci_ok && iz >= 0 && iz < c.D && iy >= 0 && iy < c.H && ix >= 0 && ix < c.W)
-                    xv = X[((((int64_t)b0 * c.D + iz) * c.H + iy) * c.W + ix) * c.Cin + ci];
-            }
-            a[i] = __builtin_bit_cast(__bf16, av);
-            bv[i] = __builtin_bit_cast(__bf16, xv);
-            // next position
-            if (++x0 == c.OW) {
-                x0 = 0;
-                if (++y0 == c.OH) {
-                    y0 = 0;
-                    if (++z0 == c.OD) {
-                        z0 = 0;
-                        ++b0;
-                    }
-                }
-            }
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc, 0, 0, 0);
-        // advance this lane's start by 32 positions
-        int step = 32;
-        while (step > 0) {
-            const int room = c.OW - ox;
-            if (step < room) {
-                ox += step;
-                step = 0;
-            } else {
-                step -= room;
-                ox = 0;
-                if (++oy == c.OH) {
-                    oy = 0;
-                    if (++oz == c.OD) {
-                        oz = 0;
-                        ++bb;
-                    }
-                }
-            }
-        }
-    }
-    // D[m = co0 + 4kq + i][n = ci0 + row]
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int com = co0 + 4 * kq + i;
-        if (com < c.Cout)
-            part[(((int64_t)split * c.Cout + com) * T + tap) * c.Cin32 + ci0 + row] = acc[i];
+    for (int j = 0; j < 4; ++j) {
+        auto w = [&](int s) {
+            return j == 0 ? r[s].x : j == 1 ? r[s].y : j == 2 ? r[s].z : r[s].w;
+        };
+        // bytes 0-1 (2-3) of both words: the even (odd) channel of two subs
+        auto lo = [&](int s) { return __builtin_amdgcn_perm(w(s + 1), w(s), 0x05040100u); };
+        auto hi = [&](int s) { return __builtin_amdgcn_perm(w(s + 1), w(s), 0x07060302u); };
+        o[2 * j] = make_uint4(lo(0), lo(2), lo(4), lo(6));
+        o[2 * j + 1] = make_uint4(hi(0), hi(2), hi(4), hi(6));
     }
 }
 
-// The same tile through LDS: per step of 32 positions each lane loads one
-// position's 8 output-gradient and 8 input channels with 16-byte loads (lane
-// = 2 * position + half), writes them transposed into LDS ([channel][k]), and
-// the MFMA operands come back as one 16-byte LDS read per lane, instead of 16
-// scattered 2-byte global loads per lane per MFMA.  Needs Cin and Cout
-// multiples of 8 and 16-byte aligned tensors (checked at launch).
-__global__ __launch_bounds__(64) void k_conv_bwd_w_lds(ConvDesc c, const uint16_t* __restrict__ X,
-                                                       const uint16_t* __restrict__ dY,
-                                                       float* __restrict__ part, int nsplit) {
-    constexpr int KP = 32 + 8;  // LDS row: 32 positions + 8 of padding (16-byte aligned rows)
-    __shared__ __align__(16) uint16_t sA[16][KP];  // [co - co0][k]
-    __shared__ __align__(16) uint16_t sB[16][KP];  // [ci - ci0][k]
-    const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
-    const int lp = lane >> 1, lh = lane & 1;  // loading role: position, channel half
-    const int T = c.kd * c.kh * c.kw;
-    const int nci = c.Cin32 / 16;
-    const int tap = blockIdx.x / nci, ci0 = (blockIdx.x % nci) * 16;
-    const int co0 = blockIdx.y * 16;
-    const int split = blockIdx.z;
-    const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
-    const int64_t chunk = ((P + nsplit - 1) / nsplit + 31) / 32 * 32;
-    const int64_t pb = split * chunk, pe = pb + chunk < P ? pb + chunk : P;
-    const int dz = tap / (c.kh * c.kw), dy = (tap / c.kw) % c.kh, dx = tap % c.kw;
-    const int col = co0 + 8 * lh, cil = ci0 + 8 * lh;  // this lane's 8 channels
-    const bool co_ok = col < c.Cout, ci_ok = cil < c.Cin;
-    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    // output position p = base + lp, advanced by 32 per step
-    int ox, oy, oz, bb;
-    {
-        int64_t t = pb + lp;
-        ox = (int)(t % c.OW);
-        t /= c.OW;
-        oy = (int)(t % c.OH);
-        t /= c.OH;
-        oz = (int)(t % c.OD);
-        bb = (int)(t / c.OD);
-    }
-    for (int64_t base = pb; base < pe; base += 32) {
-        const int64_t p = base + lp;
-        uint4 av = make_uint4(0, 0, 0, 0), xv = make_uint4(0, 0, 0, 0);
-        if (p < pe) {
-            if (co_ok) av = *reinterpret_cast<const uint4*>(dY + p * c.Cout + col);
-            const int iz = oz + dz - c.pd, iy = oy + dy - c.ph, ix = ox + dx - c.pw;
-            if (ci_ok && iz >= 0 && iz < c.D && iy >= 0 && iy < c.H && ix >= 0 && ix < c.W)
-                xv = *reinterpret_cast<const uint4*>(
-                    X + ((((int64_t)bb * c.D + iz) * c.H + iy) * c.W + ix) * c.Cin + cil);
-        }
-        const uint32_t aw[4] = {av.x, av.y, av.z, av.w}, xw[4] = {xv.x, xv.y, xv.z, xv.w};
+template <int MC, int TY, int TZ, int K>
+__global__ __launch_bounds__(256) void k_conv_wgrad(ConvDesc c, WgradShape sh,
+                                                    const uint16_t* __restrict__ X,
+                                                    const uint16_t* __restrict__ dY,
+                                                    float* __restrict__ part,
+                                                    float* __restrict__ bpart) {
+    constexpr int HX = kWgTX + K - 1, HY = TY + K - 1, HZ = TZ + K - 1, T = K * K * K;
+    constexpr int NX = HX * HY * HZ, NY = kWgTX * TY * TZ, PG = 4 / MC;
+    static_assert((TY / 4) * TZ == PG, "a place group per wave");
+    constexpr int kPl = 16 * kWgSubs;  // elements of a place: 16 channels x 8 subs
+    extern __shared__ __align__(16) uint16_t wg_lds[];
+    uint16_t* sx = wg_lds;            // [NX][16][8]
+    uint16_t* sy = wg_lds + NX * kPl;  // [MC][NY][16][8]
+    __shared__ int4 org[kWgSubs];     // first output of a sub and its batch (-1: none)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 15, kq = lane >> 4;
+    const int m = wave % MC, pg = wave / MC, y0 = 4 * (pg % (TY / 4)), z0 = pg / (TY / 4);
+    const int ci0 = blockIdx.z * 16, co0 = blockIdx.y * 16 * MC;
+
+    f4 acc[T], accb = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            sA[8 * lh + 2 * j][lp] = (uint16_t)(aw[j] & 0xffffu);
-            sA[8 * lh + 2 * j + 1][lp] = (uint16_t)(aw[j] >> 16);
-            sB[8 * lh + 2 * j][lp] = (uint16_t)(xw[j] & 0xffffu);
-            sB[8 * lh + 2 * j + 1][lp] = (uint16_t)(xw[j] >> 16);
+    for (int t = 0; t < T; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t one2 = 0x3f803f80u;  // two BF16 ones
+    const uint4 one4 = make_uint4(one2, one2, one2, one2);
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, one4);
+
+    for (int u = blockIdx.x; u < sh.nunits; u += sh.ns) {
+        __syncthreads();  // the previous unit's reads
+        if (tid < kWgSubs) {
+            int t = u * kWgSubs + tid;
+            int4 o = make_int4(0, 0, 0, -1);
+            if (t < sh.ntiles) {
+                o.x = (t % sh.ntx) * kWgTX;
+                t /= sh.ntx;
+                o.y = (t % sh.nty) * TY;
+                t /= sh.nty;
+                o.z = (t % sh.ntz) * TZ;
+                o.w = t / sh.ntz;
+            }
+            org[tid] = o;
         }
         __syncthreads();
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sA[row][8 * kq]);
-        const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&sB[row][8 * kq]);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc, 0, 0, 0);
-        __syncthreads();  // the next step's stores reuse the tiles
-        // advance this lane's position by 32
-        int step = 32;
-        while (step > 0) {
-            const int room = c.OW - ox;
-            if (step < room) {
-                ox += step;
-                step = 0;
-            } else {
-                step -= room;
-                ox = 0;
-                if (++oy == c.OH) {
-                    oy = 0;
-                    if (++oz == c.OD) {
-                        oz = 0;
-                        ++bb;
-                    }
+        for (int it = tid; it < 2 * NX; it += 256) {
+            const int pl = it >> 1, ch = ci0 + 8 * (it & 1);
+            const int px = pl % HX - c.pw, py = (pl / HX) % HY - c.ph, pz = pl / (HX * HY) - c.pd;
+            uint4 r[kWgSubs], o[8];
+#pragma unroll
+            for (int s = 0; s < kWgSubs; ++s) {
+                const int4 g = org[s];
+                const int x = g.x + px, y = g.y + py, z = g.z + pz;
+                r[s] = make_uint4(0, 0, 0, 0);
+                if (ch < c.Cin && g.w >= 0 && x >= 0 && x < c.W && y >= 0 && y < c.H && z >= 0 &&
+                    z < c.D)
+                    r[s] = *reinterpret_cast<const uint4*>(
+                        X + ((((int64_t)g.w * c.D + z) * c.H + y) * c.W + x) * c.Cin + ch);
+            }
+            transpose8(r, o);
+            uint4* d = reinterpret_cast<uint4*>(sx + pl * kPl + (it & 1) * 8 * kWgSubs);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d[j] = o[j];
+        }
+        for (int it = tid; it < 2 * MC * NY; it += 256) {
+            const int q = it >> 1, pl = q % NY, ch = co0 + 16 * (q / NY) + 8 * (it & 1);
+            const int px = pl % kWgTX, py = (pl / kWgTX) % TY, pz = pl / (kWgTX * TY);
+            uint4 r[kWgSubs], o[8];
+#pragma unroll
+            for (int s = 0; s < kWgSubs; ++s) {
+                const int4 g = org[s];
+                const int x = g.x + px, y = g.y + py, z = g.z + pz;
+                r[s] = make_uint4(0, 0, 0, 0);
+                if (ch < c.Cout && g.w >= 0 && x < c.OW && y < c.OH && z < c.OD)
+                    r[s] = *reinterpret_cast<const uint4*>(
+                        dY + ((((int64_t)g.w * c.OD + z) * c.OH + y) * c.OW + x) * c.Cout + ch);
+            }
+            transpose8(r, o);
+            uint4* d = reinterpret_cast<uint4*>(sy + q * kPl + (it & 1) * 8 * kWgSubs);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) d[j] = o[j];
+        }
+        __syncthreads();
+        const uint16_t* xr = sx + ((z0 * HY + y0 + kq) * HX) * kPl + row * kWgSubs;
+        const uint16_t* yr = sy + ((m * TZ + z0) * TY + y0 + kq) * kWgTX * kPl + row * kWgSubs;
+        bf16x8 win[K][K][K];  // [dz][dy][x mod K]
+#pragma unroll
+        for (int x = 0; x < HX; ++x) {
+#pragma unroll
+            for (int dz = 0; dz < K; ++dz)
+#pragma unroll
+                for (int dy = 0; dy < K; ++dy)
+                    win[dz][dy][x % K] = load8(xr + ((dz * HY + dy) * HX + x) * kPl);
+            if (x < K - 1) continue;
+            const int xo = x - (K - 1);
+            const bf16x8 av = load8(yr + xo * kPl);
+            accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, ones, accb, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    av, win[t / (K * K)][(t / K) % K][(xo + t % K) % K], acc[t], 0, 0, 0);
+        }
+    }
+    if (PG > 1) {  // the place groups of an output tile, in order
+        float4* red = reinterpret_cast<float4*>(wg_lds);
+        for (int p = 1; p < PG; ++p) {
+            __syncthreads();
+            if (pg == p) {
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+                    red[(m * (T + 1) + t) * 64 + lane] =
+                        make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+                red[(m * (T + 1) + T) * 64 + lane] =
+                    make_float4(accb[0], accb[1], accb[2], accb[3]);
+            }
+            __syncthreads();
+            if (pg == 0) {
+#pragma unroll
+                for (int t = 0; t <= T; ++t) {
+                    const float4 v = red[(m * (T + 1) + t) * 64 + lane];
+                    f4& d = t < T ? acc[t < T ? t : 0] : accb;
+                    d += f4{v.x, v.y, v.z, v.w};
                 }
             }
         }
+        if (pg > 0) return;
     }
-    // D[m = co0 + 4kq + i][n = ci0 + row]
+    // D[co = 4 kq + i][ci = row] of every tap
+    const int tile = blockIdx.y * MC + m;
+    if (tile >= sh.ct) return;
+    float4* out = reinterpret_cast<float4*>(part) +
+                  (((int64_t)blockIdx.x * sh.ct + tile) * sh.it + blockIdx.z) * T * 64 + lane;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+        out[t * 64] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+    if (blockIdx.z == 0 && row == 0)
+        reinterpret_cast<float4*>(bpart)[((int64_t)blockIdx.x * sh.ct + tile) * 4 + kq] =
+            make_float4(accb[0], accb[1], accb[2], accb[3]);
+}
+
+// dW[co][tap][ci] and db[co] from the splits' partials.  Block (ct, it, tap): 64
+// lanes as the MFMA leaves the 16 x 16 tile, times 4 quarters of the splits, added
+// in order; the last ct blocks: the bias.
+__global__ __launch_bounds__(256) void k_conv_wgrad_sum(ConvDesc c, WgradShape sh, int T,
+                                                        const float* __restrict__ part,
+                                                        const float* __restrict__ bpart,
+                                                        float* __restrict__ dW,
+                                                        float* __restrict__ db) {
+    __shared__ float4 red[4][64];
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int nb = sh.ct * sh.it * T, chunk = (sh.ns + 3) / 4;
+    const int s0 = q * chunk, s1 = min(s0 + chunk, sh.ns);
+    const bool bias = (int)blockIdx.x >= nb;
+    const int tile = blockIdx.x - nb;
+    const float4* p = bias ? reinterpret_cast<const float4*>(bpart) + tile * 4 + (lane & 3)
+                           : reinterpret_cast<const float4*>(part) + (int64_t)blockIdx.x * 64 + lane;
+    const int64_t stride = bias ? sh.ct * 4 : (int64_t)nb * 64;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr int U = 8;
+    for (int s = s0; s < s1; s += U) {
+        float4 v[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) v[k] = p[(int64_t)min(s + k, s1 - 1) * stride];
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (s + k < s1) {
+                a.x += v[k].x;
+                a.y += v[k].y;
+                a.z += v[k].z;
+                a.w += v[k].w;
+            }
+    }
+    red[q][lane] = a;
+    __syncthreads();
+    if (q != 0) return;
+    a = red[0][lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+        const float4 v = red[k][lane];
+        a.x += v.x;
+        a.y += v.y;
+        a.z += v.z;
+        a.w += v.w;
+    }
+    const float e[4] = {a.x, a.y, a.z, a.w};
+    if (bias) {
+        if (lane < 4)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int co = tile * 16 + 4 * lane + i;
+                if (co < c.Cout && db) db[co] = e[i];
+            }
+        return;
+    }
+    const int t = blockIdx.x % T, it = (blockIdx.x / T) % sh.it, ct = blockIdx.x / (T * sh.it);
+    const int ci = it * 16 + (lane & 15);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int com = co0 + 4 * kq + i;
-        if (com < c.Cout)
-            part[(((int64_t)split * c.Cout + com) * T + tap) * c.Cin32 + ci0 + row] = acc[i];
+        const int co = ct * 16 + 4 * (lane >> 4) + i;
+        if (co < c.Cout && ci < c.Cin) dW[((int64_t)co * T + t) * c.Cin + ci] = e[i];
     }
 }
 
-// dW = sum over splits (fixed order); db[co] = sum_p dY[p][co] (one block per co).
-__global__ __launch_bounds__(256) void k_conv_bwd_w_reduce(int n, int nsplit,
-                                                           const float* __restrict__ part,
-                                                           float* __restrict__ dW) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int k = 0; k < nsplit; ++k) s += part[(int64_t)k * n + i];
-    dW[i] = s;
+// Output tiles a workgroup: 4 of 16 channels from Cout = 64 on, 2 from 32 on, else
+// 1 with four place groups.  About 512 workgroups, at most one split a unit.
+static int wgrad_mc(int Cout) { return Cout >= 64 ? 4 : Cout >= 32 ? 2 : 1; }
+static WgradShape wgrad_shape(const ConvDesc& c) {
+    const int mc = wgrad_mc(c.Cout);
+    const int ty = mc == 1 ? 8 : 4, tz = mc == 4 ? 1 : 2;
+    WgradShape s;
+    s.ntx = (c.OW + kWgTX - 1) / kWgTX;
+    s.nty = (c.OH + ty - 1) / ty;
+    s.ntz = (c.OD + tz - 1) / tz;
+    s.ntiles = s.ntx * s.nty * s.ntz * c.B;
+    s.nunits = (s.ntiles + kWgSubs - 1) / kWgSubs;
+    s.ct = (c.Cout + 15) / 16;
+    s.it = (c.Cin + 15) / 16;
+    const int per = (s.ct + mc - 1) / mc * s.it;
+    s.ns = std::max(1, std::min(s.nunits, 512 / per));
+    return s;
+}
+size_t conv_bwd_w_floats(const ConvDesc& c) {
+    const WgradShape s = wgrad_shape(c);
+    return (size_t)s.ns * s.ct * (size_t)(s.it * c.kd * c.kh * c.kw * 256 + 16);
 }
 
-// db[co] = sum_p dY[p][co]: kBiasBlocks blocks sweep contiguous rows of dY
-// (coalesced), one partial per (block, co); a second kernel sums the
-// partials of each channel in block order.
-constexpr int kBiasBlocks = 256;
-__global__ __launch_bounds__(256) void k_bias_grad(int64_t P, int Cout,
-                                                   const uint16_t* __restrict__ dY,
-                                                   float* __restrict__ part) {
-    __shared__ float red[256];
-    const int rows = 256 / Cout;  // Cout divides 256 (8..128)
-    const int co = threadIdx.x % Cout, r = threadIdx.x / Cout;
-    const int64_t chunk = (P + gridDim.x - 1) / gridDim.x;
-    const int64_t p0 = blockIdx.x * chunk, p1 = p0 + chunk < P ? p0 + chunk : P;
-    float s = 0.f;
-    if (r < rows)
-        for (int64_t p = p0 + r; p < p1; p += rows) s += bf2f(dY[p * Cout + co]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < Cout) {
-        float t = 0.f;
-        for (int q = 0; q < rows; ++q) t += red[q * Cout + threadIdx.x];
-        part[(size_t)blockIdx.x * Cout + threadIdx.x] = t;
-    }
-}
-
-// One block per channel: thread b loads the partial of block b, then a fixed
-// reduction tree (deterministic).
-__global__ __launch_bounds__(kBiasBlocks) void k_bias_grad_finish(int Cout,
-                                                                  const float* __restrict__ part,
-                                                                  float* __restrict__ db) {
-    __shared__ float red[kBiasBlocks];
-    const int co = blockIdx.x;
-    red[threadIdx.x] = part[(size_t)threadIdx.x * Cout + co];
-    __syncthreads();
-    for (int w = kBiasBlocks / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) db[co] = red[0];
+template <int MC, int TY, int TZ, int K>
+static hipError_t launch_wgrad(const ConvDesc& c, const WgradShape& sh, const uint16_t* X,
+                               const uint16_t* dY, float* part, float* bpart, hipStream_t s) {
+    constexpr int HX = kWgTX + K - 1, HY = TY + K - 1, HZ = TZ + K - 1, T = K * K * K;
+    constexpr int stage = (HX * HY * HZ + MC * kWgTX * TY * TZ) * 256;
+    constexpr int sums = MC < 4 ? MC * (T + 1) * 64 * 16 : 0;
+    constexpr int lds = stage > sums ? stage : sums;
+    static_assert(lds <= 159 * 1024, "LDS of a CU");
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv_wgrad<MC, TY, TZ, K>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_conv_wgrad<MC, TY, TZ, K>), dim3(sh.ns, (sh.ct + MC - 1) / MC, sh.it),
+                       dim3(256), lds, s, c, sh, X, dY, part, bpart);
+    return hipGetLastError();
 }
 
 hipError_t launch_conv_bwd_w(const ConvDesc& c, const uint16_t* X, const uint16_t* dY,
-                             float* part, int nsplit, float* dW, float* db, hipStream_t s) {
-    const int T = c.kd * c.kh * c.kw;
-    dim3 grid(T * (c.Cin32 / 16), (c.Cout + 15) / 16, nsplit);
-    // TOHIP_CONV_BWDW=0 keeps the direct-gather kernel (measurement)
-    static const bool lds = [] {
-        const char* e = getenv("TOHIP_CONV_BWDW");
-        return !(e && atoi(e) == 0);
-    }();
-    const bool vec = lds && c.Cout % 8 == 0 && c.Cin % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
-                     reinterpret_cast<uintptr_t>(dY) % 16 == 0;
-    if (vec)
-        hipLaunchKernelGGL(k_conv_bwd_w_lds, grid, dim3(64), 0, s, c, X, dY, part, nsplit);
-    else
-        hipLaunchKernelGGL(k_conv_bwd_w, grid, dim3(64), 0, s, c, X, dY, part, nsplit);
-    const int n = c.Cout * T * c.Cin32;
-    hipLaunchKernelGGL(k_conv_bwd_w_reduce, dim3((n + 255) / 256), dim3(256), 0, s, n, nsplit,
-                       part, dW);
-    if (db) {
-        // the bias partials reuse the split partial buffer after the reduce above
-        if (256 % c.Cout != 0 || (int64_t)kBiasBlocks * c.Cout > (int64_t)nsplit * n)
-            return hipErrorInvalidValue;
-        const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
-        hipLaunchKernelGGL(k_bias_grad, dim3(kBiasBlocks), dim3(256), 0, s, P, c.Cout, dY, part);
-        hipLaunchKernelGGL(k_bias_grad_finish, dim3(c.Cout), dim3(kBiasBlocks), 0, s, c.Cout, part,
-                           db);
-    }
+                             float* part, float* dW, float* db, hipStream_t s) {
+    const int k = c.kd, mc = wgrad_mc(c.Cout), T = k * k * k;
+    if (c.kh != k || c.kw != k || k < 1 || k > 3 || c.Cin % 8 || c.Cout % 8 || 256 % c.Cout ||
+        reinterpret_cast<uintptr_t>(X) % 16 || reinterpret_cast<uintptr_t>(dY) % 16)
+        return hipErrorInvalidValue;
+    const WgradShape sh = wgrad_shape(c);
+    float* bpart = part + (size_t)sh.ns * sh.ct * sh.it * T * 256;
+    hipError_t e;
+#define TOHIP_WG(K)                                                                        \
+    (mc == 4 ? launch_wgrad<4, 4, 1, K>(c, sh, X, dY, part, bpart, s)                      \
+     : mc == 2 ? launch_wgrad<2, 4, 2, K>(c, sh, X, dY, part, bpart, s)                    \
+               : launch_wgrad<1, 8, 2, K>(c, sh, X, dY, part, bpart, s))
+    e = k == 3 ? TOHIP_WG(3) : k == 2 ? TOHIP_WG(2) : TOHIP_WG(1);
+#undef TOHIP_WG
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_conv_wgrad_sum, dim3(sh.ct * sh.it * T + sh.ct), dim3(256), 0, s, c, sh, T,
+                       part, bpart, dW, db);
     return hipGetLastError();
 }
 

@@ -381,24 +381,15 @@ int nn_forward(tohip_nn* nn, int B, bool train) {
     return 0;
 }
 
-int split_for(int64_t P) { return (int)std::max<int64_t>(1, std::min<int64_t>(64, P / 2048)); }
-
 // weight/bias gradient of layer li (input X, output gradient dZ)
 int nn_wgrad(tohip_nn* nn, int li, int level, int B, const uint16_t* X, const uint16_t* dZ) {
     NNLayer& l = nn->L[li];
-    ConvDesc c = conv_desc(nn, l, B, level, false);
-    const int64_t P = (int64_t)B * c.OD * c.OH * c.OW;
-    const int ns = split_for(P);
-    if ((size_t)ns * l.cout * l.T * l.cin32 > nn->part_cap) {
+    const ConvDesc c = conv_desc(nn, l, B, level, li == kNL - 1);
+    if (conv_bwd_w_floats(c) > nn->part_cap) {
         nn->err = "weight-gradient scratch too small";
         return TOHIP_ERR_STATE;
     }
-    // dW into a [cout][T][cin32] scratch, then compact into grads [cout][T][cin]
-    float* dw32 = nn->part + (size_t)ns * l.cout * l.T * l.cin32;
-    NCK(launch_conv_bwd_w(c, X, dZ, nn->part, ns, dw32, nn->grads + l.boff, nn->stream));
-    NCK(hipMemcpy2DAsync(nn->grads + l.woff, l.cin * sizeof(float), dw32, l.cin32 * sizeof(float),
-                         l.cin * sizeof(float), (size_t)l.cout * l.T, hipMemcpyDeviceToDevice,
-                         nn->stream));
+    NCK(launch_conv_bwd_w(c, X, dZ, nn->part, nn->grads + l.woff, nn->grads + l.boff, nn->stream));
     return 0;
 }
 
@@ -419,15 +410,7 @@ int nn_backward(tohip_nn* nn, int B) {
     uint16_t *g1 = nn->g1, *g2 = nn->g2;
     // output layer (identity activation)
     {
-        NNLayer& l = nn->L[14];
-        ConvDesc c = conv_desc(nn, l, B, 0, true);
-        const int64_t P = (int64_t)B * c.OD * c.OH * c.OW;
-        const int ns = split_for(P);
-        float* dw32 = nn->part + (size_t)ns * l.cout * l.T * l.cin32;
-        NCK(launch_conv_bwd_w(c, nn->d0, nn->dout, nn->part, ns, dw32, nn->grads + l.boff, s));
-        NCK(hipMemcpy2DAsync(nn->grads + l.woff, l.cin * sizeof(float), dw32,
-                             l.cin32 * sizeof(float), l.cin * sizeof(float), (size_t)l.cout * l.T,
-                             hipMemcpyDeviceToDevice, s));
+        if ((rc = nn_wgrad(nn, 14, 0, B, nn->d0, nn->dout))) return rc;
         if ((rc = nn_dgrad(nn, 14, 0, B, nn->dout, g1))) return rc;  // d d0
     }
     // a (silu) layer: dZ = silu'(Z) dA into gZ, wgrad, dgrad into gX
@@ -546,7 +529,8 @@ int nn_create_impl(tohip_nn* nn, const int64_t* nels, int maxB, int maxS, uint64
         if ((rc = nalloc(nn, &l.wf, (size_t)l.cout * l.T * l.cin32)) ||
             (rc = nalloc(nn, &l.wt, (size_t)l.cin * l.T * l.cout32)))
             return rc;
-        pc = std::max(pc, (size_t)65 * l.cout * l.T * l.cin32);
+        const int level = i < 2 || i > 11 ? 0 : i < 4 || i > 9 ? 1 : i < 6 || i > 7 ? 2 : 3;
+        pc = std::max(pc, conv_bwd_w_floats(conv_desc(nn, l, maxB, level, i == kNL - 1)));
     }
     nn->part_cap = pc;
     if ((rc = nalloc(nn, &nn->part, pc + 1))) return rc;
@@ -943,11 +927,9 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
     for (int64_t i = 0; i < ny; ++i) hdy[i] = bf(dy[i]);
     uint16_t *dX = nullptr, *dDY = nullptr, *dZ = nullptr, *dZg = nullptr, *dXb = nullptr;
     float *dW = nullptr, *dB = nullptr, *dYf = nullptr, *dDX = nullptr, *part = nullptr,
-          *dw32 = nullptr, *dbb = nullptr;
+          *dbb = nullptr;
     hipStream_t s = nullptr;
     int rc = 0;
-    const int ns = 4;
-    const size_t partn = (size_t)ns * cout * l.T * l.cin32;
     auto fail = [&](hipError_t e) {
         g_nn_error = std::string("tohip_nn_conv_check: ") + hipGetErrorString(e);
         rc = TOHIP_ERR_HIP;
@@ -970,11 +952,10 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
     QCK(hipMalloc((void**)&dB, cout * 4));
     QCK(hipMalloc((void**)&dYf, ny * 4));
     QCK(hipMalloc((void**)&dDX, nx * 4));
-    QCK(hipMalloc((void**)&part, (partn + (size_t)cout * l.T * l.cin32) * 4));
+    QCK(hipMalloc((void**)&part, conv_bwd_w_floats(c) * 4));
     QCK(hipMalloc((void**)&dbb, cout * 4));
     QCK(hipMalloc((void**)&l.wf, (size_t)cout * l.T * l.cin32 * 2));
     QCK(hipMalloc((void**)&l.wt, (size_t)cin * l.T * l.cout32 * 2));
-    dw32 = part + partn;
     QCK(hipMemcpyAsync(dX, hx.data(), nx * 2, hipMemcpyHostToDevice, s));
     QCK(hipMemcpyAsync(dDY, hdy.data(), ny * 2, hipMemcpyHostToDevice, s));
     QCK(hipMemcpyAsync(dW, w, nw * 4, hipMemcpyHostToDevice, s));
@@ -996,9 +977,7 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
         bd.OW = c.W;
         QCK(launch_conv_fwd(bd, dZg, l.wt, nullptr, nullptr, nullptr, dDX, s));
     }
-    QCK(launch_conv_bwd_w(c, dX, dZg, part, ns, dw32, dbb, s));
-    QCK(hipMemcpy2DAsync(dW, cin * sizeof(float), dw32, l.cin32 * sizeof(float),
-                         cin * sizeof(float), (size_t)cout * l.T, hipMemcpyDeviceToDevice, s));
+    QCK(launch_conv_bwd_w(c, dX, dZg, part, dW, dbb, s));
     QCK(hipMemcpyAsync(y, dYf, ny * 4, hipMemcpyDeviceToHost, s));
     QCK(hipMemcpyAsync(dx, dDX, nx * 4, hipMemcpyDeviceToHost, s));
     QCK(hipMemcpyAsync(dw, dW, nw * 4, hipMemcpyDeviceToHost, s));

@@ -23,8 +23,11 @@ struct ConvDesc {
 hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t* W,
                            const float* bias, uint16_t* Y, uint16_t* Z, float* Yf,
                            hipStream_t s);
+// dW [Cout][taps][Cin], db [Cout]; part: conv_bwd_w_floats(c) floats of scratch,
+// 16-byte aligned like X and dY.  Cubic kernels up to 3, Cout a divisor of 256.
+size_t conv_bwd_w_floats(const ConvDesc& c);
 hipError_t launch_conv_bwd_w(const ConvDesc& c, const uint16_t* X, const uint16_t* dY,
-                             float* part, int nsplit, float* dW, float* db, hipStream_t s);
+                             float* part, float* dW, float* db, hipStream_t s);
 hipError_t launch_weights_to_bf16(int Cout, int T, int Cin, int Cin32, int Cout32,
                                   const float* w, uint16_t* wf, uint16_t* wt, hipStream_t s);
 hipError_t launch_silu_bwd(int64_t n, const uint16_t* dA, const uint16_t* Z, uint16_t* dZ,
