@@ -15,7 +15,12 @@ CASES = [
     (1, (5, 6, 10), 24, 32, 3, 1, 1), (9, (2, 2, 3), 32, 64, 3, 1, 1), (1, (4, 4, 8), 192, 64, 3, 1, 1),
     (2, (1, 5, 11), 64, 128, 3, 1, 0), (1, (3, 4, 9), 128, 128, 3, 1, 1), (2, (4, 7, 12), 16, 8, 2, 1, 0),
     (1, (5, 8, 16), 8, 16, 2, 0, 0), (1, (3, 4, 5), 40, 32, 1, 0, 1), (2, (4, 4, 4), 16, 64, 2, 1, 1),
-    (1, (6, 5, 8), 16, 16, 3, 2, 0), (1, (5, 6, 9), 16, 32, 3, 0, 1), (2, (9, 10, 33), 32, 16, 3, 1, 1),
+    # enough positions for the LDS-tile forward, ragged, every tile depth and channel
+    # tile count (the input gradient's are the input channels')
+    (1, (17, 30, 70), 16, 16, 3, 1, 1), (2, (33, 31, 65), 8, 16, 3, 1, 1),
+    (1, (31, 33, 39), 48, 32, 3, 1, 1), (1, (16, 25, 90), 96, 32, 3, 1, 0),
+    (1, (14, 31, 40), 192, 64, 3, 1, 1), (1, (13, 20, 50), 24, 128, 3, 1, 1),
+    (2, (17, 32, 63), 16, 8, 2, 1, 0), (1, (6, 5, 8), 16, 16, 3, 2, 0), (1, (5, 6, 9), 16, 32, 3, 0, 1), (2, (9, 10, 33), 32, 16, 3, 1, 1),
 ]
 
 

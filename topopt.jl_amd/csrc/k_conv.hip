@@ -53,15 +53,13 @@ __device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z));
 // (8, 16, 48 channels) is packed across taps instead of padded to 32
 // channels with zeros (the weights' zero padding past Cin is never read).
 //
-// Block = 4 waves, each wave 16 output positions x 16*NSUB output channels.
-// KS = 1: the waves own 4 consecutive position tiles and walk all K-steps.
-// KS = 4: the waves share one position tile and take every 4th K-step; the
-//   4 partial accumulators are summed through LDS in wave order.  For the
-//   coarse layers, where P / 64 blocks cannot fill the chip, this gives 4x
-//   the blocks and a quarter of the dependent load -> MFMA chain per wave.
+// Block = 4 waves on 16 output positions x 16*NSUB output channels.  The waves
+// share the position tile and take every 4th K-step; the 4 partial accumulators are
+// summed through LDS in wave order: for the coarse layers, where tiles of more
+// positions cannot fill the chip, many blocks and a short load -> MFMA chain.
 constexpr int kConvMaxTaps = 32;
 
-template <int NSUB, int KS>
+template <int NSUB>
 __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __restrict__ X,
                                                   const uint16_t* __restrict__ W,
                                                   const float* __restrict__ bias,
@@ -69,7 +67,8 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
                                                   uint16_t* __restrict__ Z,
                                                   float* __restrict__ Yf) {
     __shared__ int4 taps[kConvMaxTaps];  // dz, dy, dx, element offset of the tap
-    __shared__ f4 red[KS > 1 ? KS - 1 : 1][NSUB][64];
+    constexpr int KS = 4;
+    __shared__ f4 red[KS - 1][NSUB][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane & 15, kq = lane >> 4;
     const int T = c.kd * c.kh * c.kw;
@@ -80,7 +79,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
     }
     __syncthreads();
     const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
-    const int64_t p0 = (KS == 1 ? (int64_t)blockIdx.x * 4 + wave : (int64_t)blockIdx.x) * 16;
+    const int64_t p0 = (int64_t)blockIdx.x * 16;
     const int co0 = blockIdx.y * 16 * NSUB;
 
     // this lane's A row: output position p0 + row
@@ -113,7 +112,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
     // U K-steps per iteration: all their loads are issued before the MFMAs,
     // so a wave keeps U gathers in flight (steps past S load zeros).
     constexpr int U = NSUB >= 4 ? 2 : 4;
-    for (int s0 = (KS == 1 ? 0 : wave); s0 < S; s0 += U * KS) {
+    for (int s0 = wave; s0 < S; s0 += U * KS) {
         bf16x8 a[U], bv[U][NSUB];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -142,17 +141,15 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
             for (int j = 0; j < NSUB; ++j)
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bv[u][j], acc[j], 0, 0, 0);
     }
-    if (KS > 1) {
-        if (wave > 0)
+    if (wave > 0)
 #pragma unroll
-            for (int j = 0; j < NSUB; ++j) red[wave - 1][j][lane] = acc[j];
-        __syncthreads();
-        if (wave > 0) return;
+        for (int j = 0; j < NSUB; ++j) red[wave - 1][j][lane] = acc[j];
+    __syncthreads();
+    if (wave > 0) return;
 #pragma unroll
-        for (int w = 0; w < KS - 1; ++w)
+    for (int w = 0; w < KS - 1; ++w)
 #pragma unroll
-            for (int j = 0; j < NSUB; ++j) acc[j] += red[w][j][lane];
-    }
+        for (int j = 0; j < NSUB; ++j) acc[j] += red[w][j][lane];
 #pragma unroll
     for (int j = 0; j < NSUB; ++j) {
         const int co = co0 + 16 * j + row;
@@ -174,41 +171,248 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
     }
 }
 
-// Launch shape: KS = 1 with the widest channel tile while P / 64 blocks fill
-// the chip; otherwise KS = 4 and the narrowest tile that still gives about
-// 4 blocks per CU.  TOHIP_CONV_KS = 1 / 4 forces the split (measurement).
+// ---- forward from LDS tiles ----
+// A workgroup stages its output tile's input places with their halo, 32 (16, 8)
+// channels at a time, and reads every tap's operand from there; the kernel above
+// gathers each of the K^3 taps from memory again.  An M tile is 8 x by 2 y
+// positions of one z; the workgroup's 4 waves own MT each (8 x 4 x 2, 8 x 8 x 2 or
+// 8 x 8 x 4 outputs) and all of NT x 16 output channels: per K-step of 32 MT LDS
+// reads and NT weight loads (16 bytes a lane, the next step's in flight) for MT x NT
+// MFMAs.  A K-step is one tap's 32 channels, two taps' 16 or four taps' 8.  Places
+// are padded by 16 bytes (80, 48; 16 for 8 channels), which spreads 8 x 2 places
+// over the banks and keeps the taps' offsets immediate.  Outputs of neighbouring
+// lanes are paired into 4-byte stores.
+template <int CK>
+constexpr int kFwdPitch = CK == 8 ? 16 : CK * 2 + 16;  // bytes of a staged place
+
+template <int K, int NT, int MT>
+__global__ __launch_bounds__(256) void k_conv_tile(ConvDesc c, int ntx, int nty, int ntz,
+                                                   const uint16_t* __restrict__ X,
+                                                   const uint16_t* __restrict__ W,
+                                                   const float* __restrict__ bias,
+                                                   uint16_t* __restrict__ Y,
+                                                   uint16_t* __restrict__ Z,
+                                                   float* __restrict__ Yf) {
+    constexpr int BY = MT == 1 ? 4 : 8, BZ = MT == 4 ? 4 : 2, T = K * K * K;
+    constexpr int HX = 8 + K - 1, HY = BY + K - 1, HZ = BZ + K - 1, NPL = HX * HY * HZ;
+    __shared__ __align__(16) char lds[NPL * kFwdPitch<32>];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 15, kq = lane >> 4;
+    int t = xcd_remap(blockIdx.x, gridDim.x);
+    const int x0 = (t % ntx) * 8;
+    t /= ntx;
+    const int y0 = (t % nty) * BY;
+    t /= nty;
+    const int z0 = (t % ntz) * BZ, bt = t / ntz;
+    const int co0 = blockIdx.y * 16 * NT;
+    // the wave's M tiles: z and the first y pair
+    const int wz = MT == 4 ? wave : wave & 1, wy = MT == 4 ? 0 : (wave >> 1) * 2 * MT;
+    const int place0 = (wz * HY + wy + (row >> 3)) * HX + (row & 7);
+
+    f4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+    const uint16_t* wrow[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+        wrow[n] = W + (int64_t)min(co0 + 16 * n + row, c.Cout - 1) * T * c.Cin32;
+
+    auto chunk = [&](auto ck, int c0) {
+        constexpr int CK = decltype(ck)::value, G = CK / 8, P = kFwdPitch<CK>;
+        constexpr int TS = 4 / G, S = (T + TS - 1) / TS;  // taps a K-step, K-steps
+        // this lane's share of K-step s: tap TS s + kq / G, channels 8 (kq % G) ..
+        const int lt = kq / G, lc = 8 * (kq % G);
+        auto weights = [&](int tap, bf16x8 (&b)[NT]) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                b[n] = load8(wrow[n] + min(tap, T - 1) * c.Cin32 + c0 + lc);
+        };
+        bf16x8 bn[CK == 32 ? K : 1][NT];
+#pragma unroll
+        for (int q = 0; q < (CK == 32 ? K : 1); ++q) weights(q + lt, bn[q]);
+        __syncthreads();  // the previous chunk's reads
+        for (int it = tid; it < NPL * G; it += 256) {
+            const int pl = it / G, ch = c0 + 8 * (it % G);
+            const int x = x0 - c.pw + pl % HX, y = y0 - c.ph + (pl / HX) % HY,
+                      z = z0 - c.pd + pl / (HX * HY);
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (x >= 0 && x < c.W && y >= 0 && y < c.H && z >= 0 && z < c.D)
+                v = *reinterpret_cast<const uint4*>(
+                    X + ((((int64_t)bt * c.D + z) * c.H + y) * c.W + x) * c.Cin + ch);
+            *reinterpret_cast<uint4*>(lds + pl * P + 16 * (it % G)) = v;
+        }
+        __syncthreads();
+        const char* base = lds + place0 * P + 2 * lc;
+        if constexpr (CK == 32) {
+            // a K-step is a tap; a row of K taps at a time, the next row's weights in
+            // flight (unrolled whole, every weight is loaded first: 256 registers)
+#pragma unroll 1
+            for (int r = 0; r < K * K; ++r) {
+                bf16x8 bw[K][NT];
+#pragma unroll
+                for (int q = 0; q < K; ++q)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) bw[q][n] = bn[q][n];
+                if (r + 1 < K * K)
+#pragma unroll
+                    for (int q = 0; q < K; ++q) weights((r + 1) * K + q, bn[q]);
+                const char* at = base + ((r / K) * HY + r % K) * HX * P;
+#pragma unroll
+                for (int q = 0; q < K; ++q)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        const bf16x8 av =
+                            *reinterpret_cast<const bf16x8*>(at + (2 * m * HX + q) * P);
+#pragma unroll
+                        for (int n = 0; n < NT; ++n)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                av, bw[q][n], acc[m][n], 0, 0, 0);
+                    }
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                bf16x8 bw[NT];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) bw[n] = bn[0][n];
+                if (s + 1 < S) weights(TS * (s + 1) + lt, bn[0]);
+                int off = 0;
+#pragma unroll
+                for (int q = 0; q < TS; ++q) {
+                    const int tap = TS * s + q < T ? TS * s + q : 0;
+                    const int o = P * (((tap / (K * K)) * HY + (tap / K) % K) * HX + tap % K);
+                    off = q == 0 || lt >= q ? o : off;
+                }
+                const bool on = TS * s + lt < T;  // taps past the kernel: 0
+                const bf16x8 zero = {};
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    bf16x8 av = *reinterpret_cast<const bf16x8*>(base + off + 2 * m * HX * P);
+                    if (TS * s + TS > T && !on) av = zero;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[n], acc[m][n],
+                                                                            0, 0, 0);
+                }
+            }
+        }
+    };
+    int c0 = 0;
+    for (; c0 + 32 <= c.Cin; c0 += 32) chunk(std::integral_constant<int, 32>{}, c0);
+    if (c0 + 16 <= c.Cin) {
+        chunk(std::integral_constant<int, 16>{}, c0);
+        c0 += 16;
+    }
+    if (c0 < c.Cin) chunk(std::integral_constant<int, 8>{}, c0);
+
+    // D[m = 4 kq + i][n = row]
+    const int z = z0 + wz;
+    if (z >= c.OD) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int y = y0 + wy + 2 * m + (kq >> 1);
+        if (y >= c.OH) continue;
+        const int64_t line = (((int64_t)bt * c.OD + z) * c.OH + y) * c.OW;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int co = co0 + 16 * n + row;
+            const float bb = bias && co < c.Cout ? bias[co] : 0.f;
+            float zv[4], yv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                zv[i] = acc[m][n][i] + bb;
+                yv[i] = c.act == 1 ? silu(zv[i]) : zv[i];
+            }
+            if (Yf)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int x = x0 + 4 * (kq & 1) + i;
+                    if (x < c.OW && co < c.out_cvalid) Yf[(line + x) * c.out_cvalid + co] = yv[i];
+                }
+            // an even lane stores position i of both channels, its odd neighbour
+            // position i + 1
+            const bool odd = row & 1;
+            auto store = [&](const float (&v)[4], uint16_t* out, int stride, int off) {
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const uint32_t own = f2bf(odd ? v[i + 1] : v[i]),
+                                   send = f2bf(odd ? v[i] : v[i + 1]);
+                    const uint32_t got = __builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xf, 0xf,
+                                                                     true);  // of lane ^ 1
+                    const int x = x0 + 4 * (kq & 1) + i + (odd ? 1 : 0);
+                    if (x < c.OW && co < c.Cout)
+                        *reinterpret_cast<uint32_t*>(out + (line + x) * stride + off + (co & ~1)) =
+                            odd ? got | own << 16 : own | got << 16;
+                }
+            };
+            if (!Yf) store(yv, Y, c.out_cstride, c.out_coff);
+            if (Z) store(zv, Z, c.Cout, 0);
+        }
+    }
+}
+
+template <int K, int NT, int MT>
+static hipError_t launch_conv_tile(const ConvDesc& c, const uint16_t* X, const uint16_t* W,
+                                   const float* bias, uint16_t* Y, uint16_t* Z, float* Yf,
+                                   hipStream_t s) {
+    constexpr int BY = MT == 1 ? 4 : 8, BZ = MT == 4 ? 4 : 2;
+    const int ntx = (c.OW + 7) / 8, nty = (c.OH + BY - 1) / BY, ntz = (c.OD + BZ - 1) / BZ;
+    hipLaunchKernelGGL((k_conv_tile<K, NT, MT>),
+                       dim3((unsigned)(ntx * nty * ntz * c.B), (c.Cout + 16 * NT - 1) / (16 * NT)),
+                       dim3(256), 0, s, c, ntx, nty, ntz, X, W, bias, Y, Z, Yf);
+    return hipGetLastError();
+}
+
+// The LDS-tile kernel with the largest tile that still gives a workgroup per CU;
+// with the smallest, fewer output channels a workgroup until there are two per CU
+// (all of an output's channels from one staging otherwise).  The split kernel (16
+// positions a workgroup, the K-steps over its waves) below half a workgroup per CU,
+// and for kernels and channel counts that the network has not.  MI355X, all forward
+// and input-gradient convolutions of 12 training steps at 64x32x32, batch 8, and 6
+// predictions at 120x40x40: 9.7 ms; with at least 256 / 512 / 1024 workgroups for the
+// large tiles and all channels a workgroup 10.3 / 10.4 / 11.3; a workgroup per CU for
+// the channels 10.0; never the split kernel 9.9; gathers from memory alone 15.6.
 hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t* W,
                            const float* bias, uint16_t* Y, uint16_t* Z, float* Yf,
                            hipStream_t s) {
-    static const int forced = [] {
-        const char* e = getenv("TOHIP_CONV_KS");
-        return e ? atoi(e) : 0;
-    }();
     const int T = c.kd * c.kh * c.kw;
     if (T > kConvMaxTaps || c.Cin % 8 != 0 || c.Cin32 % 32 != 0 || c.Cin > c.Cin32)
         return hipErrorInvalidValue;
-    const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
-    const int nsub_wide = c.Cout >= 64 ? 4 : c.Cout >= 32 ? 2 : 1;
-    const int64_t wide_blocks = (P + 63) / 64 * ((c.Cout + 16 * nsub_wide - 1) / (16 * nsub_wide));
-    const int ks = (forced == 1 || forced == 4) ? forced : wide_blocks >= 1024 ? 1 : 4;
-    int nsub = nsub_wide;
-    if (ks == 4)
-        while (nsub > 1 && (P + 15) / 16 * ((c.Cout + 16 * nsub - 1) / (16 * nsub)) < 1024)
-            nsub /= 2;
-    const unsigned gx = (unsigned)(ks == 1 ? (P + 63) / 64 : (P + 15) / 16);
-    const unsigned gy = (unsigned)((c.Cout + 16 * nsub - 1) / (16 * nsub));
-#define TOHIP_CONV(NS, K)                                                                     \
-    hipLaunchKernelGGL((k_conv_fwd<NS, K>), dim3(gx, gy), dim3(256), 0, s, c, X, W, bias, Y, Z, \
-                       Yf)
-    if (ks == 1) {
-        if (nsub == 4) TOHIP_CONV(4, 1);
-        else if (nsub == 2) TOHIP_CONV(2, 1);
-        else TOHIP_CONV(1, 1);
-    } else {
-        if (nsub == 4) TOHIP_CONV(4, 4);
-        else if (nsub == 2) TOHIP_CONV(2, 4);
-        else TOHIP_CONV(1, 4);
+    const bool cube3 = c.kd == 3 && c.kh == 3 && c.kw == 3,
+               cube2 = c.kd == 2 && c.kh == 2 && c.kw == 2;
+    const int ct = (c.Cout + 15) / 16;
+    int nt = ct % 4 == 0 ? 4 : ct % 3 == 0 ? 3 : ct % 2 == 0 ? 2 : 1;
+    if (c.Cout % 8 == 0 && (cube3 || (cube2 && ct == 1)) &&
+        (Yf || (c.out_cstride % 2 == 0 && c.out_coff % 2 == 0))) {
+        auto blocks = [&](int by, int bz) {
+            return (int64_t)c.B * ((c.OW + 7) / 8) * ((c.OH + by - 1) / by) *
+                   ((c.OD + bz - 1) / bz) * (ct / nt);
+        };
+        int mt = blocks(8, 4) >= 256 ? 4 : blocks(8, 2) >= 256 ? 2 : 1;
+        while (mt == 1 && nt > 1 && blocks(4, 2) < 512) nt = nt == 4 ? 2 : 1;
+        if (mt == 1 && blocks(4, 2) < 128) mt = 0;
+#define TOHIP_CT(K, N)                                                                         \
+    (mt == 4   ? launch_conv_tile<K, N, 4>(c, X, W, bias, Y, Z, Yf, s)                         \
+     : mt == 2 ? launch_conv_tile<K, N, 2>(c, X, W, bias, Y, Z, Yf, s)                         \
+               : launch_conv_tile<K, N, 1>(c, X, W, bias, Y, Z, Yf, s))
+        if (mt) {
+            if (cube2) return TOHIP_CT(2, 1);
+            return nt == 4 ? TOHIP_CT(3, 4) : nt == 3 ? TOHIP_CT(3, 3) : nt == 2 ? TOHIP_CT(3, 2)
+                                                                                 : TOHIP_CT(3, 1);
+        }
+#undef TOHIP_CT
     }
+    const int64_t P = (int64_t)c.B * c.OD * c.OH * c.OW;
+    int nsub = c.Cout >= 64 ? 4 : c.Cout >= 32 ? 2 : 1;
+    while (nsub > 1 && (P + 15) / 16 * ((c.Cout + 16 * nsub - 1) / (16 * nsub)) < 1024) nsub /= 2;
+    const dim3 grid((unsigned)((P + 15) / 16), (unsigned)((c.Cout + 16 * nsub - 1) / (16 * nsub)));
+#define TOHIP_CONV(NS)                                                                            \
+    hipLaunchKernelGGL((k_conv_fwd<NS>), grid, dim3(256), 0, s, c, X, W, bias, Y, Z, Yf)
+    if (nsub == 4) TOHIP_CONV(4);
+    else if (nsub == 2) TOHIP_CONV(2);
+    else TOHIP_CONV(1);
 #undef TOHIP_CONV
     return hipGetLastError();
 }
