@@ -231,37 +231,51 @@ int dalloc(tohip_ctx* ctx, T** p, size_t n) {
     return 0;
 }
 
-// caller order <-> internal order
-void to_internal(const tohip_ctx* ctx, const double* in, std::vector<double>& out) {
-    const int64_t n = ctx->g.ndof;
-    out.resize(n);
-    if (ctx->perm.empty())
-        std::memcpy(out.data(), in, n * sizeof(double));
-    else
-        for (int64_t i = 0; i < n; ++i) out[i] = in[ctx->perm[i]];
-}
-void to_caller(const tohip_ctx* ctx, const std::vector<double>& in, double* out) {
-    const int64_t n = ctx->g.ndof;
-    if (ctx->perm.empty())
-        std::memcpy(out, in.data(), n * sizeof(double));
-    else
-        for (int64_t i = 0; i < n; ++i) out[ctx->perm[i]] = in[i];
+bool all_finite(const double* v, int64_t n) {
+    for (int64_t i = 0; i < n; ++i)
+        if (!std::isfinite(v[i])) return false;
+    return true;
 }
 
-int upload_dofs(tohip_ctx* ctx, const double* host, double* dev) {
-    std::vector<double> tmp;
-    to_internal(ctx, host, tmp);
-    CK(hipMemcpyAsync(dev, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice,
-                      ctx->stream));
+// A host vector of DOFs into q64 (solve scratch) as it is, in the caller's order;
+// with `check`, *finite says whether every value is.  The host array has been read
+// on return.
+int stage_dofs(tohip_ctx* ctx, const double* host, bool check, bool* finite) {
+    const int64_t n = ctx->g.ndof;
+    if (check && n <= kHostCheckMax && !(*finite = all_finite(host, n))) return 0;
+    CK(hipMemcpyAsync(ctx->q64, host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    if (check && n > kHostCheckMax) {
+        long double ss;
+        double bad;
+        CK(values_check(n, ctx->q64, ctx->partials, &ss, &bad, ctx->stream));
+        *finite = bad == 0.0;
+        return 0;
+    }
     CK(hipStreamSynchronize(ctx->stream));
     return 0;
 }
+
+// The staged vector in the library's order, prescribed DOFs zeroed when `masked`.
+int unstage_dofs(tohip_ctx* ctx, double* dev, bool masked = false) {
+    CK(launch_order_gather(ctx->g.ndof, ctx->g.dim, ctx->perm, masked ? ctx->fixmask : nullptr,
+                           ctx->q64, dev, ctx->stream));
+    return 0;
+}
+
+int upload_dofs(tohip_ctx* ctx, const double* host, double* dev) {
+    if (int rc = stage_dofs(ctx, host, false, nullptr)) return rc;
+    return unstage_dofs(ctx, dev);
+}
+
+// dev must not be q64.
 int download_dofs(tohip_ctx* ctx, const double* dev, double* host) {
-    std::vector<double> tmp(ctx->g.ndof);
-    CK(hipMemcpyAsync(tmp.data(), dev, tmp.size() * sizeof(double), hipMemcpyDeviceToHost,
+    if (ctx->perm) {
+        CK(launch_order_scatter(ctx->g.ndof, ctx->perm, dev, ctx->q64, ctx->stream));
+        dev = ctx->q64;
+    }
+    CK(hipMemcpyAsync(host, dev, ctx->g.ndof * sizeof(double), hipMemcpyDeviceToHost,
                       ctx->stream));
     CK(hipStreamSynchronize(ctx->stream));
-    to_caller(ctx, tmp, host);
     return 0;
 }
 int upload_cells(tohip_ctx* ctx, const double* host, double* dev) {
@@ -1243,10 +1257,21 @@ double host_norm(const double* v, int64_t n) {
     return (double)std::sqrt(s);
 }
 
-bool all_finite(const double* v, int64_t n) {
-    for (int64_t i = 0; i < n; ++i)
-        if (!std::isfinite(v[i])) return false;
-    return true;
+// ||f|| of the load on the device; on the host where the squares leave the range.
+int load_norm(tohip_ctx* ctx, double* norm) {
+    long double ss;
+    double bad;
+    CK(values_check(ctx->g.ndof, ctx->f, ctx->partials, &ss, &bad, ctx->stream));
+    if (ss > 1e-250 && ss < 1e250) {
+        *norm = (double)std::sqrt(ss);
+        return 0;
+    }
+    std::vector<double> fh(ctx->g.ndof);
+    CK(hipMemcpyAsync(fh.data(), ctx->f, fh.size() * sizeof(double), hipMemcpyDeviceToHost,
+                      ctx->stream));
+    CK(hipStreamSynchronize(ctx->stream));
+    *norm = host_norm(fh.data(), (int64_t)fh.size());
+    return 0;
 }
 
 void free_ctx(tohip_ctx* ctx) {
@@ -1274,7 +1299,8 @@ void free_ctx(tohip_ctx* ctx) {
                     (void*)ctx->mma_x1, (void*)ctx->mma_x2, (void*)ctx->mma_st,
                     (void*)ctx->mg_M, (void*)ctx->r32b, (void*)ctx->mg_wd, (void*)ctx->r64b,
                     (void*)ctx->pcg1_part[0], (void*)ctx->pcg1_part[1], (void*)ctx->pcg1_st,
-                    (void*)ctx->csr_part, (void*)ctx->csr_st, (void*)ctx->mg_sweepM})
+                    (void*)ctx->csr_part, (void*)ctx->csr_st, (void*)ctx->mg_sweepM,
+                    (void*)ctx->perm})
         if (b) hipFree(b);
     if (ctx->h_pcg1) hipHostFree(ctx->h_pcg1);
     if (ctx->h_mma) hipHostFree(ctx->h_mma);
@@ -1368,8 +1394,9 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
 
     // DOF permutation from Metadata.node_dofs
     std::vector<uint8_t> nodemask(g.nnodes, 0);
+    std::vector<int> perm;  // internal -> caller
     if (node_dofs) {
-        ctx->perm.assign(g.ndof, -1);
+        perm.assign(g.ndof, -1);
         std::vector<uint8_t> seen(g.ndof, 0);
         for (int64_t n = 0; n < g.nnodes; ++n)
             for (int d = 0; d < dim; ++d) {
@@ -1379,12 +1406,12 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
                     return TOHIP_ERR_ARG;
                 }
                 seen[v] = 1;
-                ctx->perm[dim * n + d] = v;
+                perm[dim * n + d] = (int)v;
             }
     }
     for (int64_t n = 0; n < g.nnodes; ++n)
         for (int d = 0; d < dim; ++d) {
-            const int64_t c = node_dofs ? ctx->perm[dim * n + d] : dim * n + d;
+            const int64_t c = node_dofs ? perm[dim * n + d] : dim * n + d;
             if (fixed_mask[c]) nodemask[n] |= (uint8_t)(1u << d);
         }
 
@@ -1409,7 +1436,7 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
         (rc = dalloc(ctx, &ctx->xd, nC)) || (rc = dalloc(ctx, &ctx->xnew, nC)) ||
         (rc = dalloc(ctx, &ctx->dc, nC)) || (rc = dalloc(ctx, &ctx->ce, nC)) ||
         (rc = dalloc(ctx, &ctx->grad, nC)) || (rc = dalloc(ctx, &ctx->cellbuf, nC)) ||
-        (rc = dalloc(ctx, &ctx->oc, 1)))
+        (rc = dalloc(ctx, &ctx->oc, 1)) || (node_dofs && (rc = dalloc(ctx, &ctx->perm, nD))))
         return rc;
     CK(hipHostMalloc((void**)&ctx->h_sc, sizeof(PcgScalars), hipHostMallocDefault));
     CK(hipHostMalloc((void**)&ctx->h_scal, 8 * sizeof(double), hipHostMallocDefault));
@@ -1419,6 +1446,9 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
     *ctx->h_ecrit = EnergyCrit{};
     CK(hipMemcpyAsync(ctx->fixmask, nodemask.data(), g.nnodes, hipMemcpyHostToDevice,
                       ctx->stream));
+    if (node_dofs)
+        CK(hipMemcpyAsync(ctx->perm, perm.data(), nD * sizeof(int), hipMemcpyHostToDevice,
+                          ctx->stream));
     CK(hipStreamSynchronize(ctx->stream));
     ctx->nodemask = std::move(nodemask);
     CK(hipMemsetAsync(ctx->sc64, 0, sizeof(PcgScalars), ctx->stream));
@@ -1778,18 +1808,18 @@ int tohip_csr_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, d
         return TOHIP_ERR_ARG;
     }
     const int64_t n = ctx->g.ndof;
-    if (!all_finite(f, n) || (!initially_zero && !all_finite(u, n))) {
+    // apply!(K, f, ch) with zero prescribed values: f = 0 on the prescribed DOFs
+    bool finite = true;
+    if (int rc = stage_dofs(ctx, f, true, &finite)) return rc;
+    if (finite) {
+        if (int rc = unstage_dofs(ctx, ctx->b64, true)) return rc;
+        if (!initially_zero)
+            if (int rc = stage_dofs(ctx, u, true, &finite)) return rc;
+    }
+    if (!finite) {
         ctx->err = "tohip_csr_solve: non-finite load or initial guess";
         return TOHIP_ERR_ARG;
     }
-    // apply!(K, f, ch) with zero prescribed values: f = 0 on the prescribed DOFs
-    std::vector<double> fz(f, f + n);
-    const int dim = ctx->g.dim;
-    for (int64_t node = 0; node < ctx->g.nnodes; ++node)
-        for (int d = 0; d < dim; ++d)
-            if ((ctx->nodemask[node] >> d) & 1)
-                fz[ctx->perm.empty() ? dim * node + d : ctx->perm[dim * node + d]] = 0.0;
-    if (int rc = upload_dofs(ctx, fz.data(), ctx->b64)) return rc;
     if (int rc = csr_assemble(ctx, safe ? 1 : 0, jacobi ? 1 : 0)) return rc;
     const int nb = csr_pcg1_blocks(ctx->g);
     if (!ctx->csr_part)
@@ -1810,7 +1840,7 @@ int tohip_csr_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, d
     if (initially_zero) {
         CK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
     } else {
-        if (int rc = upload_dofs(ctx, u, ctx->u)) return rc;
+        if (int rc = unstage_dofs(ctx, ctx->u)) return rc;  // staged above
         CK(launch_csr_spmv(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->u, ctx->t64, ctx->stream));
     }
     CK(launch_pcg1_start(n, ctx->b64, initially_zero ? nullptr : ctx->t64, ctx->csr_dinv, ctx->r64,
@@ -1831,22 +1861,19 @@ int tohip_csr_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, d
 
 int tohip_mg_apply(tohip_ctx* ctx, const double* r, double* z) {
     if (!ctx || !r || !z) return TOHIP_ERR_ARG;
-    if (!all_finite(r, ctx->g.ndof)) {
+    bool finite = true;
+    if (int rc = stage_dofs(ctx, r, true, &finite)) return rc;
+    if (!finite) {
         ctx->err = "tohip_mg_apply: non-finite input";
         return TOHIP_ERR_ARG;
     }
+    if (int rc = unstage_dofs(ctx, ctx->r64)) return rc;
     if (int rc = mg_setup(ctx)) return rc;
-    if (int rc = upload_dofs(ctx, r, ctx->r64)) return rc;
     CK(launch_f64_to_f32(ctx->g.ndof, ctx->r64, ctx->b32, ctx->stream));
     if (int rc = mg_join(ctx)) return rc;
     CK(launch_vcycle(ctx, ctx->b32, nullptr, nullptr, nullptr, nullptr, ctx->mg_sweepM_now));
-    std::vector<float> zf(ctx->g.ndof);
-    CK(hipMemcpyAsync(zf.data(), ctx->mg[0].rz, zf.size() * sizeof(float),
-                      hipMemcpyDeviceToHost, ctx->stream));
-    CK(hipStreamSynchronize(ctx->stream));
-    std::vector<double> zd(zf.begin(), zf.end());
-    to_caller(ctx, zd, z);
-    return 0;
+    CK(launch_f32_to_f64(ctx->g.ndof, ctx->mg[0].rz, ctx->t64, ctx->stream));
+    return download_dofs(ctx, ctx->t64, z);
 }
 
 int tohip_mg_weights(tohip_ctx* ctx, double* omega, double* lambda_est, int max_levels,
@@ -1875,8 +1902,16 @@ int tohip_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, doubl
         ctx->err = "tohip_solve: bad tolerance, maxiter or precision";
         return TOHIP_ERR_ARG;
     }
-    if ((f && !all_finite(f, ctx->g.ndof)) ||
-        (u && !initially_zero && !all_finite(u, ctx->g.ndof))) {
+    const bool guess = u && !initially_zero;
+    bool finite = true;
+    if (f) {
+        if (int rc = stage_dofs(ctx, f, true, &finite)) return rc;
+        if (finite)
+            if (int rc = unstage_dofs(ctx, ctx->b64)) return rc;
+    }
+    if (finite && guess)
+        if (int rc = stage_dofs(ctx, u, true, &finite)) return rc;  // stays staged until below
+    if (!finite) {
         ctx->err = "tohip_solve: non-finite load or initial guess";
         return TOHIP_ERR_ARG;
     }
@@ -1888,14 +1923,11 @@ int tohip_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, doubl
         ctx->err = "tohip_solve: u = NULL with initially_zero = 0 needs a previous solve";
         return TOHIP_ERR_STATE;
     }
-    if (f) {
-        if (int rc = upload_dofs(ctx, f, ctx->b64)) return rc;
-    } else {
+    if (!f)
         CK(hipMemcpyAsync(ctx->b64, ctx->f, ctx->g.ndof * sizeof(double),
                           hipMemcpyDeviceToDevice, ctx->stream));
-    }
-    if (!initially_zero && u)
-        if (int rc = upload_dofs(ctx, u, ctx->u)) return rc;
+    if (guess)
+        if (int rc = unstage_dofs(ctx, ctx->u)) return rc;
     int rc = solve_mode(ctx, precision, abstol, reltol, maxiter, initially_zero != 0, 0.0,
                         reltol, iters_out, resid_out);
     if (rc < 0) return rc;
@@ -2055,19 +2087,14 @@ int tohip_oc_update(tohip_ctx* ctx, const double* x, const double* dc, double vo
 
 int tohip_set_load(tohip_ctx* ctx, const double* f) {
     if (!ctx || !f) return TOHIP_ERR_ARG;
-    if (!all_finite(f, ctx->g.ndof)) {
+    bool finite = true;
+    if (int rc = stage_dofs(ctx, f, true, &finite)) return rc;
+    if (!finite) {
         ctx->err = "tohip_set_load: non-finite load";
         return TOHIP_ERR_ARG;
     }
-    std::vector<double> tmp;
-    to_internal(ctx, f, tmp);
-    const int dim = ctx->g.dim;
-    for (int64_t n = 0; n < ctx->g.nnodes; ++n)  // apply_zero! on the prescribed DOFs
-        for (int d = 0; d < dim; ++d)
-            if ((ctx->nodemask[n] >> d) & 1) tmp[dim * n + d] = 0.0;
-    CK(hipMemcpyAsync(ctx->f, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice,
-                      ctx->stream));
-    CK(hipStreamSynchronize(ctx->stream));
+    // apply_zero! on the prescribed DOFs
+    if (int rc = unstage_dofs(ctx, ctx->f, true)) return rc;
     ctx->have_load = true;
     return 0;
 }
@@ -2162,11 +2189,8 @@ int simp_run_impl(tohip_ctx* ctx, const tohip_simp_opts* o, const tohip_mma_opts
     }
     if (int rc = build_filter(ctx, o->rmin)) return rc;
     const int64_t nD = ctx->g.ndof, nC = ctx->g.ncells;
-    std::vector<double> fh(nD);
-    CK(hipMemcpyAsync(fh.data(), ctx->f, nD * sizeof(double), hipMemcpyDeviceToHost,
-                      ctx->stream));
-    CK(hipStreamSynchronize(ctx->stream));
-    const double fnorm = host_norm(fh.data(), nD);
+    double fnorm;
+    if (int rc = load_norm(ctx, &fnorm)) return rc;
     if (!(fnorm > 0)) {
         ctx->err = "tohip_simp_run: the load vector is zero (tohip_set_load)";
         return TOHIP_ERR_STATE;
@@ -2313,10 +2337,8 @@ int tohip_beso_run(tohip_ctx* ctx, const tohip_beso_opts* o, const double* x0,
         return TOHIP_ERR_ARG;
     }
     if (int rc = build_filter(ctx, o->rmin)) return rc;
-    std::vector<double> fh(nD);
-    CK(hipMemcpyAsync(fh.data(), ctx->f, nD * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CK(hipStreamSynchronize(ctx->stream));
-    const double fnorm = host_norm(fh.data(), nD);
+    double fnorm;
+    if (int rc = load_norm(ctx, &fnorm)) return rc;
     if (!(fnorm > 0)) {
         ctx->err = "tohip_beso_run: the load vector is zero (tohip_set_load)";
         return TOHIP_ERR_STATE;

@@ -38,7 +38,7 @@ struct tohip_ctx {
     double meandiag = 0;
     tohip::ElemOp<double> op64{};
     tohip::ElemOp<float> op32{};
-    std::vector<int64_t> perm;  // internal DOF -> caller DOF (0-based); empty = identity
+    int* perm = nullptr;  // internal DOF -> caller DOF (0-based), device; null = identity
     std::vector<uint8_t> fixed_internal;
     hipStream_t stream = nullptr;
     std::string err;

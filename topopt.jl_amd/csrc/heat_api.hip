@@ -26,7 +26,8 @@ struct tohip_heat {
     int pbi = 1;
     double meandiag = 0.0;
     bool inhom = false;              // some prescribed temperature is nonzero
-    std::vector<int64_t> dof_node;   // caller DOF (0-based) -> node id
+    int* node_dof = nullptr;         // node id -> caller DOF (0-based), device
+    double* check = nullptr;         // partials of a vector's check
     hipStream_t stream = nullptr;
     uint8_t* fixmask = nullptr;
     double *fixv = nullptr, *x = nullptr, *E = nullptr, *dinv = nullptr;
@@ -102,28 +103,38 @@ int halloc(tohip_heat* ctx, T** p, size_t n) {
     return 0;
 }
 
-int upload_nodes(tohip_heat* ctx, const double* host, double* dev) {
-    const int64_t n = ctx->g.nnodes;
-    std::vector<double> tmp(n);
-    for (int64_t d = 0; d < n; ++d) tmp[ctx->dof_node[d]] = host[d];
-    HCK(hipMemcpyAsync(dev, tmp.data(), n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    HCK(hipStreamSynchronize(ctx->stream));
-    return 0;
-}
-
-int download_nodes(tohip_heat* ctx, const double* dev, double* host) {
-    const int64_t n = ctx->g.nnodes;
-    std::vector<double> tmp(n);
-    HCK(hipMemcpyAsync(tmp.data(), dev, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HCK(hipStreamSynchronize(ctx->stream));
-    for (int64_t d = 0; d < n; ++d) host[d] = tmp[ctx->dof_node[d]];
-    return 0;
-}
-
 bool finite_all(const double* v, int64_t n) {
     for (int64_t i = 0; i < n; ++i)
         if (!std::isfinite(v[i])) return false;
     return true;
+}
+
+// A host vector into r[1] (solve scratch) in the caller's order, then into the
+// node order; with `finite`, whether every value is (dev is left alone if not).
+// The host array has been read on return.
+int upload_nodes(tohip_heat* ctx, const double* host, double* dev, bool* finite = nullptr) {
+    const int64_t n = ctx->g.nnodes;
+    if (finite && n <= kHostCheckMax && !(*finite = finite_all(host, n))) return 0;
+    HCK(hipMemcpyAsync(ctx->r[1], host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    if (finite && n > kHostCheckMax) {
+        long double ss;
+        double bad;
+        HCK(values_check(n, ctx->r[1], ctx->check, &ss, &bad, ctx->stream));
+        if (!(*finite = bad == 0.0)) return 0;
+    } else {
+        HCK(hipStreamSynchronize(ctx->stream));
+    }
+    HCK(launch_order_gather(n, 1, ctx->node_dof, nullptr, ctx->r[1], dev, ctx->stream));
+    return 0;
+}
+
+// dev must not be r[1].
+int download_nodes(tohip_heat* ctx, const double* dev, double* host) {
+    const int64_t n = ctx->g.nnodes;
+    HCK(launch_order_scatter(n, ctx->node_dof, dev, ctx->r[1], ctx->stream));
+    HCK(hipMemcpyAsync(host, ctx->r[1], n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    HCK(hipStreamSynchronize(ctx->stream));
+    return 0;
 }
 
 int refresh(tohip_heat* ctx) {
@@ -202,7 +213,7 @@ void free_heat(tohip_heat* ctx) {
     void* bufs[] = {ctx->fixmask, ctx->fixv, ctx->x,    ctx->E,    ctx->dinv,    ctx->u,
                     ctx->r[0],    ctx->r[1], ctx->p[0], ctx->p[1], ctx->q[0],    ctx->q[1],
                     ctx->b,       ctx->t,    ctx->lam,  ctx->cell, ctx->grad,    ctx->part[0],
-                    ctx->part[1], ctx->st};
+                    ctx->part[1], ctx->st,   ctx->node_dof, ctx->check};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (ctx->h_st) hipHostFree(ctx->h_st);
@@ -256,19 +267,21 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
     ctx->pen = Penalty{TOHIP_PEN_POWER, TOHIP_PROJ_NONE, penalty_p, 0.0};
     // node_dofs: the 1 x nnodes Metadata.node_dofs (1-based), a permutation
     const int64_t n = g.nnodes;
-    ctx->dof_node.assign(n, -1);
+    std::vector<int> node_dof(n);
+    std::vector<uint8_t> seen(n, 0);
     for (int64_t node = 0; node < n; ++node) {
         const int64_t d = node_dofs[node] - 1;
-        if (d < 0 || d >= n || ctx->dof_node[d] >= 0) {
+        if (d < 0 || d >= n || seen[d]) {
             ctx->err = "node_dofs is not a permutation of 1..nnodes";
             return TOHIP_ERR_ARG;
         }
-        ctx->dof_node[d] = node;
+        seen[d] = 1;
+        node_dof[node] = (int)d;
     }
     std::vector<uint8_t> mask(n, 0);
     std::vector<double> vals(n, 0.0);
-    for (int64_t d = 0; d < n; ++d) {
-        const int64_t node = ctx->dof_node[d];
+    for (int64_t node = 0; node < n; ++node) {
+        const int64_t d = node_dof[node];
         mask[node] = fixed_mask[d] ? 1 : 0;
         if (mask[node] && fixed_values) {
             if (!std::isfinite(fixed_values[d])) {
@@ -292,9 +305,12 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
         (rc = halloc(ctx, &ctx->grad, g.ncells)) || 
         (rc = halloc(ctx, &ctx->part[0], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
         (rc = halloc(ctx, &ctx->part[1], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
-        (rc = halloc(ctx, &ctx->st, 2)))
+        (rc = halloc(ctx, &ctx->st, 2)) || (rc = halloc(ctx, &ctx->node_dof, n)) ||
+        (rc = halloc(ctx, &ctx->check, 3 * kVecBlocks)))
         return rc;
     HCK(hipHostMalloc((void**)&ctx->h_st, sizeof(Pcg1State), hipHostMallocDefault));
+    HCK(hipMemcpyAsync(ctx->node_dof, node_dof.data(), n * sizeof(int), hipMemcpyHostToDevice,
+                       ctx->stream));
     HCK(hipMemcpyAsync(ctx->fixmask, mask.data(), n, hipMemcpyHostToDevice, ctx->stream));
     HCK(hipMemcpyAsync(ctx->fixv, vals.data(), n * sizeof(double), hipMemcpyHostToDevice,
                        ctx->stream));
@@ -380,19 +396,20 @@ int tohip_heat_solve(tohip_heat* ctx, const double* rhs, double* T, double absto
         return TOHIP_ERR_ARG;
     }
     const int64_t n = ctx->g.nnodes;
-    if (!finite_all(rhs, n) || (!initially_zero && !finite_all(T, n))) {
+    bool finite = true;
+    if (int rc = upload_nodes(ctx, rhs, ctx->q[0], &finite)) return rc;
+    if (finite && !initially_zero)
+        if (int rc = upload_nodes(ctx, T, ctx->u, &finite)) return rc;
+    if (!finite) {
         ctx->err = "tohip_heat_solve: non-finite right-hand side or initial guess";
         return TOHIP_ERR_ARG;
     }
-    if (int rc = upload_nodes(ctx, rhs, ctx->q[0])) return rc;
     const bool lift = apply_dirichlet && ctx->inhom;
     if (lift)
         HCK(launch_heat_matvec(ctx->g, ctx->modes, ctx->fixv, ctx->fixmask, ctx->E, ctx->meandiag,
                                ctx->t, 2, ctx->stream));
     HCK(launch_heat_rhs(n, ctx->q[0], lift ? ctx->t : nullptr, ctx->fixmask, ctx->fixv,
                         ctx->meandiag, lift ? 1 : 0, ctx->b, ctx->stream));
-    if (!initially_zero)
-        if (int rc = upload_nodes(ctx, T, ctx->u)) return rc;
     const int rc = solve(ctx, initially_zero != 0, abstol, reltol, maxiter, iters_out, resid_out);
     if (rc < 0) return rc;
     if (int rc2 = download_nodes(ctx, ctx->u, T)) return rc2;

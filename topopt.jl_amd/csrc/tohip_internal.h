@@ -242,6 +242,22 @@ hipError_t launch_csr_build(const Grid& g, const double* Ke, const double* E,
 hipError_t launch_csr_dinv(const Grid& g, const double* diag, const uint8_t* fixmask,
                            const double* mdiag_sum, int jacobi, int safe, double* dinv,
                            hipStream_t s);
+// DOF vectors between the caller's order and the library's (k_order.hip):
+// out[i] = in[perm[i]] (perm null: in[i]), 0 where mask (null: none) has DOF i of
+// dim per node prescribed; out[perm[i]] = in[i].
+hipError_t launch_order_gather(int64_t n, int dim, const int* perm, const uint8_t* mask,
+                               const double* in, double* out, hipStream_t s);
+hipError_t launch_order_scatter(int64_t n, const int* perm, const double* in, double* out,
+                                hipStream_t s);
+// Sum of squares and count of non-finite values of a device vector, on the host
+// after the stream has drained; kVecBlocks partials of 3.
+hipError_t values_check(int64_t n, const double* x, double* partials, long double* sumsq,
+                        double* bad, hipStream_t s);
+// Vectors up to this length are checked on the host, longer ones on the device.  A
+// load set from the host takes 40 us against 63 us for 8,450 values, 83 against 82
+// for 132,098, 6.3 ms against 3.5 for 12.8 million (MI355X).
+constexpr int64_t kHostCheckMax = 1 << 16;
+
 // Sum-reductions finished by a one-block kernel: out[v] = sum_b part[b*nv+v].
 hipError_t launch_reduce(const double* partials, int nb, int nv, double* out, hipStream_t s);
 
