@@ -637,6 +637,12 @@ hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, d
     for (int l = 0; l < L; ++l) {
         const float* b = l == 0 ? r : M[l].b;
         const MgLevelView F = M[l].view(), C = M[l + 1].view();
+        if (!mg_use_zm(F.g) && mg_fuse_restrict(F.g)) {
+            if ((e = launch_mg_pre_restrict(F, M[l].omega, b, C, M[l].x, M[l + 1].b, sc,
+                                            l == 0 ? upd : nullptr, s)) != hipSuccess)
+                return e;
+            continue;
+        }
         if ((e = launch_mg_smooth(l == 0 && upd ? 3 : 0, F, M[l].omega, b, nullptr, nullptr,
                                   nullptr, M[l].x, M[l].rz, md, sc, nullptr, s,
                                   l == 0 ? upd : nullptr)) != hipSuccess)

@@ -33,6 +33,8 @@
 //   The weight w is read from device memory (wdev) when it is given, so that
 //   the captured iteration graphs follow the weight the estimate sets.
 //   k_mg_restrict: b_{l+1} = P^T r_l, one thread per coarse node.
+//   k_mg_pre_restrict: MODE 0 and the restriction in one launch (2D and small
+//     levels).
 //   k_mg_coarse:   all coarsest sweeps in one workgroup, everything in LDS.
 //   k_mg_coarsen:  coarse moduli.
 // Every kernel returns at once when the PCG state says the solve is done, so
@@ -419,6 +421,214 @@ __global__ __launch_bounds__(NT, MODE == 3 ? 4 : 1) void k_mg_smooth(
     }
 }
 
+// Pre-smoothing and restriction in one launch: x = w D^-1 b on the fine level,
+// b_c = P^T (b - K x) on the coarse one.  A workgroup owns TX x TY x TZ fine nodes
+// (even origins) and the coarse nodes among them.  It forms the residual on its
+// nodes and one layer below, all that its coarse nodes reach, so the residual
+// never leaves LDS.  Staged: two layers below the tile, one above.
+// The small levels are bound by latency: a launch (2.5 us), one round trip, three
+// barriers.  A whole V-cycle in it against the two launches a level, MI355X: 2D
+// 640x320 (5 levels) 63.3 -> 45.5 us, 60x20x20 30.7 -> 25.3 us, 30x10x10 15.7 ->
+// 13.1 us.
+// UPD: b is r - alpha q of the PCG update in flight (see MgFusedUpdate), formed on
+// every staged node by the same FMA, and stored with x += alpha p by the owner.
+// The terms and their order are those of k_mg_smooth<0> and k_mg_restrict.
+template <int DIM, bool UPD, bool CUBE, int TX, int TY, int TZ, int NT>
+__global__ __launch_bounds__(NT) void k_mg_pre_restrict(
+    Grid g, ElemOp<float> op, const float* __restrict__ E, const uint8_t* __restrict__ fixmask,
+    const float* __restrict__ dinv, float w, const float* __restrict__ b, Grid gc,
+    const uint8_t* __restrict__ cmask, float* __restrict__ xout, float* __restrict__ bc,
+    const PcgScalars* sc, MgFusedUpdate upd, const float* __restrict__ wdev) {
+    constexpr int NC = 1 << DIM;
+    constexpr int RX = TX + 1, RY = TY + 1, RZ = DIM == 3 ? TZ + 1 : 1;  // residual nodes
+    constexpr int EX = TX + 2, EY = TY + 2, EZ = DIM == 3 ? TZ + 2 : 1;
+    constexpr int IX = TX + 3, IY = TY + 3, IZ = DIM == 3 ? TZ + 3 : 1;
+    constexpr int HX = TX / 2, HY = TY / 2, HZ = DIM == 3 ? TZ / 2 : 1;
+    constexpr int NR = RX * RY * RZ, NEL = EX * EY * EZ, NIN = IX * IY * IZ, NCO = HX * HY * HZ;
+    static_assert(TX % 2 == 0 && TY % 2 == 0 && (DIM == 2 || TZ % 2 == 0), "even tiles");
+
+    __shared__ float xs[DIM][NIN];
+    __shared__ float rs[DIM][NR];  // b, then the residual
+    __shared__ float res[DIM * NC][NEL];
+    __shared__ float eloc[NEL];
+    __shared__ uint8_t ms[NR];
+    __shared__ double red[NT / 64];
+
+    if (mg_done(sc)) return;
+    if (wdev) w = *wdev;
+    const int tid = threadIdx.x;
+    const int ntx = (g.NX + TX - 1) / TX, nty = (g.NY + TY - 1) / TY;
+    const int t = xcd_remap(blockIdx.x, gridDim.x);
+    const int i0 = (t % ntx) * TX, j0 = ((t / ntx) % nty) * TY;
+    const int k0 = DIM == 3 ? (t / (ntx * nty)) * TZ : 0;
+    const long long uk = UPD ? upd.sc->k_cur : 0;
+    const float* __restrict__ up = UPD ? ((uk & 1) ? upd.p1 : upd.p0) : nullptr;
+
+    // ---- every global load first, at clamped indices (see k_mg_smooth) ----
+    constexpr int SE = (NEL + NT - 1) / NT, SI = (NIN + NT - 1) / NT;
+    float er[SE];
+#pragma unroll
+    for (int q = 0; q < SE; ++q) {
+        const int el = min(tid + q * NT, NEL - 1);
+        const int ei = el % EX, ej = (el / EX) % EY, ek = DIM == 3 ? el / (EX * EY) : 0;
+        const int gi = min(max(i0 - 2 + ei, 0), g.nx - 1), gj = min(max(j0 - 2 + ej, 0), g.ny - 1);
+        const int gk = DIM == 3 ? min(max(k0 - 2 + ek, 0), g.nz - 1) : 0;
+        er[q] = E[gi + g.nx * (gj + g.ny * gk)];
+    }
+    uint8_t mr[SI];
+    float ra[SI][DIM], rb[SI][DIM];
+    constexpr int SU = UPD ? SI : 1;
+    float rq[SU][DIM], rx[SU][DIM], rp[SU][DIM];
+#pragma unroll
+    for (int q = 0; q < SI; ++q) {
+        const int nl = min(tid + q * NT, NIN - 1);
+        const int li = nl % IX, lj = (nl / IX) % IY, lk = DIM == 3 ? nl / (IX * IY) : 0;
+        const int gi = min(max(i0 - 2 + li, 0), g.NX - 1), gj = min(max(j0 - 2 + lj, 0), g.NY - 1);
+        const int gk = DIM == 3 ? min(max(k0 - 2 + lk, 0), g.NZ - 1) : 0;
+        const int n = gi + g.NX * (gj + g.NY * gk);
+        mr[q] = fixmask[n];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            ra[q][d] = dinv[DIM * n + d];
+            rb[q][d] = b[DIM * n + d];
+            if (UPD) rq[UPD ? q : 0][d] = upd.q[DIM * n + d];
+        }
+        if (UPD) {
+            const bool own = li >= 2 && li < TX + 2 && lj >= 2 && lj < TY + 2 &&
+                             (DIM == 2 || (lk >= 2 && lk < TZ + 2));
+            if (own)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    rx[UPD ? q : 0][d] = upd.x[DIM * n + d];
+                    rp[UPD ? q : 0][d] = up[DIM * n + d];
+                }
+        }
+    }
+    double ualpha = 0.0;
+    float ua = 0.f;
+    if (UPD) {
+        const double pq = reduce_partials(upd.partA, upd.nbA, 1, 0, red);
+        if (!(pq > 0.0 && pq < INFINITY)) {  // before x or r change
+            if (blockIdx.x == 0 && tid == 0) {
+                upd.sc->err = kPcgErrIndefinite;
+                upd.sc->done = 1;
+            }
+            return;
+        }
+        ualpha = upd.sc->rho_cur / pq;
+        ua = (float)ualpha;
+    }
+#pragma unroll
+    for (int q = 0; q < SE; ++q) {
+        const int el = tid + q * NT;
+        if (el >= NEL) break;
+        const int ei = el % EX, ej = (el / EX) % EY, ek = DIM == 3 ? el / (EX * EY) : 0;
+        const int gi = i0 - 2 + ei, gj = j0 - 2 + ej, gk = DIM == 3 ? k0 - 2 + ek : 0;
+        const bool in = gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny && gk >= 0 && gk < g.nz;
+        eloc[el] = in ? er[q] : 0.f;
+    }
+    // ---- x = w D^-1 b on the staged nodes (prescribed and outside: 0) ----
+#pragma unroll
+    for (int q = 0; q < SI; ++q) {
+        const int nl = tid + q * NT;
+        if (nl >= NIN) break;
+        const int li = nl % IX, lj = (nl / IX) % IY, lk = DIM == 3 ? nl / (IX * IY) : 0;
+        const int gi = i0 - 2 + li, gj = j0 - 2 + lj, gk = DIM == 3 ? k0 - 2 + lk : 0;
+        const bool in = gi >= 0 && gi < g.NX && gj >= 0 && gj < g.NY && gk >= 0 && gk < g.NZ;
+        const bool inr = li >= 1 && li < TX + 2 && lj >= 1 && lj < TY + 2 &&
+                         (DIM == 2 || (lk >= 1 && lk < TZ + 2));
+        const bool own = in && inr && li >= 2 && lj >= 2 && (DIM == 2 || lk >= 2);
+        const int n = gi + g.NX * (gj + g.NY * gk);
+        const int r = (li - 1) + RX * ((lj - 1) + RY * (DIM == 3 ? lk - 1 : 0));
+        // a node outside the mesh or prescribed has no residual
+        const uint8_t m = in ? mr[q] : (uint8_t)((1 << DIM) - 1);
+        if (inr) ms[r] = m;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const float bv = UPD ? __fmaf_rn(-ua, rq[UPD ? q : 0][d], rb[q][d]) : rb[q][d];
+            const float v = (m >> d) & 1 ? 0.f : w * ra[q][d] * bv;
+            xs[d][nl] = v;
+            if (inr) rs[d][r] = bv;
+            if (own) {
+                xout[DIM * n + d] = v;
+                if (UPD) {
+                    upd.rnew[DIM * n + d] = bv;
+                    upd.x[DIM * n + d] =
+                        __fmaf_rn(ua, rp[UPD ? q : 0][d], rx[UPD ? q : 0][d]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int el = tid; el < NEL; el += NT) {
+        const int ei = el % EX, ej = (el / EX) % EY, ek = DIM == 3 ? el / (EX * EY) : 0;
+        const float Ee = eloc[el];
+        if (Ee != 0.f) {
+            float xe[DIM][NC], ye[DIM][NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int nl = (ei + (c & 1)) +
+                               IX * ((ej + ((c >> 1) & 1)) + IY * (ek + ((c >> 2) & 1)));
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) xe[d][c] = xs[d][nl];
+            }
+            elem_apply<float, DIM, CUBE>(op, xe, ye);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) res[c * DIM + d][el] = Ee * ye[d][c];
+        } else {
+#pragma unroll
+            for (int j = 0; j < DIM * NC; ++j) res[j][el] = 0.f;
+        }
+    }
+    __syncthreads();
+    for (int r = tid; r < NR; r += NT) {
+        const int ri = r % RX, rj = (r / RX) % RY, rk = DIM == 3 ? r / (RX * RY) : 0;
+        float s[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) s[d] = 0.f;
+#pragma unroll
+        for (int c = NC - 1; c >= 0; --c) {
+            const int e = (ri + 1 - (c & 1)) +
+                          EX * ((rj + 1 - ((c >> 1) & 1)) +
+                                EY * (DIM == 3 ? rk + 1 - ((c >> 2) & 1) : 0));
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) s[d] += res[c * DIM + d][e];
+        }
+        const uint8_t m = ms[r];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) rs[d][r] = (m >> d) & 1 ? 0.f : rs[d][r] - s[d];
+    }
+    __syncthreads();
+    for (int o = tid; o < NCO * DIM; o += NT) {
+        const int d = o / NCO, h = o % NCO;
+        const int hi = h % HX, hj = (h / HX) % HY, hk = DIM == 3 ? h / (HX * HY) : 0;
+        const int I = i0 / 2 + hi, J = j0 / 2 + hj, K = DIM == 3 ? k0 / 2 + hk : 0;
+        if (I >= gc.NX || J >= gc.NY || K >= gc.NZ) continue;
+        float s = 0.f;
+#pragma unroll
+        for (int c = 0; c < (DIM == 3 ? 3 : 1); ++c) {
+            const float wc = (DIM == 3 && c != 1) ? 0.5f : 1.f;
+#pragma unroll
+            for (int bb = 0; bb < 3; ++bb) {
+                const float wb = wc * (bb != 1 ? 0.5f : 1.f);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    const float wt = wb * (a != 1 ? 0.5f : 1.f);
+                    s += wt * rs[d][(2 * hi + a) + RX * ((2 * hj + bb) + RY * (2 * hk + c))];
+                }
+            }
+        }
+        const int N = I + gc.NX * (J + gc.NY * K);
+        bc[DIM * N + d] = ((cmask[N] >> d) & 1) ? 0.f : s;
+    }
+    if (UPD && blockIdx.x == 0 && tid == 0) {
+        upd.sc->iter = uk;
+        upd.sc->alpha = ualpha;
+    }
+}
+
 // b_c = P^T r (masked at prescribed coarse DOFs): coarse node (I, J, K) sums
 // the fine nodes (2I + a, 2J + b, 2K + c), a, b, c in {-1, 0, 1}, with weight
 // prod (1 - |a|/2), in ascending (c, b, a) order.  The stencil is fully
@@ -729,7 +939,9 @@ hipError_t launch_mg_smooth(int mode, const MgLevelView& L, float w, const float
                             float* xout, float* rout, double meandiag, const PcgScalars* sc,
                             double* part, hipStream_t s, const MgFusedUpdate* upd,
                             const float* aux) {
-    if (mode == 3 && (!upd || !upd->sc || upd->sc != sc)) return hipErrorInvalidValue;
+    // (mode 3 in 2D: launch_mg_pre_restrict)
+    if (mode == 3 && (L.g.dim != 3 || !upd || !upd->sc || upd->sc != sc))
+        return hipErrorInvalidValue;
     if (mode == 5 && (!aux || !xprev || !part)) return hipErrorInvalidValue;
     if ((mode == 0 || mode == 1) && mg_use_zm(L.g)) {
         // z-marching columns; the post-smoothing forms x' = xprev + P xc while
@@ -763,14 +975,16 @@ hipError_t launch_mg_smooth(int mode, const MgLevelView& L, float w, const float
         TOHIP_MGS(D, 0, CB, X, Y, Z, N);         \
     else if (mode == 1)                          \
         TOHIP_MGS(D, 1, CB, X, Y, Z, N);         \
-    else if (mode == 3)                          \
-        TOHIP_MGS(D, 3, CB, X, Y, Z, N);         \
     else if (mode == 5)                          \
         TOHIP_MGS(D, 5, CB, X, Y, Z, N);         \
     else                                         \
         TOHIP_MGS(D, 2, CB, X, Y, Z, N)
 #define TOHIP_MG3(X, Y, Z, N)              \
-    if (L.op.is_cube)                      \
+    if (mode == 3 && L.op.is_cube)         \
+        TOHIP_MGS(3, 3, true, X, Y, Z, N); \
+    else if (mode == 3)                    \
+        TOHIP_MGS(3, 3, false, X, Y, Z, N); \
+    else if (L.op.is_cube)                 \
         TOHIP_MGM(3, true, X, Y, Z, N);    \
     else                                   \
         TOHIP_MGM(3, false, X, Y, Z, N)
@@ -826,6 +1040,44 @@ hipError_t launch_mg_restrict(const MgLevelView& F, const MgLevelView& C, const 
                            sc);
     return hipGetLastError();
 }
+
+hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
+                                  const MgLevelView& C, float* xout, float* bc,
+                                  const PcgScalars* sc, const MgFusedUpdate* upd, hipStream_t s) {
+    if (C.g.nx * 2 != L.g.nx || C.g.ny * 2 != L.g.ny || (L.g.dim == 3 && C.g.nz * 2 != L.g.nz) ||
+        (upd && (!upd->sc || upd->sc != sc)))
+        return hipErrorInvalidValue;
+    const MgFusedUpdate u = upd ? *upd : MgFusedUpdate{};
+    // 2D: 16x8 (128 threads), 16x16, 32x8 measured 2-5 % slower at 640x320; 3D: 8x4x2,
+    // 8x4x4, 8x8x4 within 3 % of 4x4x4 at 60x20x20
+#define TOHIP_PR(D, U, CB, X, Y, Z, N)                                                          \
+    hipLaunchKernelGGL((k_mg_pre_restrict<D, U, CB, X, Y, Z, N>),                                \
+                       dim3((unsigned)(((L.g.NX + X - 1) / X) * ((L.g.NY + Y - 1) / Y) *         \
+                                       ((L.g.NZ + Z - 1) / Z))),                                 \
+                       dim3(N), 0, s, L.g, L.op, L.E32, L.fixmask, L.dinv, w, b, C.g, C.fixmask, \
+                       xout, bc, sc, u, L.wdev)
+#define TOHIP_PR2(D, CB, X, Y, Z, N)        \
+    if (upd)                                \
+        TOHIP_PR(D, true, CB, X, Y, Z, N);  \
+    else                                    \
+        TOHIP_PR(D, false, CB, X, Y, Z, N)
+    if (L.g.dim == 2) {
+        TOHIP_PR2(2, false, 16, 8, 1, 256);
+    } else if (L.op.is_cube) {
+        TOHIP_PR2(3, true, 4, 4, 4, 256);
+    } else {
+        TOHIP_PR2(3, false, 4, 4, 4, 256);
+    }
+#undef TOHIP_PR2
+#undef TOHIP_PR
+    return hipGetLastError();
+}
+
+// The tile of a 3D level stages 5 nodes per node it owns (2D: 1.6), which pays while
+// the level is latency-bound: an iteration of the multigrid PCG with every level so
+// against none, 120x40x40 (192,000 cells) 107 against 94 us, 76x36x28 (76,608) 84
+// against 87 and 82 with the levels from 9,576 cells down only.
+bool mg_fuse_restrict(const Grid& g) { return g.dim == 2 || g.ncells <= (1 << 16); }
 
 bool mg_coarse_fits(const Grid& g) {
     return g.nnodes <= kMgCoarseMaxNodes && g.ncells <= kMgCoarseMaxCells;

@@ -343,6 +343,11 @@ hipError_t launch_mg_smooth_zm(int mode, const Grid& g, const ElemOp<float>& op,
                                hipStream_t s, const Grid* gc = nullptr,
                                const float* xc = nullptr);
 // bc = P^T r, masked at the coarse level's prescribed DOFs.
+// mode 0 (with `upd`: mode 3) and the restriction of its residual in one launch
+bool mg_fuse_restrict(const Grid& g);
+hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
+                                  const MgLevelView& C, float* xout, float* bc,
+                                  const PcgScalars* sc, const MgFusedUpdate* upd, hipStream_t s);
 hipError_t launch_mg_restrict(const MgLevelView& F, const MgLevelView& C, const float* r,
                               float* bc, const PcgScalars* sc, hipStream_t s);
 // Chebyshev iteration on D^-1 K x = D^-1 b from x = 0 (a fixed polynomial):
