@@ -637,17 +637,9 @@ hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, d
     for (int l = 0; l < L; ++l) {
         const float* b = l == 0 ? r : M[l].b;
         const MgLevelView F = M[l].view(), C = M[l + 1].view();
-        if (!mg_use_zm(F.g) && mg_fuse_restrict(F.g)) {
-            if ((e = launch_mg_pre_restrict(F, M[l].omega, b, C, M[l].x, M[l + 1].b, sc,
-                                            l == 0 ? upd : nullptr, s)) != hipSuccess)
-                return e;
-            continue;
-        }
-        if ((e = launch_mg_smooth(l == 0 && upd ? 3 : 0, F, M[l].omega, b, nullptr, nullptr,
-                                  nullptr, M[l].x, M[l].rz, md, sc, nullptr, s,
-                                  l == 0 ? upd : nullptr)) != hipSuccess)
+        if ((e = launch_mg_down(F, M[l].omega, b, C, M[l].x, M[l].rz, M[l + 1].b, md, sc,
+                                l == 0 ? upd : nullptr, s)) != hipSuccess)
             return e;
-        if ((e = launch_mg_restrict(F, C, M[l].rz, M[l + 1].b, sc, s)) != hipSuccess) return e;
     }
     // coarsest level: x[L] = sweeps of damped Jacobi
     const float* xc = M[L].x;
@@ -741,8 +733,7 @@ static bool mg_fuse_update() {
 // iterate and residual at every graph boundary, as the host expects.
 int capture_mg_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters) {
     if (*exec) return 0;
-    // (the fused update is a mode of the tile smoother: not with z-marching)
-    const bool fuse = mg_fuse_update() && !mg_use_zm(ctx->g);
+    const bool fuse = mg_fuse_update();
     if (fuse && !ctx->r32b)
         if (int rc = dalloc(ctx, &ctx->r32b, ctx->g.ndof)) return rc;
     float* R[2] = {ctx->r32, ctx->r32b};  // residual of in-graph iteration i: R[i & 1]
@@ -2574,9 +2565,8 @@ int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
                 return launch_copy64(nD, ctx->r64, ctx->t64, s);
             case TOHIP_K_MG_PRE: {
                 tohip_mg_level& L0 = ctx->mg[0];
-                return launch_mg_smooth(0, L0.view(), L0.omega, ctx->r32, nullptr, nullptr,
-                                        nullptr, L0.x, ctx->q32, ctx->meandiag, nullptr, nullptr,
-                                        s);
+                return launch_mg_down(L0.view(), L0.omega, ctx->r32, ctx->mg[1].view(), L0.x,
+                                      ctx->q32, ctx->mg[1].b, ctx->meandiag, nullptr, nullptr, s);
             }
             case TOHIP_K_MG_RESTRICT:
                 return launch_mg_restrict(ctx->mg[0].view(), ctx->mg[1].view(), ctx->mg[0].rz,

@@ -98,6 +98,7 @@ static bool use_zm(const Grid& g) {
 
 template <typename T>
 int pcg_blocks(const Grid& g) {
+    if (sizeof(T) == 4) return march_use(g) ? march_blocks(g) : grid_blocks(ntiles<T>(g));
     return use_zm(g) ? zm_blocks(g) : grid_blocks(ntiles<T>(g));
 }
 int pcg_dirmatvec_blocks(const Grid& g) { return pcg_blocks<double>(g); }
@@ -350,10 +351,12 @@ static void dispatch_matvec(const Grid& g, int nb, hipStream_t s, const ElemOp<T
                             const T* E, T* y, double meandiag, PcgScalars* sc,
                             const double* partB, int nbB, double* partA) {
     const bool pre = PCG && preload_first_tile<T>();
-    if (use_zm(g)) {
-        launch_matvec_zm<T, PCG>(g, op, xin, dinv, p0, p1, fixmask, E, y, meandiag, sc, partB, nbB,
-                                 partA, pre, s);
-        return;
+    if constexpr (!(PCG && sizeof(T) == 4)) {  // (launch_march_dir)
+        if (use_zm(g)) {
+            launch_matvec_zm<T, PCG>(g, op, xin, dinv, p0, p1, fixmask, E, y, meandiag, sc, partB,
+                                     nbB, partA, pre, s);
+            return;
+        }
     }
 #define TOHIP_MV1(D, X, Y, Z, N, CB, PR)                                                       \
     hipLaunchKernelGGL((k_matvec<T, D, PCG, X, Y, Z, N, CB, PR>), dim3(nb), dim3(N), 0, s, g, \
@@ -401,6 +404,10 @@ hipError_t launch_pcg_dirmatvec(const Grid& g, const ElemOp<T>& op, const T* r, 
     const int nb = pcg_blocks<T>(g);
     if (nb > kMaxPartials) return hipErrorInvalidValue;
     if (nbA_out) *nbA_out = nb;
+    if constexpr (sizeof(T) == 4)
+        if (march_use(g))
+            return launch_march_dir(g, op, r, dinv, p0, p1, q, fixmask, E, meandiag, sc, partB, nbB,
+                                    partA, s);
     dispatch_matvec<T, true>(g, nb, s, op, r, dinv, p0, p1, fixmask, E, q, meandiag, sc, partB,
                              nbB, partA);
     return hipGetLastError();

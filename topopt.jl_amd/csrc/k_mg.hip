@@ -37,6 +37,7 @@
 //     levels).
 //   k_mg_coarse:   all coarsest sweeps in one workgroup, everything in LDS.
 //   k_mg_coarsen:  coarse moduli.
+//   3D levels of 2^17 cells and more: k_march.hip.
 // Every kernel returns at once when the PCG state says the solve is done, so
 // the iteration graphs replay as no-ops after convergence.
 #include <algorithm>
@@ -848,10 +849,9 @@ __global__ __launch_bounds__(256) void k_mg_coarsen(Grid gf, Grid gc, const doub
     E32[C] = (float)s;
 }
 
-// x' = x + P xc in place, 0 at the fine prescribed DOFs: the first half of the
-// post-smoothing when the finest level smooths by z-marching columns.  Same
-// terms and order as the tile kernel's staging (coarse corners ascending).
-template <int DIM>
+// x' = x + P xc in place on a 3D level, 0 at the fine prescribed DOFs: the separate
+// form of the prolongation in k_march, with its terms and order (the mean of four
+// coarse nodes per plane, which repeat on even coordinates, then of two planes).
 __global__ __launch_bounds__(256) void k_mg_prolong_add(Grid g, Grid gc,
                                                         const uint8_t* __restrict__ fixmask,
                                                         const float* __restrict__ xc,
@@ -860,25 +860,22 @@ __global__ __launch_bounds__(256) void k_mg_prolong_add(Grid g, Grid gc,
     if (mg_done(sc)) return;
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= g.nnodes) return;
-    const int gi = n % g.NX, gj = (n / g.NX) % g.NY, gk = DIM == 3 ? n / (g.NX * g.NY) : 0;
-    constexpr int NC = 1 << DIM;
-    const int I0 = gi >> 1, J0 = gj >> 1, K0 = gk >> 1;
-    const int oi = gi & 1, oj = gj & 1, ok = DIM == 3 ? (gk & 1) : 0;
-    float v[DIM];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) v[d] = x[DIM * n + d];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const int a = c & 1, bb = (c >> 1) & 1, cc = (c >> 2) & 1;
-        if ((a && !oi) || (bb && !oj) || (cc && !ok)) continue;
-        const float wt = (oi ? 0.5f : 1.f) * (oj ? 0.5f : 1.f) * (DIM == 3 && ok ? 0.5f : 1.f);
-        const int N = (I0 + a) + gc.NX * ((J0 + bb) + gc.NY * (K0 + cc));
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) v[d] += wt * xc[DIM * N + d];
-    }
+    const int gi = n % g.NX, gj = (n / g.NX) % g.NY, gk = n / (g.NX * g.NY);
+    const int dx = gi & 1, dy = (gj & 1) ? gc.NX : 0, dz = (gk & 1) ? gc.NX * gc.NY : 0;
+    const int N = (gi >> 1) + gc.NX * ((gj >> 1) + gc.NY * (gk >> 1));
     const uint8_t m = fixmask[n];
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) x[DIM * n + d] = ((m >> d) & 1) ? 0.f : v[d];
+    for (int d = 0; d < 3; ++d) {
+        float c[2];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const int M = N + z * dz;
+            c[z] = 0.25f * ((xc[3 * M + d] + xc[3 * (M + dx) + d]) +
+                            (xc[3 * (M + dy) + d] + xc[3 * (M + dx + dy) + d]));
+        }
+        const float v = x[3 * n + d] + 0.5f * (c[0] + c[1]);
+        x[3 * n + d] = ((m >> d) & 1) ? 0.f : v;
+    }
 }
 
 // Smoother weight from the partials of the last two power steps, one
@@ -927,7 +924,7 @@ static int mg_tile_blocks(const Grid& g) {
 }
 
 int mg_blocks(const Grid& g) {
-    if (mg_use_zm(g)) return zm_blocks(g);  // the z-marching smoother's grid
+    if (march_use(g)) return march_blocks(g);  // the marching smoother's grid
     return mg_tile_blocks(g);
 }
 
@@ -943,25 +940,21 @@ hipError_t launch_mg_smooth(int mode, const MgLevelView& L, float w, const float
     if (mode == 3 && (L.g.dim != 3 || !upd || !upd->sc || upd->sc != sc))
         return hipErrorInvalidValue;
     if (mode == 5 && (!aux || !xprev || !part)) return hipErrorInvalidValue;
-    if ((mode == 0 || mode == 1) && mg_use_zm(L.g)) {
-        // z-marching columns; the post-smoothing forms x' = xprev + P xc while
-        // staging (TOHIP_ZM_PROL=0, read on every call for comparisons: in a
-        // separate pass first, in place in xprev, which the cycle does not
-        // read again)
+    if (mode == 1 && march_use(L.g)) {
+        // the marching post-smoothing forms x' = xprev + P xc while staging
+        // (TOHIP_ZM_PROL=0, read on every call for comparisons: in a separate pass
+        // first, in place in xprev, which the cycle does not read again)
         float* xp = const_cast<float*>(xprev);
-        if (mode == 1) {
-            if (!C || !xc || !xp || C->g.nx * 2 != L.g.nx || C->g.ny * 2 != L.g.ny ||
-                C->g.nz * 2 != L.g.nz)
-                return hipErrorInvalidValue;
-            const char* e = getenv("TOHIP_ZM_PROL");
-            if (!(e && atoi(e) == 0))
-                return launch_mg_smooth_zm(2, L.g, L.op, L.E32, L.fixmask, L.dinv, w, L.wdev, xp,
-                                           b, xout, rout, meandiag, sc, part, s, &C->g, xc);
-            hipLaunchKernelGGL(k_mg_prolong_add<3>, dim3((unsigned)((L.g.nnodes + 255) / 256)),
+        if (!C || !xc || !xp || C->g.nx * 2 != L.g.nx || C->g.ny * 2 != L.g.ny ||
+            C->g.nz * 2 != L.g.nz)
+            return hipErrorInvalidValue;
+        const char* e = getenv("TOHIP_ZM_PROL");
+        if (e && atoi(e) == 0) {
+            hipLaunchKernelGGL(k_mg_prolong_add, dim3((unsigned)((L.g.nnodes + 255) / 256)),
                                dim3(256), 0, s, L.g, C->g, L.fixmask, xc, xp, sc);
+            xc = nullptr;
         }
-        return launch_mg_smooth_zm(mode == 0 ? 1 : 2, L.g, L.op, L.E32, L.fixmask, L.dinv, w,
-                                   L.wdev, xp, b, xout, rout, meandiag, sc, part, s);
+        return launch_march_post(L, w, b, xp, *C, xc, xout, sc, part, s);
     }
     const int nb = mode == 5 ? mg_power_blocks(L.g) : mg_tile_blocks(L.g);
     const Grid gc = C ? C->g : L.g;
@@ -1041,7 +1034,7 @@ hipError_t launch_mg_restrict(const MgLevelView& F, const MgLevelView& C, const 
     return hipGetLastError();
 }
 
-hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
+static hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
                                   const MgLevelView& C, float* xout, float* bc,
                                   const PcgScalars* sc, const MgFusedUpdate* upd, hipStream_t s) {
     if (C.g.nx * 2 != L.g.nx || C.g.ny * 2 != L.g.ny || (L.g.dim == 3 && C.g.nz * 2 != L.g.nz) ||
@@ -1077,7 +1070,17 @@ hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
 // the level is latency-bound: an iteration of the multigrid PCG with every level so
 // against none, 120x40x40 (192,000 cells) 107 against 94 us, 76x36x28 (76,608) 84
 // against 87 and 82 with the levels from 9,576 cells down only.
-bool mg_fuse_restrict(const Grid& g) { return g.dim == 2 || g.ncells <= (1 << 16); }
+static bool mg_fuse_restrict(const Grid& g) { return g.dim == 2 || g.ncells <= (1 << 16); }
+
+hipError_t launch_mg_down(const MgLevelView& L, float w, const float* b, const MgLevelView& C,
+                          float* xout, float* rz, float* bc, double meandiag, const PcgScalars* sc,
+                          const MgFusedUpdate* upd, hipStream_t s) {
+    if (march_use(L.g)) return launch_march_pre(L, w, b, C, xout, bc, sc, upd, s);
+    if (mg_fuse_restrict(L.g)) return launch_mg_pre_restrict(L, w, b, C, xout, bc, sc, upd, s);
+    const hipError_t e = launch_mg_smooth(upd ? 3 : 0, L, w, b, nullptr, nullptr, nullptr, xout, rz,
+                                          meandiag, sc, nullptr, s, upd);
+    return e != hipSuccess ? e : launch_mg_restrict(L, C, rz, bc, sc, s);
+}
 
 bool mg_coarse_fits(const Grid& g) {
     return g.nnodes <= kMgCoarseMaxNodes && g.ncells <= kMgCoarseMaxCells;

@@ -330,24 +330,29 @@ hipError_t launch_mg_omega(const double* prev, const double* part, int nb, float
                           float wsafe, float wmax, float margin, hipStream_t s);
 // v[i] uniform in [-0.5, 0.5) from a hash of i (start of the estimate)
 hipError_t launch_mg_fill_start(int64_t n, float* v, hipStream_t s);
-// Finest-level smoothing by z-marching columns (k_matvec_zm.hip): whether a
-// level takes it, and the launch (mode 1: pre on b; mode 2: post on xin = x').
-bool mg_use_zm(const Grid& g);
 int64_t zm_min_cells();  // smallest grid the z-marching kernels take (cells)
 int zm_blocks(const Grid& g);  // grid (= partial count) of the z-marching kernels on g
-hipError_t launch_mg_smooth_zm(int mode, const Grid& g, const ElemOp<float>& op, const float* E,
-                               const uint8_t* fixmask, const float* dinv, float w,
-                               const float* wdev, const float* xin, const float* b, float* xout,
-                               float* rout,
-                               double meandiag, const PcgScalars* sc, double* part,
-                               hipStream_t s, const Grid* gc = nullptr,
-                               const float* xc = nullptr);
 // bc = P^T r, masked at the coarse level's prescribed DOFs.
-// mode 0 (with `upd`: mode 3) and the restriction of its residual in one launch
-bool mg_fuse_restrict(const Grid& g);
-hipError_t launch_mg_pre_restrict(const MgLevelView& L, float w, const float* b,
-                                  const MgLevelView& C, float* xout, float* bc,
-                                  const PcgScalars* sc, const MgFusedUpdate* upd, hipStream_t s);
+// Pre-smoothing with restriction, post-smoothing with prolongation and the FP32
+// direction step by marching columns (k_march.hip): whether a grid takes them, and
+// the workgroups (= partials) of the latter two.
+bool march_use(const Grid& g);
+int march_blocks(const Grid& g);
+hipError_t launch_march_dir(const Grid& g, const ElemOp<float>& op, const float* r,
+                            const float* dinv, float* p0, float* p1, float* q,
+                            const uint8_t* fixmask, const float* E, double md, PcgScalars* sc,
+                            const double* partB, int nbB, double* partA, hipStream_t s);
+hipError_t launch_march_post(const MgLevelView& L, float w, const float* b, const float* x,
+                             const MgLevelView& C, const float* xc, float* z, const PcgScalars* sc,
+                             double* part, hipStream_t s);
+hipError_t launch_march_pre(const MgLevelView& L, float w, const float* b, const MgLevelView& C,
+                            float* xout, float* bc, const PcgScalars* sc, const MgFusedUpdate* upd,
+                            hipStream_t s);
+// One level down: x = w dinv b (with `upd` after the update) and bc = P^T (b - K x),
+// in one launch or two (the residual then goes through rz).
+hipError_t launch_mg_down(const MgLevelView& L, float w, const float* b, const MgLevelView& C,
+                          float* xout, float* rz, float* bc, double meandiag, const PcgScalars* sc,
+                          const MgFusedUpdate* upd, hipStream_t s);
 hipError_t launch_mg_restrict(const MgLevelView& F, const MgLevelView& C, const float* r,
                               float* bc, const PcgScalars* sc, hipStream_t s);
 // Chebyshev iteration on D^-1 K x = D^-1 b from x = 0 (a fixed polynomial):
