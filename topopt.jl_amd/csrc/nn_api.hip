@@ -324,11 +324,14 @@ ConvDesc bwd_desc(const tohip_nn* nn, const NNLayer& l, int B, int level) {
 }
 
 int nn_upload_weights(tohip_nn* nn) {
+    static_assert(kNL <= ConvWeights::kMax, "layers of one launch");
+    ConvWeights t{};
+    t.count = kNL;
     for (int i = 0; i < kNL; ++i) {
-        NNLayer& l = nn->L[i];
-        NCK(launch_weights_to_bf16(l.cout, l.T, l.cin, l.cin32, l.cout32, nn->params + l.woff,
-                                   l.wf, l.wt, nn->stream));
+        const NNLayer& l = nn->L[i];
+        t.layer[i] = {l.cout, l.T, l.cin, l.cin32, l.cout32, nn->params + l.woff, l.wf, l.wt};
     }
+    NCK(launch_weights_to_bf16(t, nn->stream));
     return 0;
 }
 
@@ -393,67 +396,61 @@ int nn_wgrad(tohip_nn* nn, int li, int level, int B, const uint16_t* X, const ui
     return 0;
 }
 
-// dX of layer li from its output gradient dZ
-int nn_dgrad(tohip_nn* nn, int li, int level, int B, const uint16_t* dZ, uint16_t* dX) {
+// dX of layer li from its output gradient dZ; with Z, times silu'(Z): the output
+// gradient of the layer that made li's input.
+int nn_dgrad(tohip_nn* nn, int li, int level, int B, const uint16_t* dZ, uint16_t* dX,
+             uint16_t* Z = nullptr) {
     NNLayer& l = nn->L[li];
     ConvDesc c = bwd_desc(nn, l, B, level);
-    NCK(launch_conv_fwd(c, dZ, l.wt, nullptr, dX, nullptr, nullptr, nn->stream));
+    if (Z) c.act = 2;
+    NCK(launch_conv_fwd(c, dZ, l.wt, nullptr, dX, Z, nullptr, nn->stream));
     return 0;
 }
 
-// Backward pass for B samples (after nn_forward(train) and the loss).
+// Backward pass for B samples (after nn_forward(train) and the loss).  Every
+// kernel that forms an activation's gradient multiplies by silu' as it stores:
+// g1 and g2 hold output gradients (dZ) in turn, 14 passes over them fewer.
 int nn_backward(tohip_nn* nn, int B) {
     hipStream_t s = nn->stream;
     const int D0 = nn->nz, H0 = nn->ny, W0 = nn->nx;
-    const int64_t P0 = B * nn->P[0], P1 = B * nn->P[1], P2 = B * nn->P[2], P3 = B * nn->P[3];
     int rc;
     uint16_t *g1 = nn->g1, *g2 = nn->g2;
-    // output layer (identity activation)
-    {
-        if ((rc = nn_wgrad(nn, 14, 0, B, nn->d0, nn->dout))) return rc;
-        if ((rc = nn_dgrad(nn, 14, 0, B, nn->dout, g1))) return rc;  // d d0
-    }
-    // a (silu) layer: dZ = silu'(Z) dA into gZ, wgrad, dgrad into gX
-    auto layer = [&](int li, int level, int64_t P, int cout, const uint16_t* dA, uint16_t* gZ,
-                     const uint16_t* X, uint16_t* gX) -> int {
-        NCK(launch_silu_bwd(P * cout, dA, nn->Z[li], gZ, s));
-        int r;
-        if ((r = nn_wgrad(nn, li, level, B, X, gZ))) return r;
-        if (gX)
-            if ((r = nn_dgrad(nn, li, level, B, gZ, gX))) return r;
-        return 0;
+    uint16_t** Z = nn->Z;
+    // layer li with input X: weight gradient from dZ, then dX (times silu'(Zx))
+    auto layer = [&](int li, int level, const uint16_t* X, const uint16_t* dZ, uint16_t* dX,
+                     uint16_t* Zx) -> int {
+        if (int r = nn_wgrad(nn, li, level, B, X, dZ)) return r;
+        return dX ? nn_dgrad(nn, li, level, B, dZ, dX, Zx) : 0;
     };
+    // output layer (identity activation)
+    if ((rc = layer(14, 0, nn->d0, nn->dout, g1, Z[13]))) return rc;
     // decoder L0
-    if ((rc = layer(13, 0, P0, 16, g1, g2, nn->ad00, g1))) return rc;
-    if ((rc = layer(12, 0, P0, 16, g1, g2, nn->cat0, nn->dcat0))) return rc;
-    NCK(launch_upsample_bwd(B, D0 >> 1, H0 >> 1, W0 >> 1, 32, nn->dcat0, 48, 0, g1, s));
+    if ((rc = layer(13, 0, nn->ad00, g1, g2, Z[12]))) return rc;
+    if ((rc = layer(12, 0, nn->cat0, g2, nn->dcat0, nullptr))) return rc;
+    NCK(launch_upsample_bwd(B, D0 >> 1, H0 >> 1, W0 >> 1, 32, nn->dcat0, 48, 0, Z[11], g1, s));
     // decoder L1
-    if ((rc = layer(11, 1, P1, 32, g1, g2, nn->ad10, g1))) return rc;
-    if ((rc = layer(10, 1, P1, 32, g1, g2, nn->cat1, nn->dcat1))) return rc;
-    NCK(launch_upsample_bwd(B, D0 >> 2, H0 >> 2, W0 >> 2, 64, nn->dcat1, 96, 0, g1, s));
+    if ((rc = layer(11, 1, nn->ad10, g1, g2, Z[10]))) return rc;
+    if ((rc = layer(10, 1, nn->cat1, g2, nn->dcat1, nullptr))) return rc;
+    NCK(launch_upsample_bwd(B, D0 >> 2, H0 >> 2, W0 >> 2, 64, nn->dcat1, 96, 0, Z[9], g1, s));
     // decoder L2
-    if ((rc = layer(9, 2, P2, 64, g1, g2, nn->ad20, g1))) return rc;
-    if ((rc = layer(8, 2, P2, 64, g1, g2, nn->cat2, nn->dcat2))) return rc;
-    NCK(launch_upsample_bwd(B, D0 >> 3, H0 >> 3, W0 >> 3, 128, nn->dcat2, 192, 0, g1, s));
+    if ((rc = layer(9, 2, nn->ad20, g1, g2, Z[8]))) return rc;
+    if ((rc = layer(8, 2, nn->cat2, g2, nn->dcat2, nullptr))) return rc;
+    NCK(launch_upsample_bwd(B, D0 >> 3, H0 >> 3, W0 >> 3, 128, nn->dcat2, 192, 0, Z[7], g1, s));
     // encoder L3
-    if ((rc = layer(7, 3, P3, 128, g1, g2, nn->a30, g1))) return rc;
-    if ((rc = layer(6, 3, P3, 128, g1, g2, nn->p3, g1))) return rc;  // g1 = d p3 (64 ch)
-    NCK(launch_avgpool_bwd(B, D0 >> 2, H0 >> 2, W0 >> 2, 64, g1, nn->dcat2, 192, 128, 1, s));
-    NCK(launch_slice_copy(P2, 64, nn->dcat2, 192, 128, g1, 0, s));  // d e2
+    if ((rc = layer(7, 3, nn->a30, g1, g2, Z[6]))) return rc;
+    if ((rc = layer(6, 3, nn->p3, g2, g1, nullptr))) return rc;  // d p3 (64 channels)
+    NCK(launch_skip_bwd(B, D0 >> 2, H0 >> 2, W0 >> 2, 64, g1, nn->dcat2, 192, 128, Z[5], g2, s));
     // encoder L2
-    if ((rc = layer(5, 2, P2, 64, g1, g2, nn->a20, g1))) return rc;
-    if ((rc = layer(4, 2, P2, 64, g1, g2, nn->p2, g1))) return rc;  // d p2 (32 ch)
-    NCK(launch_avgpool_bwd(B, D0 >> 1, H0 >> 1, W0 >> 1, 32, g1, nn->dcat1, 96, 64, 1, s));
-    NCK(launch_slice_copy(P1, 32, nn->dcat1, 96, 64, g1, 0, s));  // d e1
+    if ((rc = layer(5, 2, nn->a20, g2, g1, Z[4]))) return rc;
+    if ((rc = layer(4, 2, nn->p2, g1, g2, nullptr))) return rc;  // d p2 (32 channels)
+    NCK(launch_skip_bwd(B, D0 >> 1, H0 >> 1, W0 >> 1, 32, g2, nn->dcat1, 96, 64, Z[3], g1, s));
     // encoder L1
-    if ((rc = layer(3, 1, P1, 32, g1, g2, nn->a10, g1))) return rc;
-    if ((rc = layer(2, 1, P1, 32, g1, g2, nn->p1, g1))) return rc;  // d p1 (16 ch)
-    NCK(launch_avgpool_bwd(B, D0, H0, W0, 16, g1, nn->dcat0, 48, 32, 1, s));
-    NCK(launch_slice_copy(P0, 16, nn->dcat0, 48, 32, g1, 0, s));  // d e0
+    if ((rc = layer(3, 1, nn->a10, g1, g2, Z[2]))) return rc;
+    if ((rc = layer(2, 1, nn->p1, g2, g1, nullptr))) return rc;  // d p1 (16 channels)
+    NCK(launch_skip_bwd(B, D0, H0, W0, 16, g1, nn->dcat0, 48, 32, Z[1], g2, s));
     // encoder L0
-    if ((rc = layer(1, 0, P0, 16, g1, g2, nn->a00, g1))) return rc;
-    if ((rc = layer(0, 0, P0, 16, g1, g2, nn->feat, nullptr))) return rc;
-    return 0;
+    if ((rc = layer(1, 0, nn->a00, g2, g1, Z[0]))) return rc;
+    return layer(0, 0, nn->feat, g1, nullptr, nullptr);
 }
 
 void nn_free(tohip_nn* nn) {
@@ -767,12 +764,13 @@ int tohip_nn_add_sample(tohip_nn* nn, const double* xphys, const double* f, cons
 static int nn_batch(tohip_nn* nn, const int* idx, int B, bool train, double lr, double* loss) {
     hipStream_t s = nn->stream;
     const int64_t nd = nn->PN * 3;
-    for (int b = 0; b < B; ++b) {
-        NCK(hipMemcpyAsync(nn->feat + (size_t)b * nn->P[0] * kFeat,
-                           nn->ds_feat + (size_t)idx[b] * nn->P[0] * kFeat,
-                           nn->P[0] * kFeat * sizeof(uint16_t), hipMemcpyDeviceToDevice, s));
-        NCK(hipMemcpyAsync(nn->tgt + (size_t)b * nd, nn->ds_u + (size_t)idx[b] * nd,
-                           nd * sizeof(float), hipMemcpyDeviceToDevice, s));
+    const int64_t nf = nn->P[0] * kFeat * (int64_t)sizeof(uint16_t) / 16;
+    for (int b = 0; b < B; b += NNBatch::kMax) {
+        NNBatch t{};
+        t.count = std::min(B - b, (int)NNBatch::kMax);
+        for (int i = 0; i < t.count; ++i) t.idx[i] = idx[b + i];
+        NCK(launch_nn_gather(t, nf, nn->ds_feat, nn->feat + (size_t)b * nn->P[0] * kFeat, nd,
+                             nn->ds_u, nn->tgt + (size_t)b * nd, s));
     }
     int rc = nn_forward(nn, B, train);
     if (rc) return rc;
@@ -960,7 +958,12 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
     QCK(hipMemcpyAsync(dDY, hdy.data(), ny * 2, hipMemcpyHostToDevice, s));
     QCK(hipMemcpyAsync(dW, w, nw * 4, hipMemcpyHostToDevice, s));
     QCK(hipMemcpyAsync(dB, b, cout * 4, hipMemcpyHostToDevice, s));
-    QCK(launch_weights_to_bf16(cout, l.T, cin, l.cin32, l.cout32, dW, l.wf, l.wt, s));
+    {
+        ConvWeights wts{};
+        wts.count = 1;
+        wts.layer[0] = {cout, l.T, cin, l.cin32, l.cout32, dW, l.wf, l.wt};
+        QCK(launch_weights_to_bf16(wts, s));
+    }
     QCK(launch_conv_fwd(c, dX, l.wf, dB, nullptr, dZ, dYf, s));
     if (act) {
         QCK(launch_silu_bwd(ny, dDY, dZ, dZg, s));

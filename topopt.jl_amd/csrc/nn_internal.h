@@ -17,7 +17,7 @@ struct ConvDesc {
     int out_cstride;   // channels of the output tensor (writes into a concat view)
     int out_coff;      // channel offset of the view
     int out_cvalid;    // FP32 output: channels stored
-    int act;           // 0 identity, 1 SiLU
+    int act;           // 0 identity, 1 SiLU, 2 times silu'(Z) (Z read, not written)
 };
 
 hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t* W,
@@ -28,20 +28,36 @@ hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t*
 size_t conv_bwd_w_floats(const ConvDesc& c);
 hipError_t launch_conv_bwd_w(const ConvDesc& c, const uint16_t* X, const uint16_t* dY,
                              float* part, float* dW, float* db, hipStream_t s);
-hipError_t launch_weights_to_bf16(int Cout, int T, int Cin, int Cin32, int Cout32,
-                                  const float* w, uint16_t* wf, uint16_t* wt, hipStream_t s);
+// Layers whose FP32 weights go to BF16, in one launch.
+struct ConvWeights {
+    static constexpr int kMax = 16;
+    struct Layer {
+        int Cout, T, Cin, Cin32, Cout32;
+        const float* w;
+        uint16_t *wf, *wt;
+    } layer[kMax];
+    int count;
+};
+hipError_t launch_weights_to_bf16(const ConvWeights& t, hipStream_t s);
+// Samples of the data set into a batch (16-byte words and floats a sample).
+struct NNBatch {
+    static constexpr int kMax = 64;
+    int idx[kMax];
+    int count;
+};
+hipError_t launch_nn_gather(const NNBatch& t, int64_t nf, const void* src_f, void* dst_f, int64_t nu,
+                            const float* src_u, float* dst_u, hipStream_t s);
 hipError_t launch_silu_bwd(int64_t n, const uint16_t* dA, const uint16_t* Z, uint16_t* dZ,
                            hipStream_t s);
 hipError_t launch_avgpool_fwd(int B, int D, int H, int W, int C, const uint16_t* in, int in_cs,
                               int in_co, uint16_t* out, hipStream_t s);
-hipError_t launch_avgpool_bwd(int B, int D, int H, int W, int C, const uint16_t* dout,
-                              uint16_t* din, int in_cs, int in_co, int accumulate,
-                              hipStream_t s);
+hipError_t launch_skip_bwd(int B, int D, int H, int W, int C, const uint16_t* dpool,
+                           const uint16_t* dskip, int cs, int co, const uint16_t* Z, uint16_t* dZ,
+                           hipStream_t s);
 hipError_t launch_upsample_fwd(int B, int D, int H, int W, int C, const uint16_t* in,
                                uint16_t* out, int out_cs, int out_co, hipStream_t s);
 hipError_t launch_upsample_bwd(int B, int D, int H, int W, int C, const uint16_t* dout,
-                               int out_cs, int out_co, uint16_t* din, hipStream_t s);
-hipError_t launch_slice_copy(int64_t P, int C, const uint16_t* src, int src_cs, int src_co,
-                             uint16_t* dst, int accumulate, hipStream_t s);
+                               int out_cs, int out_co, const uint16_t* Z, uint16_t* dZ,
+                               hipStream_t s);
 
 }  // namespace tohip
