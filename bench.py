@@ -52,13 +52,13 @@ def default_weights(nels):
 
 
 KERNEL_NAMES = {
-    "pcg32": "k_matvec<float,3,PCG> (fused direction update + K p)",
+    "pcg32": "k_march DIR (fused direction update + K p; k_matvec<float,PCG> below 2^17 cells)",
     "update32": "k_pcg_update<float> (x += a p, r -= a q, partials)",
-    "mg_pre": "k_mg_smooth<3,0> finest level (x = w D^-1 b, r = b - K x)",
+    "mg_pre": "k_march PRE finest level (x = w D^-1 b, b_c = P^T (b - K x))",
     "mg_restrict": "k_mg_restrict<3> finest -> first coarse level",
     "mg_coarse": ("k_mg_dense_rows: coarsest level, x = M b with M the dense (symmetrised) "
                   "Chebyshev operator, one wave per row"),
-    "mg_post": "k_mg_smooth<3,1> finest level (x += P xc, z = x + w D^-1 (b - K x))",
+    "mg_post": "k_march POST finest level (x += P xc, z = x + w D^-1 (b - K x))",
 }
 
 
@@ -157,8 +157,9 @@ def algorithmic_bytes(prob):
     nn = nd // dim
     mv = lambda s: 2 * s * nd + s * nc  # read x, write y, read E once
     return {
-        # finest-level multigrid kernels (FP32): read b, D^-1, E, mask; write x, r
-        "mg_pre": 4 * 4 * nd + 4 * nc + nn,
+        # finest-level multigrid kernels (FP32): read b, D^-1, E, masks; write x and the
+        # coarse right-hand side (below 2^17 cells in 3D the residual too, in two launches)
+        "mg_pre": 3 * 4 * nd + 4 * nc + nn + 4 * nd1 + nn1,
         # read r (fine), write b and read the mask (first coarse level)
         "mg_restrict": 4 * nd + 4 * nd1 + nn1,
         # read b, D^-1, E, mask; write x (coarsest level, once per cycle)

@@ -371,8 +371,8 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
 #define TOHIP_K_OC 9         /* one full OC update (several launches)   */
 #define TOHIP_K_COPY64 10    /* plain copy of one FP64 DOF vector (16 B per DOF moved) */
 /* multigrid preconditioner of TOHIP_MIXED_MG (built on first use): */
-#define TOHIP_K_MG_PRE 11     /* finest level: x = w D^-1 b, r = b - K x        */
-#define TOHIP_K_MG_RESTRICT 12 /* finest -> first coarse level: P^T r          */
+#define TOHIP_K_MG_PRE 11     /* finest level: x = w D^-1 b, P^T (b - K x)       */
+#define TOHIP_K_MG_RESTRICT 12 /* finest -> first coarse level: P^T r alone    */
 #define TOHIP_K_MG_COARSE 13  /* coarsest level: all Jacobi sweeps (1 workgroup) */
 #define TOHIP_K_MG_POST 14    /* finest level: x += P xc, z = x + w D^-1 (b - K x) */
 #define TOHIP_K_VCYCLE 15     /* one whole V-cycle (every launch of it)         */

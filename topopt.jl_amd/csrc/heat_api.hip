@@ -27,7 +27,6 @@ struct tohip_heat {
     double meandiag = 0.0;
     bool inhom = false;              // some prescribed temperature is nonzero
     int* node_dof = nullptr;         // node id -> caller DOF (0-based), device
-    double* check = nullptr;         // partials of a vector's check
     hipStream_t stream = nullptr;
     uint8_t* fixmask = nullptr;
     double *fixv = nullptr, *x = nullptr, *E = nullptr, *dinv = nullptr;
@@ -119,7 +118,7 @@ int upload_nodes(tohip_heat* ctx, const double* host, double* dev, bool* finite 
     if (finite && n > kHostCheckMax) {
         long double ss;
         double bad;
-        HCK(values_check(n, ctx->r[1], ctx->check, &ss, &bad, ctx->stream));
+        HCK(values_check(n, ctx->r[1], ctx->part[0], &ss, &bad, ctx->stream));
         if (!(*finite = bad == 0.0)) return 0;
     } else {
         HCK(hipStreamSynchronize(ctx->stream));
@@ -213,7 +212,7 @@ void free_heat(tohip_heat* ctx) {
     void* bufs[] = {ctx->fixmask, ctx->fixv, ctx->x,    ctx->E,    ctx->dinv,    ctx->u,
                     ctx->r[0],    ctx->r[1], ctx->p[0], ctx->p[1], ctx->q[0],    ctx->q[1],
                     ctx->b,       ctx->t,    ctx->lam,  ctx->cell, ctx->grad,    ctx->part[0],
-                    ctx->part[1], ctx->st,   ctx->node_dof, ctx->check};
+                    ctx->st,      ctx->node_dof};
     for (void* b : bufs)
         if (b) hipFree(b);
     if (ctx->h_st) hipHostFree(ctx->h_st);
@@ -294,6 +293,8 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
     }
     HCK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     int rc;
+    // partials of one launch, or of a vector's check (3 a block)
+    const size_t npart = std::max<size_t>((size_t)kPcg1Vals * heat_pcg_blocks(g), 3 * kVecBlocks);
     if ((rc = halloc(ctx, &ctx->fixmask, n)) || (rc = halloc(ctx, &ctx->fixv, n)) ||
         (rc = halloc(ctx, &ctx->x, g.ncells)) || (rc = halloc(ctx, &ctx->E, g.ncells)) ||
         (rc = halloc(ctx, &ctx->dinv, n)) || (rc = halloc(ctx, &ctx->u, n)) ||
@@ -303,11 +304,10 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
         (rc = halloc(ctx, &ctx->b, n)) || (rc = halloc(ctx, &ctx->t, n)) ||
         (rc = halloc(ctx, &ctx->lam, n)) || (rc = halloc(ctx, &ctx->cell, g.ncells)) ||
         (rc = halloc(ctx, &ctx->grad, g.ncells)) || 
-        (rc = halloc(ctx, &ctx->part[0], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
-        (rc = halloc(ctx, &ctx->part[1], (size_t)kPcg1Vals * heat_pcg_blocks(g))) ||
-        (rc = halloc(ctx, &ctx->st, 2)) || (rc = halloc(ctx, &ctx->node_dof, n)) ||
-        (rc = halloc(ctx, &ctx->check, 3 * kVecBlocks)))
+        (rc = halloc(ctx, &ctx->part[0], 2 * npart)) || (rc = halloc(ctx, &ctx->st, 2)) ||
+        (rc = halloc(ctx, &ctx->node_dof, n)))
         return rc;
+    ctx->part[1] = ctx->part[0] + npart;
     HCK(hipHostMalloc((void**)&ctx->h_st, sizeof(Pcg1State), hipHostMallocDefault));
     HCK(hipMemcpyAsync(ctx->node_dof, node_dof.data(), n * sizeof(int), hipMemcpyHostToDevice,
                        ctx->stream));
