@@ -451,9 +451,9 @@ hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t*
 //
 // Bound by the staging (the halo is read 3 to 4 times from L2) and, per MFMA, by
 // little else: MI355X, 64x32x32, batch 8, the weight and bias gradients of a step's
-// 15 layers take 0.55 ms, against 2.34 ms for a wave per tap and 16 x 16 tile that
+// 15 layers take 0.51 ms, against 2.34 ms for a wave per tap and 16 x 16 tile that
 // gathered both operands again for every tap, with kernels of their own for the
-// bias (130 TFLOP/s against 30).
+// bias (140 TFLOP/s against 30).
 constexpr int kWgTX = 8, kWgSubs = 8;
 
 struct WgradShape {
@@ -613,16 +613,19 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(ConvDesc c, WgradShape sh,
 }
 
 // dW[co][tap][ci] and db[co] from the splits' partials.  Block (ct, it, tap): 64
-// lanes as the MFMA leaves the 16 x 16 tile, times 4 quarters of the splits, added
-// in order; the last ct blocks: the bias.
-__global__ __launch_bounds__(256) void k_conv_wgrad_sum(ConvDesc c, WgradShape sh, int T,
+// lanes as the MFMA leaves the 16 x 16 tile, times Q shares of the splits, added
+// in order; the last ct blocks: the bias.  A share is a chain of round trips of 8
+// loads: 16 shares from 64 splits on, 8.7 -> 6.1 us on average over the 15 layers at
+// 64x32x32, batch 8 (line at 32: 6.3).
+template <int Q>
+__global__ __launch_bounds__(64 * Q) void k_conv_wgrad_sum(ConvDesc c, WgradShape sh, int T,
                                                         const float* __restrict__ part,
                                                         const float* __restrict__ bpart,
                                                         float* __restrict__ dW,
                                                         float* __restrict__ db) {
-    __shared__ float4 red[4][64];
+    __shared__ float4 red[Q][64];
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int nb = sh.ct * sh.it * T, chunk = (sh.ns + 3) / 4;
+    const int nb = sh.ct * sh.it * T, chunk = (sh.ns + Q - 1) / Q;
     const int s0 = q * chunk, s1 = min(s0 + chunk, sh.ns);
     const bool bias = (int)blockIdx.x >= nb;
     const int tile = blockIdx.x - nb;
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad_sum(ConvDesc c, WgradShape s
     if (q != 0) return;
     a = red[0][lane];
 #pragma unroll
-    for (int k = 1; k < 4; ++k) {
+    for (int k = 1; k < Q; ++k) {
         const float4 v = red[k][lane];
         a.x += v.x;
         a.y += v.y;
@@ -731,8 +734,13 @@ hipError_t launch_conv_bwd_w(const ConvDesc& c, const uint16_t* X, const uint16_
     e = k == 3 ? TOHIP_WG(3) : k == 2 ? TOHIP_WG(2) : TOHIP_WG(1);
 #undef TOHIP_WG
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_conv_wgrad_sum, dim3(sh.ct * sh.it * T + sh.ct), dim3(256), 0, s, c, sh, T,
-                       part, bpart, dW, db);
+    const dim3 grid(sh.ct * sh.it * T + sh.ct);
+    if (sh.ns >= 64)
+        hipLaunchKernelGGL(k_conv_wgrad_sum<16>, grid, dim3(1024), 0, s, c, sh, T, part, bpart, dW,
+                           db);
+    else
+        hipLaunchKernelGGL(k_conv_wgrad_sum<4>, grid, dim3(256), 0, s, c, sh, T, part, bpart, dW,
+                           db);
     return hipGetLastError();
 }
 
