@@ -65,7 +65,7 @@ __device__ __forceinline__ uint16_t silu_bwd(uint16_t dA, uint16_t zb) {
 // positions cannot fill the chip, many blocks and a short load -> MFMA chain.
 constexpr int kConvMaxTaps = 32;
 
-template <int NSUB>
+template <int NSUB, bool BWD>
 __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __restrict__ X,
                                                   const uint16_t* __restrict__ W,
                                                   const float* __restrict__ bias,
@@ -171,9 +171,9 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
                 if (co < c.out_cvalid) Yf[pos * c.out_cvalid + co] = y;
             } else {
                 Y[pos * c.out_cstride + c.out_coff + co] =
-                    c.act == 2 ? silu_bwd(f2bf(y), Z[pos * c.Cout + co]) : f2bf(y);
+                    BWD ? silu_bwd(f2bf(y), Z[pos * c.Cout + co]) : f2bf(y);
             }
-            if (Z && c.act != 2) Z[pos * c.Cout + co] = f2bf(z);
+            if (!BWD && Z) Z[pos * c.Cout + co] = f2bf(z);
         }
     }
 }
@@ -192,7 +192,8 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvDesc c, const uint16_t* __
 template <int CK>
 constexpr int kFwdPitch = CK == 8 ? 16 : CK * 2 + 16;  // bytes of a staged place
 
-template <int K, int NT, int MT>
+// BWD (act 2) is a form of its own: its epilogue as a branch cost a prediction 1-2 %.
+template <int K, int NT, int MT, bool BWD>
 __global__ __launch_bounds__(256) void k_conv_tile(ConvDesc c, int ntx, int nty, int ntz,
                                                    const uint16_t* __restrict__ X,
                                                    const uint16_t* __restrict__ W,
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(256) void k_conv_tile(ConvDesc c, int ntx, int nty,
             const float bb = bias && co < c.Cout ? bias[co] : 0.f;
             float zv[4], yv[4];
             uint16_t zb[4] = {};
-            if (c.act == 2)
+            if (BWD)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int x = min(x0 + 4 * (kq & 1) + i, c.OW - 1);
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(256) void k_conv_tile(ConvDesc c, int ntx, int nty,
             for (int i = 0; i < 4; ++i) {
                 zv[i] = acc[m][n][i] + bb;
                 yv[i] = c.act == 1 ? silu(zv[i]) : zv[i];
-                if (c.act == 2) yv[i] = bf2f(silu_bwd(f2bf(yv[i]), zb[i]));
+                if (BWD) yv[i] = bf2f(silu_bwd(f2bf(yv[i]), zb[i]));
             }
             if (Yf)
 #pragma unroll
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(256) void k_conv_tile(ConvDesc c, int ntx, int nty,
                 }
             };
             if (!Yf) store(yv, Y, c.out_cstride, c.out_coff);
-            if (Z && c.act != 2) store(zv, Z, c.Cout, 0);
+            if (!BWD && Z) store(zv, Z, c.Cout, 0);
         }
     }
 }
@@ -374,9 +375,13 @@ static hipError_t launch_conv_tile(const ConvDesc& c, const uint16_t* X, const u
                                    hipStream_t s) {
     constexpr int BY = MT == 1 ? 4 : 8, BZ = MT == 4 ? 4 : 2;
     const int ntx = (c.OW + 7) / 8, nty = (c.OH + BY - 1) / BY, ntz = (c.OD + BZ - 1) / BZ;
-    hipLaunchKernelGGL((k_conv_tile<K, NT, MT>),
-                       dim3((unsigned)(ntx * nty * ntz * c.B), (c.Cout + 16 * NT - 1) / (16 * NT)),
-                       dim3(256), 0, s, c, ntx, nty, ntz, X, W, bias, Y, Z, Yf);
+    const dim3 grid((unsigned)(ntx * nty * ntz * c.B), (c.Cout + 16 * NT - 1) / (16 * NT));
+    if (c.act == 2)
+        hipLaunchKernelGGL((k_conv_tile<K, NT, MT, true>), grid, dim3(256), 0, s, c, ntx, nty, ntz,
+                           X, W, bias, Y, Z, Yf);
+    else
+        hipLaunchKernelGGL((k_conv_tile<K, NT, MT, false>), grid, dim3(256), 0, s, c, ntx, nty, ntz,
+                           X, W, bias, Y, Z, Yf);
     return hipGetLastError();
 }
 
@@ -423,11 +428,18 @@ hipError_t launch_conv_fwd(const ConvDesc& c, const uint16_t* X, const uint16_t*
     int nsub = c.Cout >= 64 ? 4 : c.Cout >= 32 ? 2 : 1;
     while (nsub > 1 && (P + 15) / 16 * ((c.Cout + 16 * nsub - 1) / (16 * nsub)) < 1024) nsub /= 2;
     const dim3 grid((unsigned)((P + 15) / 16), (unsigned)((c.Cout + 16 * nsub - 1) / (16 * nsub)));
-#define TOHIP_CONV(NS)                                                                            \
-    hipLaunchKernelGGL((k_conv_fwd<NS>), grid, dim3(256), 0, s, c, X, W, bias, Y, Z, Yf)
-    if (nsub == 4) TOHIP_CONV(4);
-    else if (nsub == 2) TOHIP_CONV(2);
-    else TOHIP_CONV(1);
+#define TOHIP_CONV(NS)                                                                              \
+    if (c.act == 2)                                                                                 \
+        hipLaunchKernelGGL((k_conv_fwd<NS, true>), grid, dim3(256), 0, s, c, X, W, bias, Y, Z, Yf); \
+    else                                                                                            \
+        hipLaunchKernelGGL((k_conv_fwd<NS, false>), grid, dim3(256), 0, s, c, X, W, bias, Y, Z, Yf)
+    if (nsub == 4) {
+        TOHIP_CONV(4);
+    } else if (nsub == 2) {
+        TOHIP_CONV(2);
+    } else {
+        TOHIP_CONV(1);
+    }
 #undef TOHIP_CONV
     return hipGetLastError();
 }
