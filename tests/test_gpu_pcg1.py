@@ -116,3 +116,125 @@ def test_assembled_product_and_solve(T, O, gpu, nels, jacobi):
         if n < it:
             s(abstol=0.0, reltol=1e-11, maxiter=n)
             assert s.last_iters == n and not s.converged
+
+
+# More work than workgroups at once (768 in 2D and for heat, 512 in 3D): two columns of
+# tiles, the second one node wide, and a long ragged side
+STRIDED = [((15, 8000), None), ((15, 5800), (1.0, 1.5)), ((15, 3880, 2), None),
+           ((15, 4100, 2), (1.0, 1.5, 0.75))]
+
+
+@pytest.mark.parametrize("case", range(len(STRIDED)))
+def test_strided_elastic(T, O, gpu, case):
+    """The iterates after 0 .. 9 iterations against the oracle's.  The load on the
+    prescribed DOFs goes in the first one, which leaves r.z a millionth of what it was:
+    the launch that applies the update alone."""
+    from topopt_jl_amd._lib import dptr
+    import ctypes as C
+    nels, h = STRIDED[case]
+    prob = T.PointLoadCantilever(nels, sizes=h)
+    s = T.FEASolver(T.HIPMatrixFreeSolver, prob, penalty=T.PowerPenaltyFun(3.0))
+    orc = O.Oracle(O.Cantilever(tuple(nels)), p=3.0, h=h)
+    g = np.random.default_rng(case)
+    x = g.uniform(0.5, 1.0, prob.ncells)
+    s.set_densities(x)
+    orc.set_vars(x)
+    fixed = prob.fixed.astype(bool)
+    b = np.where(fixed, 1e3, 1e-3) * g.standard_normal(prob.ndofs)
+    z = orc.jacobi_diag() ** -1 * b
+    z1 = b - (b @ z) / (z @ orc.matvec(z)) * orc.matvec(z)
+    assert z1 @ (z1 / orc.jacobi_diag()) < 5e-4 * (b @ z)  # due below 1e-3
+    for n in (0, 1, 2, 9):
+        u, again = np.zeros(prob.ndofs), np.zeros(prob.ndofs)
+        it, res = C.c_int64(), C.c_double()
+        for v in (u, again):
+            assert s.lib.tohip_solve(s.ctx.ptr, dptr(b), dptr(v), 0.0, 1e-30, n, 1, 0,
+                                     C.byref(it), C.byref(res)) == 1  # not converged
+        assert it.value == n and np.array_equal(u, again)
+        ue, ite, rese = orc.pcg(b, reltol=1e-30, maxiter=n)
+        assert ite == n
+        # 1e-16 over the part of the residual that the first iteration leaves
+        assert relerr(u, ue) < 1e-9 and abs(res.value - rese) < 1e-9 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("nels", [(15, 8000), (421, 420), (15, 5791, 2)])
+def test_strided_heat(T, gpu, nels):
+    """As above: the guess at the prescribed nodes goes in the first iteration."""
+    import ctypes as C
+    import scipy.sparse as sp
+    from oracle import heat_oracle as H
+    from topopt_jl_amd._lib import dptr
+    sizes = (1.0, 0.7, 1.6)[:len(nels)]
+    prob = T.HeatConductionProblem(nels, sizes, 1.3, Tleft=0.0, Tright=None)
+    s = T.FEASolver(T.HIPMatrixFreeSolver, prob, xmin=0.01, penalty=T.PowerPenaltyFun(3.0))
+    g = np.random.default_rng(sum(nels))
+    x = g.uniform(0.3, 1.0, prob.ncells)
+    s.set_densities(x)
+    dofs = (np.asarray(prob.cell_dofs).T - 1).astype(np.int64)
+    Ke, rho, nc = H.heat_ke(len(nels), sizes, 1.3), 0.01 + 0.99 * x**3, dofs.shape[1]
+    K = sp.csr_matrix(((rho[:, None, None] * Ke).ravel(),
+                       (np.repeat(dofs, nc, axis=1).ravel(), np.tile(dofs, (1, nc)).ravel())))
+    fixed = prob.fixed.astype(bool)
+    md = np.trace(Ke) * prob.ncells
+    diag = np.where(fixed, md, K.diagonal())
+    A = lambda v: np.where(fixed, md * v, K @ np.where(fixed, 0.0, v))
+    v = g.standard_normal(prob.ndofs)
+    assert relerr(s.matvec(v), A(v)) < 1e-14
+    b = np.where(fixed, 0.0, g.standard_normal(prob.ndofs))
+    u0 = np.where(fixed, 1.0, 0.0)
+    u, p, rho_prev = u0.copy(), 0.0, 1.0
+    r = b - A(u)
+    for n in range(10):
+        if n in (0, 1, 2, 9):
+            t, it, res = u0.copy(), C.c_int64(), C.c_double()
+            assert s.lib.tohip_heat_solve(s.ptr, dptr(b), dptr(t), 0.0, 1e-30, n, 0, 0,
+                                          C.byref(it), C.byref(res)) == 1
+            assert it.value == n and relerr(t, u) < 1e-9
+            assert abs(res.value - np.linalg.norm(r)) < 1e-9 * np.linalg.norm(A(u0))
+        z = r / diag
+        rz = r @ z
+        if n == 1:
+            assert rz < 5e-4 * rho_prev  # an update alone is due below 1e-3
+        p = z + rz / rho_prev * p
+        q = A(p)
+        a = rz / (p @ q)
+        u, r, rho_prev = u + a * p, r - a * q, rz
+
+
+def test_iteration_time_grows_with_the_grid(T, gpu):
+    """FP64 elasticity and heat: 1000x990 against 640x320 cells, 4.8 times the nodes.
+    Every workgroup sums every workgroup's partials, so that an iteration of one
+    workgroup a tile took 7.5 and 8 times as long."""
+    import time
+    from topopt_jl_amd import _lib
+    import ctypes as C
+
+    def per_iteration(run):
+        best = []
+        for n in (64, 320):
+            run(n)
+            t = []
+            for _ in range(5):
+                t0 = time.perf_counter()
+                run(n)
+                t.append(time.perf_counter() - t0)
+            best.append(min(t))
+        return best[1] - best[0]
+
+    el, he = [], []
+    for nels in ((640, 320), (1000, 990)):
+        nn = (nels[0] + 1) * (nels[1] + 1)
+        fixed = np.repeat(np.arange(nn) % (nels[0] + 1) == 0, 2).astype(np.uint8)
+        c = _lib.Context(2, nels, np.ones(2), 1.0, 0.3, 1e-3, 3.0, True, None, fixed)
+        g = np.random.default_rng(nn)
+        assert c.lib.tohip_set_densities(c.ptr, _lib.dptr(g.uniform(0.3, 1, c.ncells))) == 0
+        assert c.lib.tohip_set_load(c.ptr, _lib.dptr(g.standard_normal(c.ndofs))) == 0
+        it, res = C.c_int64(), C.c_double()
+        el.append(per_iteration(lambda n: c.lib.tohip_solve(
+            c.ptr, None, None, 0.0, 1e-30, n, 1, 0, C.byref(it), C.byref(res))))
+        prob = T.HeatConductionProblem(nels, (1.0, 1.0), 1.0, Tleft=1.0)
+        s = T.FEASolver(T.HIPMatrixFreeSolver, prob, abstol=0.0, reltol=1e-30)
+        b = g.standard_normal(prob.ndofs)
+        he.append(per_iteration(lambda n: s(rhs=b, maxiter=n)))
+    assert el[1] < 4.8 * el[0], (el[0] / 256, el[1] / 256)
+    assert he[1] < 4.8 * he[0], (he[0] / 256, he[1] / 256)

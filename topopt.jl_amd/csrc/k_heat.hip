@@ -43,9 +43,9 @@ __device__ __forceinline__ int heat_corner(int ox, int oy, int oz) {
 constexpr int kHC = 16, kHO = kHC - 1, kHS = kHC + 1;
 
 // Columns of 15 x 15 nodes and chunks of zc planes, about 768 workgroups when the
-// grid has them; beyond kMaxPartials they stride over the rest.  Fewer planes a
-// chunk fill the chip better but re-stage more (zc + 2 planes each): a PCG
-// iteration at 128x96x80 takes 23.8 us with 756 workgroups, 26.0 with 1008.
+// grid has them.  Fewer planes a chunk fill the chip better but re-stage more (zc + 2
+// planes each): a PCG iteration at 128x96x80 takes 23.8 us with 756 workgroups, 26.0
+// with 1008.
 struct HeatShape {
     int ncx, ncy, zc, nch, nwork;
 };
@@ -60,8 +60,17 @@ static HeatShape heat_shape(const HeatGrid& g) {
     s.nwork = (int)(cols * s.nch);
     return s;
 }
-static int heat_op_blocks(const HeatShape& s) { return std::min(s.nwork, kMaxPartials); }
-int heat_pcg_blocks(const HeatGrid& g) { return heat_op_blocks(heat_shape(g)); }
+// Workgroups of the operator alone, and of a PCG iteration, where every workgroup
+// sums every workgroup's row of partials: no more than run at once (three per CU), the
+// rest of the work strided over.  MI355X, us an iteration with at most 512 / 768 / 1024
+// / 4096 workgroups, and of three launches: 640x320 9.6 / 10.4 / 11.2 / 11.2 and 18.5,
+// 1000x990 24 / 22 / 29 / 91 and 44, 2400x2400 144 / 134 / 162 / 199 and 198, 900x900x2
+// 52 / 49 / 55 / 88 and 150.
+constexpr int kHeatPcgBlocks = 768;
+static int heat_op_blocks(const HeatShape& s, bool pcg) {
+    return std::min(s.nwork, pcg ? kHeatPcgBlocks : kMaxPartials);
+}
+int heat_pcg_blocks(const HeatGrid& g) { return heat_op_blocks(heat_shape(g), true); }
 
 // A staged node's operands.
 struct HeatNode {
@@ -295,8 +304,8 @@ static hipError_t launch_heat_op(const HeatGrid& g, const HeatModes& B, const do
                                  const uint8_t* fixmask, const double* E, double meandiag,
                                  double* y, const Pcg1Args& a, hipStream_t s) {
     const HeatShape sh = heat_shape(g);
-    const dim3 grid(heat_op_blocks(sh)), block(kThreads);
-    const bool loop = sh.nwork > kMaxPartials;
+    const dim3 grid(heat_op_blocks(sh, MODE == 1)), block(kThreads);
+    const bool loop = sh.nwork > (int)grid.x;
     if ((int64_t)g.NX * kHS * 8 >= ((int64_t)1 << 32))
         hipLaunchKernelGGL((k_heat_op<DIM, MODE, uint64_t, true>), grid, block, 0, s, g, B, sh, x,
                            fixmask, E, meandiag, y, a);

@@ -35,7 +35,7 @@ constexpr int kPC = 16, kPO = kPC - 1, kPS = kPC + 1, kPP = kPS * kPS;
 
 // Columns of 15 x 15 nodes and chunks of zc planes (zc + 2 are staged).  A
 // workgroup per CU where that takes chunks of at most 5 planes, else two (256
-// VGPRs: two run per CU); beyond kMaxPartials workgroups stride over the rest.
+// VGPRs: two run per CU).
 // One iteration on MI355X, in the LOOP form (a straight body is 3-7 % faster),
 // with 243 / 378 / 756 workgroups: 120x40x40 23.1 / 22.8 / 30.0 us; with 162 /
 // 486 / 972: 256x128x128 408 / 272 / 297 us; with 180 / 270: 76x36x28 16.6 / 18.1.
@@ -521,9 +521,18 @@ __global__ __launch_bounds__(2 * kThreads) void k_pcg1_plane(Grid g, ElemOp<doub
     pcg1_store_sums<NT>(sum, red, a.partn);
 }
 
+// Work beyond what the chip holds at once (three workgroups per CU in 2D, two in
+// 3D, by the registers of the LOOP form) is strided over: every workgroup sums every
+// workgroup's row of partials, so their number enters squared.  MI355X, us an
+// iteration with at most 512 / 768 / 1024 / 4096 workgroups, and of the direction +
+// update pair: 2D 640x320 11.1 / 11.9 / 13.1 / 13.0 and 17.0, 1000x990 30 / 31 / 37 /
+// 97 and 41, 1500x1500 88 / 84 / 94 / 147 and 81, 2400x2400 213 / 227 / 254 / 274 and
+// 236; 3D 900x900x2 167 / 186 / 174 / 215 and 180, 500x500x2 43 / 48 / 49 / 49 and 90.
+static int pcg1_resident(const Grid& g) { return g.dim == 2 ? 768 : 512; }
+
 int pcg1_blocks(const Grid& g) {
     const int n = pcg1_planes(g);
-    return n ? n : std::min(pcg1_shape(g).nwork, kMaxPartials);
+    return n ? n : std::min(pcg1_shape(g).nwork, pcg1_resident(g));
 }
 
 template <int DIM, bool CUBE>
@@ -531,7 +540,7 @@ static void launch_pcg1_march(const Grid& g, const ElemOp<double>& op, const uin
                               const double* E, double md, const Pcg1Args& a, hipStream_t s) {
     const Pcg1Shape sh = pcg1_shape(g);
     const dim3 grid(pcg1_blocks(g)), block(kThreads);
-    if (sh.nwork > kMaxPartials)
+    if (sh.nwork > (int)grid.x)
         hipLaunchKernelGGL((k_pcg1<DIM, CUBE, true>), grid, block, 0, s, g, op, sh, fixmask, E, md,
                            a);
     else
