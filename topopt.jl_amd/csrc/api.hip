@@ -947,13 +947,15 @@ int solve_fp64(tohip_ctx* ctx, double abstol, double reltol, int64_t maxiter, bo
     if (energy)
         CK(launch_energy_check(n, ctx->u, ctx->r64, ctx->b64, ctx->pcg1_st, ctx->ecrit,
                                ctx->partials, ctx->stream));
-    hipGraphExec_t& lg = energy ? ctx->g64e : ctx->g64;
-    hipGraphExec_t& sg = energy ? ctx->g64es : ctx->g64s;
-    if (int rc = capture_pcg1_graph(ctx, &lg, kPcg1GraphLong, energy)) return rc;
-    if (int rc = capture_pcg1_graph(ctx, &sg, kPcg1GraphShort, energy)) return rc;
+    hipGraphExec_t* graphs = energy ? ctx->g64e : ctx->g64;
     if (ctx->time_graphs) CK(hipEventRecord(ctx->graph_ev[0], ctx->stream));
-    CK(pcg1_replay(lg, sg, ctx->pcg1_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
-                   &ctx->graph_launches));
+    Pcg1Schedule sch;
+    do {
+        const int k = sch.graph;
+        if (int rc = capture_pcg1_graph(ctx, &graphs[k], kPcg1GraphIters[k], energy)) return rc;
+        CK(pcg1_replay(graphs[k], sch, ctx->pcg1_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
+                       &ctx->graph_launches));
+    } while (!ctx->h_pcg1->done);
     if (ctx->time_graphs) {
         CK(hipEventRecord(ctx->graph_ev[1], ctx->stream));
         CK(hipEventSynchronize(ctx->graph_ev[1]));
@@ -1274,7 +1276,7 @@ int load_norm(tohip_ctx* ctx, double* norm) {
 void free_ctx(tohip_ctx* ctx) {
     if (!ctx) return;
     if (ctx->nn) nn_detach_ctx(ctx->nn, ctx);
-    for (hipGraphExec_t ge : {ctx->g64, ctx->g32, ctx->g64s, ctx->g32s})
+    for (hipGraphExec_t ge : {ctx->g32, ctx->g32s})
         if (ge) hipGraphExecDestroy(ge);
     void* bufs[] = {ctx->fixmask, ctx->xt,       ctx->E64,      ctx->E32,    ctx->f,
                     ctx->u,       ctx->b64,      ctx->r64,      ctx->t64,    ctx->dinv64,
@@ -1287,9 +1289,11 @@ void free_ctx(tohip_ctx* ctx) {
     if (ctx->mg_stream) hipStreamSynchronize(ctx->mg_stream);  // a rebuild may be in flight
     for (void* b : bufs)
         if (b) hipFree(b);
-    for (hipGraphExec_t ge : {ctx->g32mg, ctx->g32mgs, ctx->g64e, ctx->g64es, ctx->gcsr, ctx->gcsrs,
-                              ctx->g64mg, ctx->g64mgs})
+    for (hipGraphExec_t ge : {ctx->g32mg, ctx->g32mgs, ctx->g64mg, ctx->g64mgs})
         if (ge) hipGraphExecDestroy(ge);
+    for (auto* graphs : {ctx->g64, ctx->g64e, ctx->gcsr})
+        for (int k = 0; k < kPcg1Graphs; ++k)
+            if (graphs[k]) hipGraphExecDestroy(graphs[k]);
     for (void* b : {(void*)ctx->csr_rowptr, (void*)ctx->csr_cols, (void*)ctx->csr_vals,
                     (void*)ctx->csr_diag, (void*)ctx->csr_dinv, (void*)ctx->csr_ke,
                     (void*)ctx->csr_md, (void*)ctx->mma_L, (void*)ctx->mma_U,
@@ -1842,10 +1846,13 @@ int tohip_csr_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, d
     }
     CK(launch_pcg1_start(n, ctx->b64, initially_zero ? nullptr : ctx->t64, ctx->csr_dinv, ctx->r64,
                          ctx->p64[0], ctx->csr_part, nb, ctx->stream));
-    if (int rc = capture_csr_graph(ctx, &ctx->gcsr, kPcg1GraphLong)) return rc;
-    if (int rc = capture_csr_graph(ctx, &ctx->gcsrs, kPcg1GraphShort)) return rc;
-    CK(pcg1_replay(ctx->gcsr, ctx->gcsrs, ctx->csr_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
-                   &ctx->graph_launches));
+    Pcg1Schedule sch;
+    do {
+        const int k = sch.graph;
+        if (int rc = capture_csr_graph(ctx, &ctx->gcsr[k], kPcg1GraphIters[k])) return rc;
+        CK(pcg1_replay(ctx->gcsr[k], sch, ctx->csr_st, ctx->h_pcg1, ctx->stream, &ctx->host_syncs,
+                       &ctx->graph_launches));
+    } while (!ctx->h_pcg1->done);
     const Pcg1State& h = *ctx->h_pcg1;
     if (iters_out) *iters_out = h.iter;
     if (resid_out) *resid_out = std::sqrt(h.rr);

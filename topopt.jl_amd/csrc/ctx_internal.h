@@ -78,7 +78,7 @@ struct tohip_ctx {
     double *r64b = nullptr, *pcg1_part[2] = {nullptr, nullptr};
     tohip::Pcg1State *pcg1_st = nullptr, *h_pcg1 = nullptr;
     // captured PCG iteration graphs
-    hipGraphExec_t g64 = nullptr, g32 = nullptr, g64s = nullptr, g32s = nullptr;
+    hipGraphExec_t g64[tohip::kPcg1Graphs] = {}, g32 = nullptr, g32s = nullptr;
     bool have_u = false;
     bool have_load = false;  // tohip_set_load was called
     int device = 0;          // the GPU the context was created on
@@ -90,7 +90,7 @@ struct tohip_ctx {
     int conv_kind = 0;
     tohip::EnergyCrit* ecrit = nullptr;
     tohip::EnergyCrit* h_ecrit = nullptr;
-    hipGraphExec_t g64e = nullptr, g64es = nullptr;
+    hipGraphExec_t g64e[tohip::kPcg1Graphs] = {};
     // assembled K (CGAssemblySolver comparator): CSR in node-major DOF order
     int64_t csr_nnz = 0;
     int64_t* csr_rowptr = nullptr;
@@ -108,7 +108,7 @@ struct tohip_ctx {
     // solve after an operator refresh (mg_sweepM_now: it is of this operator)
     float* mg_sweepM = nullptr;
     bool mg_sweepM_now = false;
-    hipGraphExec_t gcsr = nullptr, gcsrs = nullptr;
+    hipGraphExec_t gcsr[tohip::kPcg1Graphs] = {};
     double* csr_part = nullptr;  // partial sums and states of its PCG (k_pcg1.h)
     tohip::Pcg1State* csr_st = nullptr;
     int last_replacements = 0;

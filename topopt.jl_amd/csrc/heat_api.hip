@@ -36,7 +36,7 @@ struct tohip_heat {
            *cell = nullptr, *grad = nullptr;
     double* part[2] = {nullptr, nullptr};
     Pcg1State *st = nullptr, *h_st = nullptr;
-    hipGraphExec_t graph = nullptr, graph_short = nullptr;
+    hipGraphExec_t graphs[kPcg1Graphs] = {};
     std::string err;
 };
 
@@ -188,11 +188,13 @@ int solve(tohip_heat* ctx, bool zero, double abstol, double reltol, int64_t maxi
                                ctx->t, 0, ctx->stream));
     HCK(launch_pcg1_start(n, ctx->b, zero ? nullptr : ctx->t, ctx->dinv, ctx->r[0], ctx->p[0],
                           ctx->part[0], heat_pcg_blocks(ctx->g), ctx->stream));
-    if (int rc = capture(ctx, &ctx->graph, kPcg1GraphLong)) return rc;
-    if (int rc = capture(ctx, &ctx->graph_short, kPcg1GraphShort)) return rc;
-    int64_t syncs = 0, graphs = 0;
-    HCK(pcg1_replay(ctx->graph, ctx->graph_short, ctx->st, ctx->h_st, ctx->stream, &syncs,
-                    &graphs));
+    int64_t syncs = 0, launches = 0;
+    Pcg1Schedule sch;
+    do {
+        const int k = sch.graph;
+        if (int rc = capture(ctx, &ctx->graphs[k], kPcg1GraphIters[k])) return rc;
+        HCK(pcg1_replay(ctx->graphs[k], sch, ctx->st, ctx->h_st, ctx->stream, &syncs, &launches));
+    } while (!ctx->h_st->done);
     const Pcg1State& h = *ctx->h_st;
     if (iters) *iters = h.iter;
     if (resid) *resid = std::sqrt(h.rr);
@@ -207,7 +209,7 @@ int solve(tohip_heat* ctx, bool zero, double abstol, double reltol, int64_t maxi
 
 void free_heat(tohip_heat* ctx) {
     if (!ctx) return;
-    for (hipGraphExec_t ge : {ctx->graph, ctx->graph_short})
+    for (hipGraphExec_t ge : ctx->graphs)
         if (ge) hipGraphExecDestroy(ge);
     void* bufs[] = {ctx->fixmask, ctx->fixv, ctx->x,    ctx->E,    ctx->dinv,    ctx->u,
                     ctx->r[0],    ctx->r[1], ctx->p[0], ctx->p[1], ctx->q[0],    ctx->q[1],

@@ -21,11 +21,10 @@
 // their halos), so launches alternate and a graph holds an even number.  x is
 // read and written by the owner of a node only.
 #pragma once
-#include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 #include "k_common.h"
+#include "pcg1_schedule.h"
 
 namespace tohip {
 
@@ -207,45 +206,20 @@ hipError_t launch_csr_pcg1(const Grid& g, const int64_t* rowptr, const double* v
                            double* r, double* p, double* q, const double* dinv,
                            const Pcg1State* st, Pcg1State* stn, double* part, hipStream_t s);
 
-// Iterations (launches) of the long and the short captured graph; even, so that
-// a graph starts and ends on the first set of vectors.
-constexpr int kPcg1GraphLong = 64, kPcg1GraphShort = 8;
-
-// Replays the graphs until the device has set `done`; st[0] ends up in *h.  Long
-// graphs while the residual's history predicts many iterations to go, several
-// per host check far from the end; then short ones, which leave fewer launches
-// that find nothing to do.
-inline hipError_t pcg1_replay(hipGraphExec_t lg, hipGraphExec_t sg, const Pcg1State* st,
+// Launches the graph that sch names, as often as it says, and brings st[0] to *h; sch
+// then has what comes next unless the solve is done.
+inline hipError_t pcg1_replay(hipGraphExec_t graph, Pcg1Schedule& sch, const Pcg1State* st,
                               Pcg1State* h, hipStream_t s, int64_t* syncs, int64_t* graphs) {
-    double prev_res = -1.0;
-    long long prev_it = -1;
-    bool brief = false;
-    int launches = 1;
-    for (;;) {
-        hipError_t e;
-        for (int l = 0; l < launches; ++l)
-            if ((e = hipGraphLaunch(brief ? sg : lg, s)) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(h, st, sizeof(Pcg1State), hipMemcpyDeviceToHost, s)) != hipSuccess)
-            return e;
-        if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-        *syncs += 1;
-        *graphs += launches;
-        if (h->done) return hipSuccess;
-        const double res = std::sqrt(h->rr);
-        brief = false;
-        launches = 1;
-        if (prev_res > 0 && res > 0 && h->tol > 0 && h->iter > prev_it) {
-            const double rate = std::log(res / prev_res) / double(h->iter - prev_it);
-            if (rate < 0) {
-                const double togo = std::min(std::log(h->tol / res) / rate, 1e6);
-                brief = togo < 0.75 * kPcg1GraphLong;
-                launches = brief ? std::max(1, (int)(togo / kPcg1GraphShort))
-                                 : std::max(1, std::min(4, (int)(togo / (1.5 * kPcg1GraphLong))));
-            }
-        }
-        prev_res = res;
-        prev_it = h->iter;
-    }
+    hipError_t e;
+    for (int l = 0; l < sch.launches; ++l)
+        if ((e = hipGraphLaunch(graph, s)) != hipSuccess) return e;
+    if ((e = hipMemcpyAsync(h, st, sizeof(Pcg1State), hipMemcpyDeviceToHost, s)) != hipSuccess)
+        return e;
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+    *syncs += 1;
+    *graphs += sch.launches;
+    if (!h->done) sch.next(h->iter, h->maxiter, h->rr, h->rr0, h->tol);
+    return hipSuccess;
 }
 
 }  // namespace tohip
