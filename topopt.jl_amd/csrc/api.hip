@@ -55,10 +55,13 @@ constexpr double kRestartRatio = 3.0;
 
 
 
+// (the runtime keeps the error until it is asked for, and the launchers ask: without
+// hipGetLastError here a later call, made again with memory to spare, would fail of it)
 #define CK(call)                                                                        \
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
         if (e_ != hipSuccess) {                                                         \
+            (void)hipGetLastError();                                                    \
             ctx->err = std::string(#call) + ": " + hipGetErrorString(e_);               \
             return TOHIP_ERR_HIP;                                                       \
         }                                                                               \

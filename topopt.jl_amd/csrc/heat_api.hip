@@ -48,6 +48,7 @@ thread_local std::string g_heat_error;
     do {                                                           \
         hipError_t e_ = (call);                                    \
         if (e_ != hipSuccess) {                                    \
+            (void)hipGetLastError(); /* kept until asked for */    \
             ctx->err = std::string(#call) + ": " + hipGetErrorString(e_); \
             return TOHIP_ERR_HIP;                                  \
         }                                                          \

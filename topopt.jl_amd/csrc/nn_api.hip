@@ -87,6 +87,7 @@ struct tohip_nn {
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
         if (e_ != hipSuccess) {                                                         \
+            (void)hipGetLastError(); /* kept until asked for */                         \
             nn->err = std::string(#call) + ": " + hipGetErrorString(e_);                \
             return TOHIP_ERR_HIP;                                                       \
         }                                                                               \
@@ -936,6 +937,7 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
     do {                             \
         hipError_t e_ = (call);      \
         if (e_ != hipSuccess) {      \
+            (void)hipGetLastError(); \
             fail(e_);                \
             goto done;               \
         }                            \
