@@ -444,6 +444,7 @@ void free_mg_levels(std::vector<tohip_mg_level>& lv) {
     lv.clear();
 }
 
+int mg_build(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<tohip_mg_level>& lv);
 int mg_build_levels(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<tohip_mg_level>& lv);
 
 // Largest eigenvalue of diag(Ke)^-1/2 Ke diag(Ke)^-1/2 (power iteration on a
@@ -480,7 +481,8 @@ double jacobi_bound(const std::vector<double>& Ke, int nd) {
 }
 
 // Builds the hierarchy once: levels are added while every cell count is even,
-// until the coarsest fits the one-workgroup coarse kernel.
+// until the coarsest fits the one-workgroup coarse kernel.  A set-up that fails
+// leaves the context without any of it, so that the next one starts afresh.
 int mg_setup(tohip_ctx* ctx) {
     if (!ctx->mg.empty()) return 0;
     std::vector<Grid> gs{ctx->g};
@@ -493,7 +495,31 @@ int mg_setup(tohip_ctx* ctx) {
         ctx->err = "multigrid: every cell count must be even to build a coarse level";
         return TOHIP_ERR_ARG;
     }
+    if (!ctx->ones32) {
+        std::vector<float> ones(ctx->g.ndof, 1.0f);
+        if (int rc = dalloc(ctx, &ctx->ones32, ctx->g.ndof)) return rc;
+        CK(hipMemcpyAsync(ctx->ones32, ones.data(), ones.size() * sizeof(float),
+                          hipMemcpyHostToDevice, ctx->stream));
+        CK(hipStreamSynchronize(ctx->stream));
+    }
+    const size_t held = ctx->dev_bytes;
     std::vector<tohip_mg_level> lv(gs.size());
+    const int rc = mg_build(ctx, gs, lv);
+    if (!rc) return 0;
+    hipStreamSynchronize(ctx->stream);
+    if (ctx->mg_stream) hipStreamSynchronize(ctx->mg_stream);
+    free_mg_levels(lv);
+    free_mg_levels(ctx->mg);
+    for (float** p : {&ctx->mg_M, &ctx->mg_sweepM, &ctx->mg_wd}) {
+        if (*p) hipFree(*p);
+        *p = nullptr;
+    }
+    ctx->mg_pending = false;
+    ctx->dev_bytes = held;
+    return rc;
+}
+
+int mg_build(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<tohip_mg_level>& lv) {
     // coarsest solve: Chebyshev iteration on [lbound / kappa, lbound]
     // (TOHIP_MG_ITERS / TOHIP_MG_KAPPA override the defaults for measurement)
     int iters = kMgCoarseIters;
@@ -502,11 +528,7 @@ int mg_setup(tohip_ctx* ctx) {
     const char* ek = getenv("TOHIP_MG_KAPPA");
     if (ei && atoi(ei) >= 1 && atoi(ei) <= kMgChebMax) iters = atoi(ei);
     if (ek && atof(ek) > 1.0) kappa = atof(ek);
-    if (int rc = mg_build_levels(ctx, gs, lv)) {
-        hipStreamSynchronize(ctx->stream);
-        free_mg_levels(lv);
-        return rc;
-    }
+    if (int rc = mg_build_levels(ctx, gs, lv)) return rc;
     ctx->mg_cheb = mg_chebyshev(lv.back().lbound, kappa, iters);
     ctx->mg_sweeps = kMgFallbackSweeps;
     // the coarsest solve as a dense matrix applied across the chip (rebuilt
@@ -515,20 +537,12 @@ int mg_setup(tohip_ctx* ctx) {
     const char* ed = getenv("TOHIP_MG_DENSE");
     if (mg_coarse_fits(lv.back().g) && !(ed && atoi(ed) == 0)) {
         const int64_t n = lv.back().g.ndof;
-        int rc;
-        if ((rc = dalloc(ctx, &ctx->mg_M, (size_t)(n * n)))) {
-            hipStreamSynchronize(ctx->stream);
-            free_mg_levels(lv);
-            return rc;
-        }
+        if (int rc = dalloc(ctx, &ctx->mg_M, (size_t)(n * n))) return rc;
     }
     if (mg_sweeps_dense_fits(lv.back().g) && !(ed && atoi(ed) == 0)) {
         const Grid& gc = lv.back().g;
-        if (int rc = dalloc(ctx, &ctx->mg_sweepM, (size_t)gc.ndof * mg_sweeps_dense_ld(gc))) {
-            hipStreamSynchronize(ctx->stream);
-            free_mg_levels(lv);
+        if (int rc = dalloc(ctx, &ctx->mg_sweepM, (size_t)gc.ndof * mg_sweeps_dense_ld(gc)))
             return rc;
-        }
     }
     // smoother weights in device memory: the bound's weight until the first
     // estimate; TOHIP_MG_WADAPT=0 (or a forced TOHIP_MG_OMEGA) keeps it
@@ -545,24 +559,16 @@ int mg_setup(tohip_ctx* ctx) {
             hw[4 * l + 1] = 1.f;
         }
         hw[4 * nl] = 1.f;
-        // the level count is fixed per context: a set-up retried after a
-        // failure reuses the array
-        int rc = ctx->mg_wd ? 0 : dalloc(ctx, &ctx->mg_wd, hw.size());
-        for (int l = 0; rc == 0 && l < nl; ++l) {
+        if (int rc = dalloc(ctx, &ctx->mg_wd, hw.size())) return rc;
+        for (int l = 0; l < nl; ++l) {
             lv[l].wd = ctx->mg_wd + 4 * l;
-            if (l < nl - 1 && ctx->mg_wadapt && (rc = dalloc(ctx, &lv[l].pw, lv[l].g.ndof)) == 0)
-                if (launch_mg_fill_start(lv[l].g.ndof, lv[l].pw, ctx->stream) != hipSuccess)
-                    rc = TOHIP_ERR_HIP;
+            if (l == nl - 1 || !ctx->mg_wadapt) continue;
+            if (int rc = dalloc(ctx, &lv[l].pw, lv[l].g.ndof)) return rc;
+            CK(launch_mg_fill_start(lv[l].g.ndof, lv[l].pw, ctx->stream));
         }
-        if (rc == 0 && hipMemcpyAsync(ctx->mg_wd, hw.data(), hw.size() * sizeof(float),
-                                      hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
-            rc = TOHIP_ERR_HIP;
-        if (rc == 0 && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = TOHIP_ERR_HIP;
-        if (rc) {
-            hipStreamSynchronize(ctx->stream);
-            free_mg_levels(lv);
-            return rc;
-        }
+        CK(hipMemcpyAsync(ctx->mg_wd, hw.data(), hw.size() * sizeof(float), hipMemcpyHostToDevice,
+                          ctx->stream));
+        CK(hipStreamSynchronize(ctx->stream));
     }
     ctx->mg = std::move(lv);
     if (int rc = mg_refresh(ctx)) return rc;
@@ -612,13 +618,6 @@ int mg_build_levels(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<toh
         }
         int rc = 0;
         if ((rc = dalloc(ctx, &L.x, L.g.ndof)) || (rc = dalloc(ctx, &L.rz, L.g.ndof))) return rc;
-    }
-    if (!ctx->ones32) {
-        std::vector<float> ones(ctx->g.ndof, 1.0f);
-        if (int rc = dalloc(ctx, &ctx->ones32, ctx->g.ndof)) return rc;
-        CK(hipMemcpyAsync(ctx->ones32, ones.data(), ones.size() * sizeof(float),
-                          hipMemcpyHostToDevice, ctx->stream));
-        CK(hipStreamSynchronize(ctx->stream));
     }
     return 0;
 }
