@@ -1,6 +1,9 @@
 /* TEST INFRASTRUCTURE ONLY: the HIP entry points that libtopopt_hip imports, on host
  * memory: allocations are calloc'ed and counted, copies are memcpy, kernels and graphs
- * do nothing.  stub_fail_in(n) makes the n-th allocation from now fail (0: none). */
+ * do nothing.  stub_fail_in(n) makes the n-th allocation from now fail (0: none),
+ * stub_fail_graphs(1) every launch of a graph (nothing else ends an iteration here).
+ * Memory starts as doubles of 1. */
+#include <stddef.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -12,7 +15,10 @@ struct block {
     char pad[48];
 };
 
+static int g_fail_graphs;
+
 void stub_fail_in(long n) { g_fail_in = n; }
+void stub_fail_graphs(int f) { g_fail_graphs = f; }
 long stub_live(void) { return g_live; }
 long stub_bytes(void) { return g_bytes; }
 long stub_count(void) { return g_count; }
@@ -23,6 +29,7 @@ int hipMalloc(void** p, size_t n) {
     struct block* b = calloc(1, sizeof(struct block) + n);
     if (!b) return g_last = 2;
     b->n = n;
+    for (size_t i = 0; i < n / sizeof(double); ++i) ((double*)(b + 1))[i] = 1.0;
     g_live += 1;
     g_bytes += (long)n;
     *p = b + 1;
@@ -93,7 +100,7 @@ int hipStreamEndCapture(void* s, void** g) { return handle(g); }
 int hipGraphInstantiate(void** e, void* g, void** n, char* l, size_t z) { return handle(e); }
 int hipGraphDestroy(void* g) { return 0; }
 int hipGraphExecDestroy(void* e) { return 0; }
-int hipGraphLaunch(void* e, void* s) { return 0; }
+int hipGraphLaunch(void* e, void* s) { return g_fail_graphs ? (g_last = 719) : 0; }
 int hipEventCreate(void** e) { return handle(e); }
 int hipEventCreateWithFlags(void** e, unsigned f) { return handle(e); }
 int hipEventDestroy(void* e) { return 0; }

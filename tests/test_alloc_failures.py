@@ -83,6 +83,77 @@ SWEEP = SETUP + textwrap.dedent("""
     print(json.dumps(dict(rows=rows, live=stub.stub_live())), flush=True)
 """)
 
+# Calls that make their buffers on first use.  Graph launches fail, which ends the
+# solver runs after they have all that they need.
+GROUPS = SETUP + textwrap.dedent("""
+    stub.stub_fail_graphs(1)
+
+    def held():
+        b = C.c_int64()
+        assert L.tohip_memory(c.ptr, C.byref(b), None, None) == 0
+        return b.value
+
+    def start():
+        global c, x
+        c = context()
+        c.lib.tohip_set_densities(c.ptr, _lib.dptr(x))
+        c.lib.tohip_set_load(c.ptr, _lib.dptr(r))
+        assert c.lib.tohip_filter_setup(c.ptr, 1.5) == 0
+
+    def csr():
+        return L.tohip_csr_matvec(c.ptr, _lib.dptr(r), _lib.dptr(z)), 0
+
+    def solve():
+        it, rs = C.c_int64(), C.c_double()
+        return L.tohip_solve(c.ptr, _lib.dptr(r), None, 0.0, 1e-8, 10, 1, 0, C.byref(it),
+                             C.byref(rs)), -2
+
+    def mma():
+        o = _lib.SimpOpts(volfrac=0.5, rmin=1.5, move=0.2, oc_tol=1e-9, rel_tol=1e-8,
+                          iterations=1, maxiter=10, inner_rel_tol=0.1)
+        m = _lib.MmaOpts(s_init=0.5, s_incr=1.2, s_decr=0.7)
+        h = np.empty(4), np.empty(4, np.int64), np.empty(4)
+        return L.tohip_simp_run_mma(c.ptr, C.byref(o), C.byref(m), _lib.dptr(x.copy()),
+                                    _lib.dptr(h[0]), h[1].ctypes.data_as(C.POINTER(C.c_int64)), _lib.dptr(h[2])), -2
+
+    def beso():
+        o = _lib.BesoOpts(maxiter=2, vol_limit=0.5, rmin=1.5, er=0.02, tol=1e-4, sens_tol=1e-6,
+                          k=4, penalty_p=3.0, rel_tol=1e-8, pcg_maxiter=10)
+        res, out, hist = _lib.BesoResultC(), np.empty(c.ncells), np.empty(4)
+        return L.tohip_beso_run(c.ptr, C.byref(o), _lib.dptr(np.ones(c.ncells)), None,
+                                _lib.dptr(out), C.byref(res), _lib.dptr(hist)), -2
+
+    def filt():
+        return L.tohip_filter_setup(c.ptr, 2.5), 0
+
+    for name, f in dict(csr=csr, solve=solve, mma=mma, beso=beso, filt=filt).items():
+        start()
+        f()
+        whole = held()
+        start()
+        b0, k = held(), 0
+        while True:
+            k += 1
+            stub.stub_fail_in(k)
+            rc, good = f()
+            stub.stub_fail_in(0)
+            err = L.tohip_last_error(c.ptr).decode()
+            if k > 40 or rc == good and (rc == 0 or "out of memory" not in err):
+                break
+            assert rc == -2 and "out of memory" in err, (name, k, rc, err)
+            rc, good = f() if k % 2 == 0 else (good, good)
+            assert rc == good, (name, k, rc, L.tohip_last_error(c.ptr).decode())
+            if k % 2 == 0:
+                assert held() == whole, (name, k, held(), whole)
+                start()
+        assert k > 2 and k < 40, (name, k)
+        print(name, k, whole - b0)
+    del c
+    import gc
+    gc.collect()
+    assert stub.stub_live() == 0, stub.stub_live()
+""")
+
 
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
@@ -113,3 +184,11 @@ def test_multigrid_setup(T, stub, nels):
         assert rc == (0 if k == len(out["rows"]) - 1 else -2), (k, rc)
         assert over == 0 and rc2 == 0, (k, over, rc2)
     assert out["live"] == 0
+
+
+def test_groups_of_buffers(T, stub):
+    """Buffers made on first use: when one of them cannot be had, the call made again gets
+    the rest, and no more."""
+    p = subprocess.run([sys.executable, "-c", GROUPS, stub, ROOT, "[6, 4, 4]"],
+                       stdout=subprocess.PIPE, stderr=subprocess.PIPE, timeout=120)
+    assert p.returncode == 0, p.stdout.decode() + p.stderr.decode()[-2000:]

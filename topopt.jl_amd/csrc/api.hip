@@ -233,6 +233,12 @@ int dalloc(tohip_ctx* ctx, T** p, size_t n) {
     ctx->dev_bytes += n * sizeof(T);
     return 0;
 }
+// For buffers made on first use, several of them: the ones that an earlier attempt got
+// are kept.  What says that the group is whole is set after the last.
+template <typename T>
+int dneed(tohip_ctx* ctx, T** p, size_t n) {
+    return *p ? 0 : dalloc(ctx, p, n);
+}
 
 bool all_finite(const double* v, int64_t n) {
     for (int64_t i = 0; i < n; ++i)
@@ -1225,14 +1231,23 @@ int build_filter(tohip_ctx* ctx, double rmin) {
         ctx->err = "DensityFilterFun: rmin too large for the stencil table";
         return TOHIP_ERR_ARG;
     }
+    // the new tables before the old ones go: what was set up stays if they don't fit
+    int* new_offs = nullptr;
+    double* new_wts = nullptr;
+    if (int rc = dalloc(ctx, &new_offs, offs.size())) return rc;
+    if (int rc = dalloc(ctx, &new_wts, wts.size())) {
+        hipFree(new_offs);
+        ctx->dev_bytes -= offs.size() * sizeof(int);
+        return rc;
+    }
     if (ctx->f_offs) {
         CK(hipFree(ctx->f_offs));
         CK(hipFree(ctx->f_wts));
-        ctx->f_offs = nullptr;
-        ctx->f_wts = nullptr;
+        ctx->dev_bytes -= (size_t)ctx->f_count * (3 * sizeof(int) + sizeof(double));
     }
-    if (int rc = dalloc(ctx, &ctx->f_offs, offs.size())) return rc;
-    if (int rc = dalloc(ctx, &ctx->f_wts, wts.size())) return rc;
+    ctx->f_offs = new_offs;
+    ctx->f_wts = new_wts;
+    ctx->f_rmin = -1;
     CK(hipMemcpyAsync(ctx->f_offs, offs.data(), offs.size() * sizeof(int), hipMemcpyHostToDevice,
                       ctx->stream));
     CK(hipMemcpyAsync(ctx->f_wts, wts.data(), wts.size() * sizeof(double), hipMemcpyHostToDevice,
@@ -1480,7 +1495,7 @@ int csr_assemble(tohip_ctx* ctx, int safe, int jacobi) {
     const Grid& g = ctx->g;
     const int dim = g.dim;
     bool pattern = false;
-    if (!ctx->csr_rowptr) {
+    if (!ctx->csr_nnz) {
         std::vector<int64_t> rowptr(g.ndof + 1, 0);
         for (int64_t n = 0; n < g.nnodes; ++n) {
             const int i = (int)(n % g.NX), j = (int)((n / g.NX) % g.NY);
@@ -1499,10 +1514,10 @@ int csr_assemble(tohip_ctx* ctx, int safe, int jacobi) {
         std::vector<double> Ke;
         element_stiffness_bits(dim, ctx->E, ctx->nu, ctx->h, Ke);
         int rc;
-        if ((rc = dalloc(ctx, &ctx->csr_rowptr, g.ndof + 1)) ||
-            (rc = dalloc(ctx, &ctx->csr_cols, nnz)) || (rc = dalloc(ctx, &ctx->csr_vals, nnz)) ||
-            (rc = dalloc(ctx, &ctx->csr_diag, g.ndof)) || (rc = dalloc(ctx, &ctx->csr_dinv, g.ndof)) ||
-            (rc = dalloc(ctx, &ctx->csr_ke, nd * nd)) || (rc = dalloc(ctx, &ctx->csr_md, 3)))
+        if ((rc = dneed(ctx, &ctx->csr_rowptr, g.ndof + 1)) ||
+            (rc = dneed(ctx, &ctx->csr_cols, nnz)) || (rc = dneed(ctx, &ctx->csr_vals, nnz)) ||
+            (rc = dneed(ctx, &ctx->csr_diag, g.ndof)) || (rc = dneed(ctx, &ctx->csr_dinv, g.ndof)) ||
+            (rc = dneed(ctx, &ctx->csr_ke, nd * nd)) || (rc = dneed(ctx, &ctx->csr_md, 3)))
             return rc;
         CK(hipMemcpyAsync(ctx->csr_rowptr, rowptr.data(), rowptr.size() * sizeof(int64_t),
                           hipMemcpyHostToDevice, ctx->stream));
@@ -1764,7 +1779,7 @@ int tohip_csr_assemble(tohip_ctx* ctx, int safe) {
 int tohip_csr_info(const tohip_ctx* cctx, int64_t* nnz, int64_t* bytes, double* meandiag) {
     if (!cctx) return TOHIP_ERR_ARG;
     tohip_ctx* ctx = const_cast<tohip_ctx*>(cctx);  // for the error message only
-    if (!ctx->csr_rowptr) {
+    if (!ctx->csr_nnz) {
         ctx->err = "tohip_csr_info: no assembled matrix";
         return TOHIP_ERR_STATE;
     }
@@ -1783,7 +1798,7 @@ int tohip_csr_info(const tohip_ctx* cctx, int64_t* nnz, int64_t* bytes, double* 
 int tohip_csr_download(const tohip_ctx* cctx, int64_t* rowptr, int* cols, double* vals) {
     if (!cctx || !rowptr || !cols || !vals) return TOHIP_ERR_ARG;
     tohip_ctx* ctx = const_cast<tohip_ctx*>(cctx);  // for the error message only
-    if (!ctx->csr_rowptr) {
+    if (!ctx->csr_nnz) {
         ctx->err = "tohip_csr_download: no assembled matrix";
         return TOHIP_ERR_STATE;
     }
@@ -2211,11 +2226,11 @@ int simp_run_impl(tohip_ctx* ctx, const tohip_simp_opts* o, const tohip_mma_opts
         ctx->nn_misses = 0;
         ctx->nn_off = false;
     }
-    if (mma && !ctx->mma_st) {
+    if (mma && !ctx->h_mma) {
         int rc;
-        if ((rc = dalloc(ctx, &ctx->mma_L, nC)) || (rc = dalloc(ctx, &ctx->mma_U, nC)) ||
-            (rc = dalloc(ctx, &ctx->mma_x1, nC)) || (rc = dalloc(ctx, &ctx->mma_x2, nC)) ||
-            (rc = dalloc(ctx, &ctx->mma_st, 1)))
+        if ((rc = dneed(ctx, &ctx->mma_L, nC)) || (rc = dneed(ctx, &ctx->mma_U, nC)) ||
+            (rc = dneed(ctx, &ctx->mma_x1, nC)) || (rc = dneed(ctx, &ctx->mma_x2, nC)) ||
+            (rc = dneed(ctx, &ctx->mma_st, 1)))
             return rc;
         CK(hipHostMalloc((void**)&ctx->h_mma, sizeof(MmaState), hipHostMallocDefault));
         ctx->mma_iter = 0;
@@ -2349,10 +2364,10 @@ int tohip_beso_run(tohip_ctx* ctx, const tohip_beso_opts* o, const double* x0,
         ctx->err = "tohip_beso_run: the load vector is zero (tohip_set_load)";
         return TOHIP_ERR_STATE;
     }
-    if (!ctx->beso_st) {
+    if (!ctx->h_beso) {
         int rc = 0;
-        if ((rc = dalloc(ctx, &ctx->beso_sens[0], nC)) || (rc = dalloc(ctx, &ctx->beso_sens[1], nC)) ||
-            (rc = dalloc(ctx, &ctx->beso_mask, nC)) || (rc = dalloc(ctx, &ctx->beso_st, 1)))
+        if ((rc = dneed(ctx, &ctx->beso_sens[0], nC)) || (rc = dneed(ctx, &ctx->beso_sens[1], nC)) ||
+            (rc = dneed(ctx, &ctx->beso_mask, nC)) || (rc = dneed(ctx, &ctx->beso_st, 1)))
             return rc;
         CK(hipHostMalloc((void**)&ctx->h_beso, sizeof(BesoState), hipHostMallocDefault));
     }
