@@ -170,8 +170,9 @@ int tohip_solve(tohip_ctx* ctx, const double* f, double* u, double abstol, doubl
 
 /* z = M r for the multigrid preconditioner of TOHIP_MIXED_MG at the current
  * densities (FP32 V-cycle; r and z in the caller's DOF order, FP64 at the
- * boundary).  No reference counterpart: it exposes the preconditioner for
- * inspection and testing. */
+ * boundary).  A coarsest level of damped Jacobi sweeps is applied by sweeps, which
+ * the solves apply as their matrix: the same operator, other FP32 roundings.  No
+ * reference counterpart: it exposes the preconditioner for inspection and testing. */
 int tohip_mg_apply(tohip_ctx* ctx, const double* r, double* z);
 
 /* Damped-Jacobi weights of the multigrid levels (omega[l]) and the current

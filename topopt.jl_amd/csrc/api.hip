@@ -634,7 +634,7 @@ int mg_build_levels(tohip_ctx* ctx, const std::vector<Grid>& gs, std::vector<toh
 // first applies the pending PCG update to r and x (the cycle then runs on the
 // new residual, which it writes to upd->rnew).
 // `dense`: apply a coarsest level of sweeps as its matrix (the solves' graphs, which
-// run after mg_solve_ready; elsewhere while it is of the current operator).
+// run after mg_solve_ready); one cycle alone runs the sweeps.
 hipError_t launch_vcycle(tohip_ctx* ctx, const float* r, const PcgScalars* sc, double* part,
                          int* nb_part, const MgFusedUpdate* upd = nullptr, bool dense = true) {
     std::vector<tohip_mg_level>& M = ctx->mg;
@@ -1892,7 +1892,8 @@ int tohip_mg_apply(tohip_ctx* ctx, const double* r, double* z) {
     if (int rc = mg_setup(ctx)) return rc;
     CK(launch_f64_to_f32(ctx->g.ndof, ctx->r64, ctx->b32, ctx->stream));
     if (int rc = mg_join(ctx)) return rc;
-    CK(launch_vcycle(ctx, ctx->b32, nullptr, nullptr, nullptr, nullptr, ctx->mg_sweepM_now));
+    // (by sweeps whether or not a solve has built their matrix: the same bits every time)
+    CK(launch_vcycle(ctx, ctx->b32, nullptr, nullptr, nullptr, nullptr, false));
     CK(launch_f32_to_f64(ctx->g.ndof, ctx->mg[0].rz, ctx->t64, ctx->stream));
     return download_dofs(ctx, ctx->t64, z);
 }
