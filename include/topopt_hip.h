@@ -331,6 +331,9 @@ void tohip_nn_destroy(tohip_nn* nn);
 int64_t tohip_nn_num_params(const tohip_nn* nn);
 int tohip_nn_get_params(tohip_nn* nn, float* params);
 int tohip_nn_set_params(tohip_nn* nn, const float* params);
+/* Gradient of the last training step's loss, in the order of the parameters (0 before
+ * the first), for inspection and testing. */
+int tohip_nn_get_gradient(tohip_nn* nn, float* grad);
 /* Training pair: filtered densities (cells), load and displacement (DOFs). */
 int tohip_nn_add_sample(tohip_nn* nn, const double* xphys, const double* f, const double* u);
 int tohip_nn_clear_samples(tohip_nn* nn);

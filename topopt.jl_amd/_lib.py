@@ -157,6 +157,7 @@ SIGNATURES = {
     "tohip_nn_destroy": (None, [C.c_void_p]),
     "tohip_nn_num_params": (C.c_int64, [C.c_void_p]),
     "tohip_nn_get_params": (C.c_int, [C.c_void_p, C.POINTER(C.c_float)]),
+    "tohip_nn_get_gradient": (C.c_int, [C.c_void_p, C.POINTER(C.c_float)]),
     "tohip_nn_set_params": (C.c_int, [C.c_void_p, C.POINTER(C.c_float)]),
     "tohip_nn_add_sample": (C.c_int, [C.c_void_p, _dp, _dp, _dp]),
     "tohip_nn_clear_samples": (C.c_int, [C.c_void_p]),

@@ -721,6 +721,14 @@ int tohip_nn_get_params(tohip_nn* nn, float* out) {
     return 0;
 }
 
+int tohip_nn_get_gradient(tohip_nn* nn, float* out) {
+    if (!nn || !out) return TOHIP_ERR_ARG;
+    NCK(hipMemcpyAsync(out, nn->grads, nn->nparam * sizeof(float), hipMemcpyDeviceToHost,
+                       nn->stream));
+    NCK(hipStreamSynchronize(nn->stream));
+    return 0;
+}
+
 int tohip_nn_set_params(tohip_nn* nn, const float* in) {
     if (!nn || !in) return TOHIP_ERR_ARG;
     NCK(hipMemcpyAsync(nn->params, in, nn->nparam * sizeof(float), hipMemcpyHostToDevice,

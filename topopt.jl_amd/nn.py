@@ -85,6 +85,12 @@ class WarmStartNet:
         self._check(self.lib.tohip_nn_get_params(self.ptr, _fptr(p)), "get_params")
         return p
 
+    def get_gradient(self) -> np.ndarray:
+        """Gradient of the last training step's loss, in the order of the parameters."""
+        g = np.empty(self.nparams, np.float32)
+        self._check(self.lib.tohip_nn_get_gradient(self.ptr, _fptr(g)), "get_gradient")
+        return g
+
     def set_params(self, p):
         p = np.ascontiguousarray(p, np.float32)
         if p.size != self.nparams:
