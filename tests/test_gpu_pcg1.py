@@ -238,3 +238,66 @@ def test_iteration_time_grows_with_the_grid(T, gpu):
         he.append(per_iteration(lambda n: s(rhs=b, maxiter=n)))
     assert el[1] < 4.8 * el[0], (el[0] / 256, el[1] / 256)
     assert he[1] < 4.8 * he[0], (he[0] / 256, he[1] / 256)
+
+
+def test_heat_rows_past_32_bit_offsets(T, gpu):
+    """A grid whose 17 rows of a column span 4 GiB: 31,580,641 x 1 cells.  Operator and
+    three iterations on loads in three windows (the last one at the far end), against the
+    windows alone."""
+    import ctypes as C
+    import scipy.sparse as sp
+    from oracle import heat_oracle as H
+    from topopt_jl_amd import _lib
+    nx, wn = 31580641, 40
+    NX, n = nx + 1, 2 * (nx + 1)
+    assert NX * 17 * 8 >= 2**32
+    lib = T.load_library()
+    ptr, order = C.c_void_p(), np.arange(1, n + 1)
+    fixed = np.zeros(n, np.uint8)
+    fixed[0] = 1
+    h = np.array([1.0, 0.7])
+    assert lib.tohip_heat_create(C.byref(ptr), 2, _lib.i64ptr(np.array([nx, 1])), _lib.dptr(h), 1.3,
+                                 1e-3, 3.0, 1, _lib.i64ptr(order), _lib.u8ptr(fixed), None) == 0
+    del order, fixed
+    try:
+        Ke = H.heat_ke(2, tuple(h), 1.3)  # densities are 1 from the start
+        c = np.arange(wn)
+        dofs = np.stack([c, c + 1, c + wn + 2, c + wn + 1], 1)  # window nodes, x fastest
+        K = sp.csr_matrix((np.tile(Ke.ravel(), wn), (np.repeat(dofs, 4, axis=1).ravel(),
+                                                     np.tile(dofs, (1, 4)).ravel()))).toarray()
+        starts = (1000, 2**24 - 20, nx - wn)
+        at = [np.concatenate([s + np.arange(wn + 1), NX + s + np.arange(wn + 1)]) for s in starts]
+        g = np.random.default_rng(0)
+        b, loads = np.zeros(n), []
+        for k, idx in enumerate(at):
+            f = np.zeros(2 * (wn + 1))
+            # away from the window's ends, and at the grid's own
+            on = np.arange(wn - 9, wn + 1) if k == 2 else np.arange(15, 25)
+            f[np.concatenate([on, wn + 1 + on])] = g.standard_normal(20)
+            b[idx] = f
+            loads.append(f)
+        y = np.empty(n)
+        assert lib.tohip_heat_matvec(ptr, _lib.dptr(b), _lib.dptr(y)) == 0
+        for idx, f in zip(at, loads):
+            assert np.linalg.norm(y[idx] - K @ f) < 1e-14 * np.linalg.norm(K @ f)
+            y[idx] = 0.0
+        assert not y.any()
+        u, it, res = np.zeros(n), C.c_int64(), C.c_double()
+        assert lib.tohip_heat_solve(ptr, _lib.dptr(b), _lib.dptr(u), 0.0, 1e-30, 3, 1, 0,
+                                    C.byref(it), C.byref(res)) == 1
+        r, p = np.stack(loads), 0.0  # a row a window
+        x, diag, rho_prev = np.zeros_like(r), K.diagonal(), 1.0
+        for _ in range(3):
+            z = r / diag
+            rho = (r * z).sum()
+            p = z + rho / rho_prev * p
+            q = p @ K
+            a = rho / (p * q).sum()
+            x, r, rho_prev = x + a * p, r - a * q, rho
+        assert it.value == 3
+        for idx, v in zip(at, x):
+            assert np.linalg.norm(u[idx] - v) < 1e-12 * np.linalg.norm(v)
+            u[idx] = 0.0
+        assert not u.any()
+    finally:
+        lib.tohip_heat_destroy(ptr)
