@@ -1,6 +1,7 @@
 """GPU tests of the caller's DOF order at the entry points: a context with a
 shuffled order against one in the library's own, bit for bit, and refused values on
-both sides of the length (2^16) where the check moves from the host to the device."""
+both sides of the lengths where the check (2^16) and the way back to the caller's order
+(2^15) move from the host to the device."""
 import ctypes as C
 
 import numpy as np
@@ -8,7 +9,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-GRIDS = [(1, 1), (13, 7), (180, 180), (181, 181), (3, 2, 2), (28, 27, 27)]
+GRIDS = [(1, 1), (13, 7), (180, 180), (181, 181), (3, 2, 2), (28, 27, 27), (127, 127), (128, 127)]
 
 
 def _contexts(T, nels):
@@ -100,7 +101,7 @@ def test_refused_values(T, gpu, nels, bad):
     assert lib.tohip_get_u(c.ptr, ptr(now)) == 0 and np.array_equal(now, u)
 
 
-@pytest.mark.parametrize("nels", [(12, 9), (255, 254), (256, 255), (40, 40, 39)])
+@pytest.mark.parametrize("nels", [(12, 9), (255, 254), (256, 255), (40, 40, 39), (181, 179), (181, 180)])
 def test_heat_values(T, gpu, nels):
     """Heat: refused values on both sides of the rule; the temperature comes back in
     the order it was given (no iterations: the guess with its prescribed values)."""

@@ -278,6 +278,15 @@ int upload_dofs(tohip_ctx* ctx, const double* host, double* dev) {
 
 // dev must not be q64.
 int download_dofs(tohip_ctx* ctx, const double* dev, double* host) {
+    if (!ctx->perm_host.empty()) {
+        const size_t n = ctx->perm_host.size();
+        std::vector<double> tmp(n);
+        CK(hipMemcpyAsync(tmp.data(), dev, n * sizeof(double), hipMemcpyDeviceToHost,
+                          ctx->stream));
+        CK(hipStreamSynchronize(ctx->stream));
+        for (size_t i = 0; i < n; ++i) host[ctx->perm_host[i]] = tmp[i];
+        return 0;
+    }
     if (ctx->perm) {
         CK(launch_order_scatter(ctx->g.ndof, ctx->perm, dev, ctx->q64, ctx->stream));
         dev = ctx->q64;
@@ -1468,6 +1477,7 @@ int create_impl(tohip_ctx* ctx, int dim, const int64_t* nels, const double* h, d
         CK(hipMemcpyAsync(ctx->perm, perm.data(), nD * sizeof(int), hipMemcpyHostToDevice,
                           ctx->stream));
     CK(hipStreamSynchronize(ctx->stream));
+    if (node_dofs && nD <= kHostOrderMax) ctx->perm_host = std::move(perm);
     ctx->nodemask = std::move(nodemask);
     CK(hipMemsetAsync(ctx->sc64, 0, sizeof(PcgScalars), ctx->stream));
     CK(hipMemsetAsync(ctx->sc32, 0, sizeof(PcgScalars), ctx->stream));

@@ -39,6 +39,7 @@ struct tohip_ctx {
     tohip::ElemOp<double> op64{};
     tohip::ElemOp<float> op32{};
     int* perm = nullptr;  // internal DOF -> caller DOF (0-based), device; null = identity
+    std::vector<int> perm_host;  // the same up to kHostOrderMax DOFs, else empty
     std::vector<uint8_t> fixed_internal;
     hipStream_t stream = nullptr;
     std::string err;

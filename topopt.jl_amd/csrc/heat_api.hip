@@ -27,6 +27,7 @@ struct tohip_heat {
     double meandiag = 0.0;
     bool inhom = false;              // some prescribed temperature is nonzero
     int* node_dof = nullptr;         // node id -> caller DOF (0-based), device
+    std::vector<int> node_dof_host;  // the same up to kHostOrderMax nodes, else empty
     hipStream_t stream = nullptr;
     uint8_t* fixmask = nullptr;
     double *fixv = nullptr, *x = nullptr, *E = nullptr, *dinv = nullptr;
@@ -131,6 +132,14 @@ int upload_nodes(tohip_heat* ctx, const double* host, double* dev, bool* finite 
 // dev must not be r[1].
 int download_nodes(tohip_heat* ctx, const double* dev, double* host) {
     const int64_t n = ctx->g.nnodes;
+    if (!ctx->node_dof_host.empty()) {
+        std::vector<double> tmp(n);
+        HCK(hipMemcpyAsync(tmp.data(), dev, n * sizeof(double), hipMemcpyDeviceToHost,
+                           ctx->stream));
+        HCK(hipStreamSynchronize(ctx->stream));
+        for (int64_t i = 0; i < n; ++i) host[ctx->node_dof_host[i]] = tmp[i];
+        return 0;
+    }
     HCK(launch_order_scatter(n, ctx->node_dof, dev, ctx->r[1], ctx->stream));
     HCK(hipMemcpyAsync(host, ctx->r[1], n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HCK(hipStreamSynchronize(ctx->stream));
@@ -323,6 +332,7 @@ int create_heat(tohip_heat* ctx, int dim, const int64_t* nels, const double* h, 
     HCK(hipMemsetAsync(ctx->u, 0, n * sizeof(double), ctx->stream));
     if ((rc = refresh(ctx))) return rc;
     HCK(hipStreamSynchronize(ctx->stream));
+    if (n <= kHostOrderMax) ctx->node_dof_host = std::move(node_dof);
     return 0;
 }
 

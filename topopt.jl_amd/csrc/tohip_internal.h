@@ -257,6 +257,11 @@ hipError_t values_check(int64_t n, const double* x, double* partials, long doubl
 // load set from the host takes 40 us against 63 us for 8,450 values, 83 against 82
 // for 132,098, 6.3 ms against 3.5 for 12.8 million (MI355X).
 constexpr int64_t kHostCheckMax = 1 << 16;
+// Vectors up to this length are brought back to the caller's order on the host, longer
+// ones on the device before the copy: a displacement is read in 18 us against 27 for
+// 13,202 values, 27 against 32 for 27,783, 50 against 44 for 64,722.  (Setting one
+// takes the same on both sides there: its kernel runs while the host goes on.)
+constexpr int64_t kHostOrderMax = 1 << 15;
 
 // Sum-reductions finished by a one-block kernel: out[v] = sum_b part[b*nv+v].
 hipError_t launch_reduce(const double* partials, int nb, int nv, double* out, hipStream_t s);
