@@ -110,7 +110,7 @@ def run_path(T, name, nels, precision, warm, steps, warmup, volfrac, rmin, rel_t
 
 ALL_KERNELS = ("matvec64", "matvec32", "pcg64", "pcg32", "update64", "update32", "filter",
                "filter_t", "energy", "oc", "copy64", "mg_pre", "mg_restrict", "mg_coarse",
-               "mg_post", "vcycle", "csr_spmv")
+               "mg_post", "vcycle", "csr_spmv", "pcg1_64")
 
 
 def kernel_times(T, s, prob, reps, rmin, names=ALL_KERNELS):
@@ -168,14 +168,18 @@ def algorithmic_bytes(prob):
         # read x, b, D^-1, E, mask, the coarse correction; write z
         "mg_post": 4 * 4 * nd + 4 * nc + nn + 4 * nd1,
         "matvec64": mv(8), "matvec32": mv(4),
-        "pcg64": mv(8) + 3 * 8 * nd, "pcg32": mv(4) + 3 * 4 * nd,  # + read r, dinv; write p
+        # + read r, dinv; write p (pcg64 and update64: the multigrid-preconditioned FP64
+        # solver; the Jacobi one's iteration is pcg1_64)
+        "pcg64": mv(8) + 3 * 8 * nd, "pcg32": mv(4) + 3 * 4 * nd,
         "update64": 7 * 8 * nd, "update32": 7 * 4 * nd,  # x,r rw; p,q,dinv read
+        # read x, r, p, q, dinv, E, mask; write x, r, p, q
+        "pcg1_64": 9 * 8 * nd + 8 * nc + nn,
         "filter": 2 * 8 * nc, "filter_t": 2 * 8 * nc,
         "energy": 8 * nd + 3 * 8 * nc,  # read u, x~; write ce, grad
         "copy64": 16 * nd,  # plain copy: the counter-scaling reference
-        # assembled K: every stored entry (value + column), the row pointers,
-        # x read once, y written
-        "csr_spmv": 12 * csr_nnz(prob.nels) + 8 * (nd + 1) + 16 * nd,
+        # assembled K: every stored value (the columns follow from the grid), a row
+        # pointer a node, x read once, y written
+        "csr_spmv": 8 * csr_nnz(prob.nels) + 8 * nn + 16 * nd,
     }
 
 

@@ -365,9 +365,9 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
  * tohip_set_densities / tohip_matvec / tohip_filter_setup). */
 #define TOHIP_K_MATVEC64 0   /* y = K x, FP64                          */
 #define TOHIP_K_MATVEC32 1   /* y = K x, FP32                          */
-#define TOHIP_K_PCG64 2      /* fused p = z + beta p, q = K p, p.q FP64 */
+#define TOHIP_K_PCG64 2      /* fused p = z + beta p, q = K p, p.q FP64 (TOHIP_FP64_MG) */
 #define TOHIP_K_PCG32 3      /* same, FP32 vectors, FP64 reductions     */
-#define TOHIP_K_UPDATE64 4   /* x += a p, r -= a q, r.z, r.r  FP64      */
+#define TOHIP_K_UPDATE64 4   /* x += a p, r -= a q, r.z, r.r  FP64 (TOHIP_FP64_MG) */
 #define TOHIP_K_UPDATE32 5   /* same, FP32 vectors                      */
 #define TOHIP_K_FILTER 6     /* x~ = J x                                */
 #define TOHIP_K_FILTER_T 7   /* J^T y                                   */
@@ -381,6 +381,7 @@ int tohip_nn_conv_check(int B, const int* dims, int cin, int cout, int k, int pa
 #define TOHIP_K_MG_POST 14    /* finest level: x += P xc, z = x + w D^-1 (b - K x) */
 #define TOHIP_K_VCYCLE 15     /* one whole V-cycle (every launch of it)         */
 #define TOHIP_K_CSR_SPMV 16   /* assembled K (CSR) times x, FP64 (assembles K first) */
+#define TOHIP_K_PCG1_64 17    /* a whole FP64 Jacobi PCG iteration, one launch (TOHIP_FP64) */
 int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us);
 
 /* ---- BESO (src/Algorithms/beso.jl) ---------------------------------------

@@ -175,7 +175,7 @@ SIGNATURES = {
 # tohip_bench_kernel ids
 KERNELS = {"matvec64": 0, "matvec32": 1, "pcg64": 2, "pcg32": 3, "update64": 4, "update32": 5,
            "filter": 6, "filter_t": 7, "energy": 8, "oc": 9, "copy64": 10, "mg_pre": 11,
-           "mg_restrict": 12, "mg_coarse": 13, "mg_post": 14, "vcycle": 15, "csr_spmv": 16}
+           "mg_restrict": 12, "mg_coarse": 13, "mg_post": 14, "vcycle": 15, "csr_spmv": 16, "pcg1_64": 17}
 
 _lib = None
 

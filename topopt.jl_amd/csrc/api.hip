@@ -880,27 +880,38 @@ int pcg_breakdown(tohip_ctx* ctx, int err) {
     return TOHIP_BREAKDOWN;
 }
 
+// What the one-launch PCG needs beyond the context's vectors, on first use.
+int pcg1_setup(tohip_ctx* ctx) {
+    if (int rc = dneed(ctx, &ctx->r64b, ctx->g.ndof)) return rc;
+    for (double*& p : ctx->pcg1_part)
+        if (int rc = dneed(ctx, &p, (size_t)kPcg1Vals * pcg1_blocks(ctx->g))) return rc;
+    if (int rc = dneed(ctx, &ctx->pcg1_st, 2)) return rc;
+    if (!ctx->h_pcg1)
+        CK(hipHostMalloc((void**)&ctx->h_pcg1, sizeof(Pcg1State), hipHostMallocDefault));
+    return 0;
+}
+
+// Launch number `it` of a solve: the sets of vectors alternate, r the first residual.
+Pcg1Args pcg1_args(tohip_ctx* ctx, int it, double* r0) {
+    double *r[2] = {r0, ctx->r64b}, *q[2] = {ctx->q64, ctx->t64};
+    const int i = it & 1, o = i ^ 1;
+    return {ctx->u,           r[i], ctx->p64[i],      q[i], ctx->dinv64, r[o], ctx->p64[o], q[o],
+            ctx->pcg1_st + i, ctx->pcg1_st + o,
+            ctx->pcg1_part[i], ctx->pcg1_part[o], pcg1_blocks(ctx->g)};
+}
+
 // One captured graph of `iters` one-launch PCG iterations (even), each followed by
 // the EnergyCriteria check when `energy`.
 int capture_pcg1_graph(tohip_ctx* ctx, hipGraphExec_t* exec, int iters, bool energy) {
     if (*exec) return 0;
-    double *r[2] = {ctx->r64, ctx->r64b}, *q[2] = {ctx->q64, ctx->t64};
     hipGraph_t graph;
     CK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     for (int it = 0; it < iters; ++it) {
-        const int i = it & 1, o = i ^ 1;
-        const Pcg1Args a{ctx->u,           r[i],
-                         ctx->p64[i],      q[i],
-                         ctx->dinv64,      r[o],
-                         ctx->p64[o],      q[o],
-                         ctx->pcg1_st + i, ctx->pcg1_st + o,
-                         ctx->pcg1_part[i], ctx->pcg1_part[o],
-                         pcg1_blocks(ctx->g)};
+        const Pcg1Args a = pcg1_args(ctx, it, ctx->r64);
         if (launch_pcg1(ctx->g, ctx->op64, ctx->fixmask, ctx->E64, ctx->meandiag, a,
                         ctx->stream) != hipSuccess ||
-            (energy && launch_energy_check(ctx->g.ndof, ctx->u, r[o], ctx->b64, ctx->pcg1_st + o,
-                                           ctx->ecrit, ctx->partials,
-                                           ctx->stream) != hipSuccess)) {
+            (energy && launch_energy_check(ctx->g.ndof, ctx->u, a.rn, ctx->b64, a.sn, ctx->ecrit,
+                                           ctx->partials, ctx->stream) != hipSuccess)) {
             hipStreamEndCapture(ctx->stream, &graph);
             ctx->err = "PCG graph capture failed";
             return TOHIP_ERR_HIP;
@@ -927,16 +938,7 @@ int solve_fp64(tohip_ctx* ctx, double abstol, double reltol, int64_t maxiter, bo
         ctx->err = "EnergyCriteria needs a positive tolerance";
         return TOHIP_ERR_ARG;
     }
-    const int nb = pcg1_blocks(ctx->g);
-    if (!ctx->r64b)
-        if (int rc = dalloc(ctx, &ctx->r64b, n)) return rc;
-    for (double*& p : ctx->pcg1_part)
-        if (!p)
-            if (int rc = dalloc(ctx, &p, (size_t)kPcg1Vals * nb)) return rc;
-    if (!ctx->pcg1_st)
-        if (int rc = dalloc(ctx, &ctx->pcg1_st, 2)) return rc;
-    if (!ctx->h_pcg1)
-        CK(hipHostMalloc((void**)&ctx->h_pcg1, sizeof(Pcg1State), hipHostMallocDefault));
+    if (int rc = pcg1_setup(ctx)) return rc;
     Pcg1State hs{};
     hs.rho_prev = 1.0;  // IterativeSolvers starts from rho_prev = 1 (multiplies p = 0)
     hs.tol = -1.0;
@@ -960,7 +962,7 @@ int solve_fp64(tohip_ctx* ctx, double abstol, double reltol, int64_t maxiter, bo
         CK(launch_matvec<double>(ctx->g, ctx->op64, ctx->u, ctx->fixmask, ctx->E64, ctx->t64,
                                  ctx->meandiag, ctx->stream));
     CK(launch_pcg1_start(n, ctx->b64, zero ? nullptr : ctx->t64, ctx->dinv64, ctx->r64,
-                         ctx->p64[0], ctx->pcg1_part[0], nb, ctx->stream));
+                         ctx->p64[0], ctx->pcg1_part[0], pcg1_blocks(ctx->g), ctx->stream));
     if (energy)
         CK(launch_energy_check(n, ctx->u, ctx->r64, ctx->b64, ctx->pcg1_st, ctx->ecrit,
                                ctx->partials, ctx->stream));
@@ -2499,7 +2501,7 @@ int tohip_beso_run(tohip_ctx* ctx, const tohip_beso_opts* o, const double* x0,
 }
 
 int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
-    if (!ctx || !avg_us || reps < 1 || kernel < 0 || kernel > TOHIP_K_CSR_SPMV)
+    if (!ctx || !avg_us || reps < 1 || kernel < 0 || kernel > TOHIP_K_PCG1_64)
         return TOHIP_ERR_ARG;
     if (kernel >= TOHIP_K_MG_PRE && kernel <= TOHIP_K_VCYCLE)
         if (int rc = mg_setup(ctx)) return rc;
@@ -2553,6 +2555,19 @@ int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
         if (int rc = mg_solve_ready(ctx)) return rc;
         CK(launch_vcycle(ctx, ctx->r32, nullptr, nullptr, nullptr));
     }
+    if (kernel == TOHIP_K_PCG1_64) {
+        // a solve with the load r64 from zero that does not end (b64 holds the residual)
+        if (int rc = pcg1_setup(ctx)) return rc;
+        Pcg1State h1{};
+        h1.rho_prev = 1.0;
+        h1.maxiter = 1LL << 60;
+        *ctx->h_pcg1 = h1;
+        CK(hipMemcpyAsync(ctx->pcg1_st, ctx->h_pcg1, sizeof(Pcg1State), hipMemcpyHostToDevice, s));
+        CK(hipMemsetAsync(ctx->u, 0, nD * sizeof(double), s));
+        CK(launch_pcg1_start(nD, ctx->r64, nullptr, ctx->dinv64, ctx->b64, ctx->p64[0],
+                             ctx->pcg1_part[0], pcg1_blocks(ctx->g), s));
+    }
+    int pcg1_it = 0;
     if (kernel == TOHIP_K_OC) {
         CK(hipMemcpyAsync(ctx->xd, ctx->xt, ctx->g.ncells * sizeof(double),
                           hipMemcpyDeviceToDevice, s));
@@ -2622,6 +2637,9 @@ int tohip_bench_kernel(tohip_ctx* ctx, int kernel, int reps, double* avg_us) {
             }
             case TOHIP_K_VCYCLE:
                 return launch_vcycle(ctx, ctx->r32, nullptr, nullptr, nullptr);
+            case TOHIP_K_PCG1_64:
+                return launch_pcg1(ctx->g, ctx->op64, ctx->fixmask, ctx->E64, ctx->meandiag,
+                                   pcg1_args(ctx, pcg1_it++, ctx->b64), s);
             case TOHIP_K_CSR_SPMV:
                 return launch_csr_spmv(ctx->g, ctx->csr_rowptr, ctx->csr_vals, ctx->r64,
                                        ctx->q64, s);
