@@ -390,7 +390,8 @@ static void dispatch_matvec(const Grid& g, int nb, hipStream_t s, const ElemOp<T
 template <typename T>
 hipError_t launch_matvec(const Grid& g, const ElemOp<T>& op, const T* x, const uint8_t* fixmask,
                          const T* E, T* y, double meandiag, hipStream_t s) {
-    dispatch_matvec<T, false>(g, pcg_blocks<T>(g), s, op, x, (const T*)nullptr,
+    // (not pcg_blocks: the FP32 direction step's may be the marching columns')
+    dispatch_matvec<T, false>(g, grid_blocks(ntiles<T>(g)), s, op, x, (const T*)nullptr,
                               (T*)nullptr, (T*)nullptr, fixmask, E, y, meandiag,
                               (PcgScalars*)nullptr, (const double*)nullptr, 0, (double*)nullptr);
     return hipGetLastError();
