@@ -36,10 +36,11 @@ __device__ __forceinline__ int heat_corner(int ox, int oy, int oz) {
 // in place of 64 products and 27 bounds-tested loads a node.
 //
 // One launch is a whole PCG iteration.  Bound by latency on small grids, by the
-// cache traffic of its 4 vectors in (1.3 x (zc + 2) / zc with the halo) and 4
-// out on larger ones.  MI355X, one iteration: 128x96x80 23.8 us (direction, a
-// 27-point gather of K p and update in three launches: 85 us; the 57 MB it must
-// move take 12 us at the copy rate), 80x60 5.7 us (14 us).
+// cache traffic of its vectors on larger ones: p, r, q, D^-1 in with the halo (1.3 x
+// (zc + 2) / zc), x in and x, r, p, q out at the owner.  MI355X, one iteration:
+// 128x96x80 22.4 us (direction, a 27-point gather of K p and update in three
+// launches: 85 us; the 82 MB it must move take 17 us at the copy rate), 80x60 5.0 us
+// (14 us).
 constexpr int kHC = 16, kHO = kHC - 1, kHS = kHC + 1;
 
 // Columns of 15 x 15 nodes and chunks of zc planes, about 768 workgroups when the

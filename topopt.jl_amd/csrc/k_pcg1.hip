@@ -21,8 +21,8 @@
 // Bound by latency below a few 100k nodes (an iteration's launch, loads, sums and
 // one plane step are a chain), above by the loads of four vectors on the halo
 // and 250 registers (two workgroups per CU).  MI355X, an iteration against the
-// direction + update pair: 2D 160x40 5.4 us (12.2), 27x14x10 8.5 (12.0), 76x36x28
-// 15.4 (23.1), 120x40x40 22.0 (33.7), 256x128x128 267 (307).
+// direction + update pair: 2D 160x40 5.2 us (12.2), 27x14x10 7.6 (12.0), 76x36x28
+// 13.9 (23.1), 120x40x40 19.8 (33.7), 256x128x128 268 (307).
 #include <algorithm>
 
 #include "k_pcg1.h"
@@ -337,8 +337,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_pcg1(Grid g, ElemOp<double> op,
 // 3D grids too small for the chunks to matter: one output plane a workgroup, 512
 // threads, one group of 256 for the layer below the plane and one for the layer
 // above, so that the three planes are loaded and the two layers computed at the
-// same time instead of in turn.  27x14x10 box cells: 8.5 us an iteration, 13.2
-// marching.  164 VGPRs: one workgroup per CU, so a grid of more planes than CUs is
+// same time instead of in turn.  27x14x10 box cells: 8.5 us an iteration against 13.2
+// marching (whole solves).  164 VGPRs: one workgroup per CU, so a grid of more planes than CUs is
 // left to the marching kernel (76x36x28: 26 against 15 us; 120x40x40: 47 against 22;
 // bounded to two workgroups per CU it spills: 38 and 65).
 static int pcg1_planes(const Grid& g) {
